@@ -54,6 +54,8 @@ struct DevPhys {
   // conduction denominator Re*Pr_tur*(gama-1)*Ma^2 (NS_Solver.cpp:540),
   // Pr^(1/3) of the wall-temperature relation (FlowConstants.cpp:44)
   double nut_inf, nut_inlet, qkt_den, pr_cuberoot;
+  // derived: 1/(gama - 1), Cv/Rg, Cv/Rg + 1, 1/Re, 1/qkt_den
+  double ig1, cvR, cpR, iRe, iqkt;
 };
 
 // Every copy of the cell state that a once-per-step ghost fill must keep
@@ -91,7 +93,7 @@ __device__ __forceinline__ bool wg_halted(const unsigned long long *err) {
 }
 
 struct BlkInfo {
-  double h[3], invh[3], area[3], vol, step_num;
+  double h[3], invh[3], area[3], vol, invvol, step_num;
   int case_id, level, finest, pad;
 };
 

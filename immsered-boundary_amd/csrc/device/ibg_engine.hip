@@ -1076,6 +1076,7 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
     // ComptFaceArea MeshOp.H:17-36, ComptCellParams MeshOp.H:4-12
     B.area[0] = h[1] * h[2]; B.area[1] = h[2] * h[0]; B.area[2] = h[0] * h[1];
     B.vol = h[0] * h[1] * h[2];
+    B.invvol = 1.0 / B.vol;
     const int l = b % L;
     B.step_num = c->cfg.temporal_refine ? (double)(1 << (L - 1 - l)) : 1.0;
     B.case_id = b / L;
@@ -1097,6 +1098,11 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
     P.nut_inf = p.nut_inf; P.nut_inlet = p.nut_inlet;
     P.qkt_den = p.Re * p.Pr_tur * (p.gama - 1) * pow(p.Ma, 2);
     P.pr_cuberoot = pow(p.Pr, 1.0 / 3.0);
+    P.ig1 = 1.0 / (p.gama - 1.0);
+    P.cvR = p.Cv / p.Rg;
+    P.cpR = P.cvR + 1.0;
+    P.iRe = 1.0 / p.Re;
+    P.iqkt = 1.0 / P.qkt_den;
   }
   // ---- per-cell arrays (device order)
   std::vector<int16_t> cellblk(N);

@@ -116,10 +116,10 @@ struct ViscArgs {
 template <typename R, int D>
 __device__ __forceinline__ ViscPhys<R, D> visc_phys(const BlkInfo &bi, const DevPhys &P) {
   ViscPhys<R, D> vp;
-  vp.Rg = (R)P.Rg; vp.Re = (R)P.Re; vp.qk = (R)P.qk; vp.SoT = (R)P.SoT;
+  vp.Rg = (R)P.Rg; vp.iRe = std::is_same<R, float>::value ? c_rcp((R)P.Re) : (R)P.iRe; vp.qk = (R)P.qk; vp.SoT = (R)P.SoT;
   vp.ih0 = (R)bi.invh[0]; vp.ih1 = (R)bi.invh[1]; vp.ih2 = (R)bi.invh[2];
   vp.ar0 = (R)bi.area[0]; vp.ar1 = (R)bi.area[1]; vp.ar2 = (R)bi.area[2];
-  vp.qkt = (R)P.qkt_den;
+  vp.iqkt = std::is_same<R, float>::value ? c_rcp((R)P.qkt_den) : (R)P.iqkt;
   return vp;
 }
 
@@ -145,9 +145,9 @@ __device__ __forceinline__ void visc_face(const ViscArgs<R, D> &a, const ViscPhy
   }
   mf = R(0);
   if (a.turb)
-    visc_flux<R, D>(L, Rr, t, dir, vp, out, true, a.nu[st.y], a.nu[st.z], &mf);
+    visc_flux_cells<R, D>(L, Rr, t, dir, vp, out, true, a.nu[st.y], a.nu[st.z], &mf);
   else
-    visc_flux<R, D>(L, Rr, t, dir, vp, out);
+    visc_flux_cells<R, D>(L, Rr, t, dir, vp, out, false, R(0), R(0), &mf);
 }
 
 // Once per step (ComptViscousStress NS_Solver.cpp:365-629 is frozen across
@@ -226,7 +226,7 @@ __device__ __forceinline__ void visc_prep_tile(const ViscArgs<R, D> &a, const Ti
 #pragma unroll
   for (int k = 0; k < NV; ++k) rv[k] = (R)s[k];
   vstore<R, D>(a.Rv, c, rv);
-  if (a.turb) a.mutf[c] = (R)(tot / bi.vol / P.Re);
+  if (a.turb) a.mutf[c] = (R)n_div(n_div(tot, bi.vol), P.Re);
 }
 
 template <typename R, int D>
@@ -441,8 +441,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, int tile) {
 
   const BlkInfo &bi = a.blk[ti.blk];
   const DevPhys &P = a.phys[bi.case_id];
-  PhysR<R> ph;
-  ph.gama = (R)P.gama; ph.Rg = (R)P.Rg; ph.Cv = (R)P.Cv; ph.Ma = (R)P.Ma;
+  const PhysR<R> ph = phys_r<R>(P);
   const R areas[3] = {(R)bi.area[0], (R)bi.area[1], (R)bi.area[2]};
 
   for (int f = threadIdx.x; f < ti.nface; f += blockDim.x) {
@@ -453,10 +452,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, int tile) {
     const Prim<R, D> q2 = pload<R, D>(a.Win, st.z);
     const Prim<R, D> q3 = pload<R, D>(a.Win, st.w);
     R flux[NV];
-    if constexpr (kMixed)
-      roe_flux_fast<D>(q0, q1, q2, q3, dir, areas[dir], ph, a.limiter, flux);
-    else
-      roe_flux<R, D>(q0, q1, q2, q3, dir, areas[dir], ph, a.limiter, flux);
+    roe_flux<D>(q0, q1, q2, q3, dir, areas[dir], ph, a.limiter, flux);
     if (a.rbal) {
       // a coarse/fine face of the optional balance: its balanced flux
       const int q = a.tmod[ti.face0 + f];
@@ -477,7 +473,6 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, int tile) {
   if (halt) return;   // uniform: the flag was written before the barrier
 
   const double level_ts = a.alpha * a.dt[bi.case_id] * bi.step_num;
-  const double inv_vol = 1.0 / bi.vol;
   double mx[NV], sq[NV];
 #pragma unroll
   for (int k = 0; k < NV; ++k) { mx[k] = 0.0; sq[k] = 0.0; }
@@ -642,22 +637,18 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, int tile) {
       double U[NV];
       {
         const Prim<double, D> w0 = pload<double, D>(a.W64, c);
-        const double T0 = w0.p / (w0.r * P.Rg);
         const double ke0 = (D == 3) ? 0.5 * (w0.u * w0.u + w0.v * w0.v + w0.w * w0.w)
                                     : 0.5 * (w0.u * w0.u + w0.v * w0.v);
-        const double e0 = P.Cv * T0 + ke0;
+        double re0;
+        if constexpr (kMixed) re0 = w0.r * (P.Cv * n_div(w0.p, w0.r * P.Rg) + ke0);
+        else re0 = P.cvR * w0.p + w0.r * ke0;   // roe T = p / Rg
         U[0] = w0.r; U[1] = w0.r * w0.u; U[2] = w0.r * w0.v;
-        if (D == 3) { U[3] = w0.r * w0.w; U[4] = w0.r * e0; } else U[3] = w0.r * e0;
+        if (D == 3) { U[3] = w0.r * w0.w; U[4] = re0; } else U[3] = re0;
       }
-      if constexpr (kMixed) {
-        const double sc = level_ts * inv_vol;
+      // cv_old + source * level_ts / v  (NS_Solver.cpp:870)
+      const double sc = level_ts * bi.invvol;
 #pragma unroll
-        for (int k = 0; k < NV; ++k) U[k] = U[k] + s[k] * sc;
-      } else {
-        // cv_old + source * level_ts / v  (NS_Solver.cpp:870)
-#pragma unroll
-        for (int k = 0; k < NV; ++k) U[k] = U[k] + s[k] * level_ts / bi.vol;
-      }
+      for (int k = 0; k < NV; ++k) U[k] = fma(s[k], sc, U[k]);
       if (a.turb) {
         // viseddy = max(c_vis_old + mutsource * level_ts, 0) (:874-876, :955-957)
         nu_new = a.nu64[c] + snu * level_ts;
@@ -667,19 +658,27 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, int tile) {
       if (fg & F_PRIM) {
         // Get_Prim_Vars FlowVariables.H:50-57
         wr = U[0];
-        double e;
         if constexpr (kMixed) {
-          const double ir = 1.0 / U[0];
+          const double ir = n_div(1.0, U[0]);
           wu = U[1] * ir;
           wv = U[2] * ir;
-          if (D == 3) { ww = U[3] * ir; e = U[4] * ir; } else e = U[3] * ir;
+          if (D == 3) ww = U[3] * ir;
+          const double ke = (D == 3) ? 0.5 * (wu * wu + wv * wv + ww * ww) : 0.5 * (wu * wu + wv * wv);
+          wp = (U[D == 3 ? 4 : 3] * ir - ke) * (P.gama - 1.0) * wr;
         } else {
-          wu = U[1] / U[0];
-          wv = U[2] / U[0];
-          if (D == 3) { ww = U[3] / U[0]; e = U[4] / U[0]; } else e = U[3] / U[0];
+          // the quotients share one reciprocal, each with its exact residual
+          // added back
+          const double ir = n_rcp(U[0]);
+          auto over_r = [&](double x) {
+            const double q = x * ir;
+            return fma(fma(-U[0], q, x), ir, q);
+          };
+          wu = over_r(U[1]);
+          wv = over_r(U[2]);
+          if (D == 3) ww = over_r(U[3]);
+          const double ke = (D == 3) ? 0.5 * (wu * wu + wv * wv + ww * ww) : 0.5 * (wu * wu + wv * wv);
+          wp = (U[D == 3 ? 4 : 3] - ke * wr) * (P.gama - 1.0);
         }
-        const double ke = (D == 3) ? 0.5 * (wu * wu + wv * wv + ww * ww) : 0.5 * (wu * wu + wv * wv);
-        wp = (e - ke) * (P.gama - 1.0) * wr;
         // T = p/(roe Rg) < 0  (NS_Solver.cpp:55-66), Rg > 0
         if ((wp < 0.0) != (wr < 0.0)) report_error(a.err, c, 37);
         write = true;
@@ -1298,12 +1297,11 @@ __global__ void k_face_probe(int nface, const int4 *st, const int8_t *dir, const
   constexpr int NV = D + 2;
   const BlkInfo &bi = blk[fblk[f]];
   const DevPhys &P = phys[bi.case_id];
-  PhysR<R> ph;
-  ph.gama = (R)P.gama; ph.Rg = (R)P.Rg; ph.Cv = (R)P.Cv; ph.Ma = (R)P.Ma;
+  const PhysR<R> ph = phys_r<R>(P);
   const int4 s = st[f];
   R flux[NV];
-  roe_flux<R, D>(pload<R, D>(W, s.x), pload<R, D>(W, s.y), pload<R, D>(W, s.z),
-                 pload<R, D>(W, s.w), dir[f], (R)bi.area[dir[f]], ph, lim, flux);
+  roe_flux<D>(pload<R, D>(W, s.x), pload<R, D>(W, s.y), pload<R, D>(W, s.z),
+              pload<R, D>(W, s.w), dir[f], (R)bi.area[dir[f]], ph, lim, flux);
   double *o = out + (size_t)f * 5;
   if (D == 3) { for (int k = 0; k < 5; ++k) o[k] = flux[k]; }
   else { o[0] = flux[0]; o[1] = flux[1]; o[2] = flux[2]; o[3] = 0.0; o[4] = flux[3]; }
@@ -1318,11 +1316,7 @@ __global__ void k_visc_probe(int nface, const int4 *st, const int4 *vst, const i
   constexpr int NV = D + 2;
   const BlkInfo &bi = blk[fblk[f]];
   const DevPhys &P = phys[bi.case_id];
-  ViscPhys<R, D> vp;
-  vp.Rg = (R)P.Rg; vp.Re = (R)P.Re; vp.qk = (R)P.qk; vp.SoT = (R)P.SoT;
-  vp.ih0 = (R)bi.invh[0]; vp.ih1 = (R)bi.invh[1]; vp.ih2 = (R)bi.invh[2];
-  vp.ar0 = (R)bi.area[0]; vp.ar1 = (R)bi.area[1]; vp.ar2 = (R)bi.area[2];
-  vp.qkt = (R)P.qkt_den;
+  const ViscPhys<R, D> vp = visc_phys<R, D>(bi, P);
   const int4 s = st[f];
   Prim<R, D> t[(D == 3) ? 8 : 4];
   const int4 v0 = vst[(size_t)f * (D - 1)];
@@ -1336,11 +1330,8 @@ __global__ void k_visc_probe(int nface, const int4 *st, const int4 *vst, const i
   }
   R o5[NV];
   R mf = R(0);
-  if (nu)
-    visc_flux<R, D>(pload<R, D>(W, s.y), pload<R, D>(W, s.z), t, dir[f], vp, o5, true, nu[s.y],
-                    nu[s.z], &mf);
-  else
-    visc_flux<R, D>(pload<R, D>(W, s.y), pload<R, D>(W, s.z), t, dir[f], vp, o5);
+  visc_flux_cells<R, D>(pload<R, D>(W, s.y), pload<R, D>(W, s.z), t, dir[f], vp, o5, nu != nullptr,
+                        nu ? nu[s.y] : R(0), nu ? nu[s.z] : R(0), &mf);
   if (mout) mout[f] = mf;
   double *o = out + (size_t)f * 5;
   if (D == 3) { for (int k = 0; k < 5; ++k) o[k] = o5[k]; }

@@ -305,7 +305,7 @@ __device__ __forceinline__ R sa_pointwise(R nu, R mu0, R roe, R sd, R olen, R Re
   R bigs = olen + v_div(v_div(nu * fv2, segdis), Re);
   bigs = (R(0.3) * olen < bigs) ? bigs : R(0.3) * olen;
   const R ft2 = R(SA::ct3) * r_exp(-R(SA::ct4) * bigx * bigx);
-  R rr = v_div(v_div(nu, bigs * segdis), Re);
+  R rr = sa_r(nu, bigs * segdis, Re);
   rr = (R(10.0) < rr) ? R(10.0) : rr;
   const R rsix = r_pow6(rr);
   const R g = rr + R(SA::cw2) * (rsix - rr);

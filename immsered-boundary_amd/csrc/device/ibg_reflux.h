@@ -66,7 +66,6 @@ k_balance_inv(const RfPair *pairs, int n, const int4 *tst, const int8_t *tdir, P
               const BlkInfo *blk, const DevPhys *phys, int limiter, R *rbal,
               const unsigned long long *err) {
   constexpr int NV = D + 2;
-  constexpr bool kMixed = std::is_same<R, float>::value;
   const int j = blockIdx.x * blockDim.x + threadIdx.x;
   if (j >= n || halted(err)) return;
   const RfPair p = pairs[j];
@@ -78,8 +77,7 @@ k_balance_inv(const RfPair *pairs, int n, const int4 *tst, const int8_t *tdir, P
     const int s = k == 0 ? p.cslot : p.fslot[k - 1];
     const BlkInfo &bi = blk[k == 0 ? p.cblk : p.fblk];
     const DevPhys &P = phys[bi.case_id];
-    PhysR<R> ph;
-    ph.gama = (R)P.gama; ph.Rg = (R)P.Rg; ph.Cv = (R)P.Cv; ph.Ma = (R)P.Ma;
+    const PhysR<R> ph = phys_r<R>(P);
     const int4 st = tst[s];
     const int dir = tdir[s];
     const Prim<R, D> q0 = pload<R, D>(Win, st.x);
@@ -87,10 +85,7 @@ k_balance_inv(const RfPair *pairs, int n, const int4 *tst, const int8_t *tdir, P
     const Prim<R, D> q2 = pload<R, D>(Win, st.z);
     const Prim<R, D> q3 = pload<R, D>(Win, st.w);
     const R area = (R)bi.area[dir];
-    if constexpr (kMixed)
-      roe_flux_fast<D>(q0, q1, q2, q3, dir, area, ph, limiter, F[k]);
-    else
-      roe_flux<R, D>(q0, q1, q2, q3, dir, area, ph, limiter, F[k]);
+    roe_flux<D>(q0, q1, q2, q3, dir, area, ph, limiter, F[k]);
   }
   balance_faces<R, NV>(p.mode, F);
 #pragma unroll
