@@ -58,6 +58,14 @@ struct DevPhys {
   double ig1, cvR, cpR, iRe, iqkt;
 };
 
+// Tables that no kernel reading them writes and whose index is uniform over
+// the workgroup (tiles, blocks, physics, dt, the network's statistics): read
+// through the constant address space they stay scalar loads into SGPRs.  As
+// plain pointers the compiler keeps them scalar only up to the first barrier
+// and reloads them per lane afterwards.
+template <typename T> using Uni = const __attribute__((address_space(4))) T *;
+template <typename T> __device__ __forceinline__ Uni<T> uni(const T *p) { return (Uni<T>)p; }
+
 // Every copy of the cell state that a once-per-step ghost fill must keep
 // consistent: the FP64 master and the stencil buffers the stages rotate
 // through.  Plain mode: stencil buffer 0 is the master; d1, d2 are extra
@@ -97,8 +105,10 @@ struct BlkInfo {
   int case_id, level, finest, pad;
 };
 
+// halo0: first entry of a block tile's halo list, -1 for a general tile
+// (whose faces are [face0, face0 + nface) of the tile face lists)
 struct TileInfo {
-  int cell0, ncell, face0, nface, blk, pad0, pad1, pad2;
+  int cell0, ncell, face0, nface, blk, halo0, pad1, pad2;
 };
 
 struct Motion {

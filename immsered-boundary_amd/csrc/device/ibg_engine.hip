@@ -101,6 +101,8 @@ struct ibg_ctx {
   uint8_t *flags = nullptr;
   int *cellcase = nullptr, *nb27 = nullptr;
   TileInfo *tiles = nullptr;
+  int *halo = nullptr;         // halo lists of the block tiles (ibg_block.h)
+  int nblock = 0;              // block tiles
   int *case_tiles = nullptr;   // [case][level] = {first tile, end tile}
   int4 *tst = nullptr, *tvs = nullptr;
   int8_t *tdir = nullptr;
@@ -239,7 +241,9 @@ namespace {
 size_t ml_resident_offset(const ibg_ctx *c) {
   size_t per = 4 * sizeof(float) + (c->D == 3 ? sizeof(float) : 0);
   if (c->turb) per += 2 * sizeof(int);
-  return ((size_t)c->max_tile_faces * per + 15) & ~(size_t)15;
+  size_t b = (size_t)c->max_tile_faces * per;
+  if (c->nblock > 0) b = std::max(b, blk_smem(sizeof(float), c->turb, false));
+  return (b + 15) & ~(size_t)15;
 }
 
 #define HIPCHK(x)                                                        \
@@ -362,21 +366,24 @@ inline int transfer_due(const ibg_ctx *c, int cl, int ts) {
 }
 inline unsigned grid(int n, int b) { return (unsigned)((n + b - 1) / b); }
 
-// LDS of the tiled kernels: face fluxes (4 values + the 3D fifth), then for
-// the SA closure either the two face-cell indices (stage) or the face flux
-// of the working variable (viscous pass; a fused first stage holds either).
-size_t tile_smem(const ibg_ctx *c, size_t rsize, bool stage) {
+// LDS of the tiled kernels, the larger of the two kinds of tile.  General:
+// face fluxes (4 values + the 3D fifth), then for the SA closure either the
+// two face-cell indices (stage) or the face flux of the working variable
+// (viscous pass; a fused first stage holds either).  Block: blk_smem.
+size_t tile_smem(const ibg_ctx *c, size_t rsize, bool stage, bool fused = false) {
   size_t per = 4 * rsize + (c->D == 3 ? rsize : 0);
   if (c->turb) per += stage ? std::max<size_t>(2 * sizeof(int), rsize) : rsize;
-  const size_t b = (size_t)c->max_tile_faces * per;
+  size_t b = (size_t)c->max_tile_faces * per;
+  if (c->nblock > 0) b = std::max(b, blk_smem(rsize, c->turb, fused || !stage));
   if (stage && c->cl.on) {
     // the network's weights: after every face array, resident across the
     // tiles (persistent schedule), or after the face fluxes over the
     // face-cell indices (one workgroup per tile)
     if (c->cfg.schedule == 1) return ml_resident_offset(c) + kStageMlSmem;
-    const size_t m = (c->D == 2 ? ml_smem_offset<float, 2>(c->max_tile_faces)
-                                : ml_smem_offset<float, 3>(c->max_tile_faces)) + kStageMlSmem;
-    return std::max(b, m);
+    size_t m = c->D == 2 ? ml_smem_offset<float, 2>(c->max_tile_faces)
+                         : ml_smem_offset<float, 3>(c->max_tile_faces);
+    if (c->nblock > 0) m = std::max(m, blk_state_offset(rsize));
+    return std::max(b, m + kStageMlSmem);
   }
   return b;
 }
@@ -396,6 +403,7 @@ template <typename R, int D>
 ViscArgs<R, D> visc_args(ibg_ctx *c) {
   ViscArgs<R, D> a;
   a.tiles = c->tiles; a.tst = c->tst; a.tvs = c->tvs; a.tdir = c->tdir; a.slots = c->slots;
+  a.halo = c->halo;
   a.blk = c->blk; a.phys = c->phys;
   a.W = c->sbuf<R, D>(0);
   a.Rv = c->rv<R, D>();
@@ -416,7 +424,7 @@ ibg_status launch_stage(ibg_ctx *c, int ntile, int ncell, int subt, bool last, d
   int bin = 0, bout = 0;
   stage_bufs(c->cfg.nstage, subt, &bin, &bout);
   StageArgs<R, D> a;
-  a.tiles = c->tiles; a.tst = c->tst; a.tdir = c->tdir; a.slots = c->slots;
+  a.tiles = c->tiles; a.tst = c->tst; a.tdir = c->tdir; a.slots = c->slots; a.halo = c->halo;
   a.flags = c->flags; a.blk = c->blk; a.phys = c->phys; a.dt = c->dt;
   a.Win = c->sbuf<R, D>(bin);
   a.Wout = c->sbuf<R, D>(bout);
@@ -452,7 +460,7 @@ ibg_status launch_stage(ibg_ctx *c, int ntile, int ncell, int subt, bool last, d
     HIPCHK(hipGetLastError());
     a.rbal = (const R *)c->rbal;
   }
-  const size_t smem = tile_smem(c, sizeof(R), true);
+  const size_t smem = tile_smem(c, sizeof(R), true, a.fuse_visc);
   a.ntile = ntile;
   a.mlw_off = (unsigned)ml_resident_offset(c);
   if (c->cfg.schedule == 1 && ntile >= 8) {
@@ -767,6 +775,111 @@ ibg_status read_err(ibg_ctx *c, int64_t *cell, int32_t *code) {
   return IBG_OK;
 }
 
+}  // namespace
+
+// The block tiles of an uploaded 2D mesh: isblk[i] for the first device cell
+// i of every run of 256 cells that fills a 16 x 16 square of its (level,
+// case) in Morton order and whose every face has the stencil its position
+// gives (checked face by face, so a block tile computes from the same cells
+// as a general tile over the same run); halo gets kHalo cells per square, in
+// cell order.  With the optional coarse/fine balance, a square with a
+// balanced face stays general (its fluxes come from the pre-pass by face).
+namespace {
+template <class FI, class F4v, class FD>
+void find_blocks(ibg_ctx *c, const ibg_mesh_soa *m, const std::vector<int> &order,
+                       const FI &cfaces, const F4v &face_st, const F4v &face_vst,
+                       const FD &face_dir, std::vector<uint8_t> &isblk, hvec<int> &halo) {
+  const int L = c->L, Nn = c->Nn;
+  std::vector<uint8_t> bal;
+  if (c->cfg.reflux && m->nmdy > 0) {
+    bal.assign(c->F, 0);
+    for (int i = 0; i < m->nmdy; ++i)
+      for (int k = 1; k < 6; ++k) {
+        const int f = m->mdy[(size_t)i * 6 + k];
+        if (f >= 0 && f < c->F) bal[c->fh2d[f]] = 1;
+      }
+  }
+  // candidates: the corners' keys first (nearly every start fails there),
+  // then every key
+  auto key = [&](int i, int d) { return m->key[(size_t)order[i] * 3 + d]; };
+  std::vector<int> cand;
+  int pos = 0;
+  for (int l = L - 1; l >= 0; --l)
+    for (int cs = 0; cs < c->ncases; ++cs) {
+      const int end = pos + m->blk_nnormal[cs * L + l];
+      for (int t = pos; t + kBlkCells <= end;) {
+        const int x0 = key(t, 0), y0 = key(t, 1);
+        bool ok = key(t + 255, 0) == x0 + 15 && key(t + 255, 1) == y0 + 15 &&
+                  key(t + 85, 0) == x0 + 15 && key(t + 85, 1) == y0;
+        for (int i = 0; ok && i < kBlkCells; ++i) {
+          int x, y;
+          blk_xy(i, x, y);
+          ok = key(t + i, 0) == x0 + x && key(t + i, 1) == y0 + y && key(t + i, 2) == key(t, 2);
+        }
+        if (ok) cand.push_back(t);
+        t += ok ? kBlkCells : 1;
+      }
+      pos = end;
+    }
+  const int n = (int)cand.size();
+  hvec<int> all((size_t)n * kHalo);
+  std::vector<uint8_t> good(n, 0);
+  host_parallel(n, [&](int lo, int hi) {
+    for (int q = lo; q < hi; ++q) {
+      const int t = cand[q];
+      int P[kBoxCells];
+      for (int &v : P) v = -1;
+      int cell[kBlkN][kBlkN];   // [y][x]
+      for (int i = 0; i < kBlkCells; ++i) {
+        int x, y;
+        blk_xy(i, x, y);
+        P[box_pos(x, y)] = cell[y][x] = t + i;
+      }
+      auto face = [&](int x, int y, int s) { return cfaces[(size_t)cell[y][x] * 4 + s]; };
+      for (int k = 0; k < kBlkN; ++k) {
+        const int4 xl = face_st[face(0, k, 0)], xh = face_st[face(kBlkN - 1, k, 1)];
+        const int4 yl = face_st[face(k, 0, 2)], yh = face_st[face(k, kBlkN - 1, 3)];
+        P[box_pos(-2, k)] = xl.x; P[box_pos(-1, k)] = xl.y;
+        P[box_pos(kBlkN, k)] = xh.z; P[box_pos(kBlkN + 1, k)] = xh.w;
+        P[box_pos(k, -2)] = yl.x; P[box_pos(k, -1)] = yl.y;
+        P[box_pos(k, kBlkN)] = yh.z; P[box_pos(k, kBlkN + 1)] = yh.w;
+      }
+      P[box_pos(-1, -1)] = face_vst[face(0, 0, 0)].z;
+      P[box_pos(kBlkN, -1)] = face_vst[face(kBlkN - 1, 0, 1)].w;
+      P[box_pos(-1, kBlkN)] = face_vst[face(0, kBlkN - 1, 0)].x;
+      P[box_pos(kBlkN, kBlkN)] = face_vst[face(kBlkN - 1, kBlkN - 1, 1)].y;
+      bool ok = true;
+      for (int y = 0; ok && y < kBlkN; ++y)
+        for (int x = 0; ok && x < kBlkN; ++x)
+          for (int s = 0; ok && s < 4; ++s) {
+            const int f = face(x, y, s), d = s >> 1;
+            const int st = d == 0 ? 1 : kBoxP, tt = d == 0 ? kBoxP : 1;
+            const int p = box_pos(x, y) + (s & 1) * st;   // the face's high-side cell
+            const int4 a = face_st[f], v = face_vst[f];
+            ok = face_dir[f] == d && a.x == P[p - 2 * st] && a.y == P[p - st] && a.z == P[p] &&
+                 a.w == P[p + st] && v.x == P[p - st + tt] && v.y == P[p + tt] &&
+                 v.z == P[p - st - tt] && v.w == P[p - tt] && (bal.empty() || !bal[f]);
+          }
+      for (int h = 0; ok && h < kHalo; ++h) {
+        const int v = P[halo_pos(h)];
+        all[(size_t)q * kHalo + h] = v;
+        ok = v >= 0 && v < c->N;
+      }
+      good[q] = ok;
+    }
+  }, 64);
+  isblk.assign(Nn, 0);
+  size_t w = 0;
+  for (int q = 0; q < n; ++q) {
+    if (!good[q]) continue;
+    isblk[cand[q]] = 1;
+    if (w != (size_t)q)
+      std::copy(all.begin() + (size_t)q * kHalo, all.begin() + (size_t)(q + 1) * kHalo, all.begin() + w * kHalo);
+    ++w;
+  }
+  all.resize(w * kHalo);
+  halo.swap(all);
+}
 }  // namespace
 
 // Host-side validation of every index a kernel will dereference, so that a
@@ -1188,13 +1301,19 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
     }
   }
   });
-  // ---- tiles over each (level, case) run of normal cells.  A tile's face
-  // list is the faces of its cells in first-occurrence order (cells in
-  // order, each cell's faces low/high per direction); the lists are formed
-  // per tile in parallel, placed by a prefix sum, then filled in parallel.
+  // ---- tiles over each (level, case) run of normal cells: block tiles
+  // (ibg_block.h) where 256 consecutive cells fill a square, general tiles
+  // over the runs between them.  A general tile's face list is the faces of
+  // its cells in first-occurrence order (cells in order, each cell's faces
+  // low/high per direction); the lists are formed per tile in parallel,
+  // placed by a prefix sum, then filled in parallel.
+  std::vector<uint8_t> isblk;      // by device cell: the first cell of a square
+  hvec<int> halo;
+  if (D == 2 && c->tile == kBlkCells) find_blocks(c, m, order, cfaces, face_st, face_vst, face_dir, isblk, halo);
   std::vector<TileInfo> tiles;
   std::vector<int> case_tiles((size_t)nc * L * 2, 0);   // [case][level] = {first, end}
   c->tile_end.assign(L, 0);
+  c->nblock = 0;
   {
     int pos = 0;
     for (int l = L - 1; l >= 0; --l) {
@@ -1202,13 +1321,27 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
         const int b = cs * L + l;
         const int n = m->blk_nnormal[b];
         case_tiles[(size_t)b * 2] = (int)tiles.size();
-        for (int t0 = 0; t0 < n; t0 += c->tile) {
+        auto emit = [&](int cell0, int ncell, int halo0) {
           TileInfo ti{};
-          ti.cell0 = pos + t0;
-          ti.ncell = std::min(c->tile, n - t0);
+          ti.cell0 = cell0;
+          ti.ncell = ncell;
           ti.blk = b;
+          ti.halo0 = halo0;
           tiles.push_back(ti);
+        };
+        int run = pos;   // start of the general run not yet emitted
+        auto flush = [&](int end) {
+          for (; run < end; run += c->tile) emit(run, std::min(c->tile, end - run), -1);
+          run = end;
+        };
+        for (int t = pos; !isblk.empty() && t + kBlkCells <= pos + n;) {
+          if (!isblk[t]) { ++t; continue; }
+          flush(t);
+          emit(t, kBlkCells, kHalo * c->nblock++);
+          t += kBlkCells;
+          run = t;
         }
+        flush(pos + n);
         case_tiles[(size_t)b * 2 + 1] = (int)tiles.size();
         pos += n;
       }
@@ -1228,6 +1361,11 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
       const TileInfo &ti = tiles[t];
       std::vector<int> &used = tface[t];
       used.clear();
+      if (ti.halo0 >= 0) {
+        // a block tile lists no faces and reads no slots
+        std::fill(slots.begin() + (size_t)ti.cell0 * q2, slots.begin() + (size_t)(ti.cell0 + ti.ncell) * q2, 0);
+        continue;
+      }
       std::vector<int> touched;
       for (int k = 0; k < ti.ncell; ++k) {
         const int dc = ti.cell0 + k;
@@ -1261,16 +1399,14 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
   const size_t nts = ntl ? (size_t)tiles[ntl - 1].face0 + tiles[ntl - 1].nface : 0;
   hvec<int4> tst(nts), tvs(nts * (D - 1));
   hvec<int8_t> tdir(nts);
-  // per device face: its first tile face (the lowest slot), the number of
-  // tiles naming it; set with atomics while the tile faces are filled
-  std::vector<std::atomic<int>> fslot(F), fcount(F);
+  // per device face: its first tile face (the lowest slot); set with
+  // atomics while the tile faces are filled
+  std::vector<std::atomic<int>> fslot(F);
   host_parallel(F, [&](int lo, int hi) {
     for (int f = lo; f < hi; ++f) {
       fslot[f].store(INT_MAX, std::memory_order_relaxed);
-      fcount[f].store(0, std::memory_order_relaxed);
     }
   });
-  hvec<int> slot_tile(nts);
   host_parallel(ntl, [&](int lo, int hi) {
     for (int t = lo; t < hi; ++t) {
       const size_t f0 = (size_t)tiles[t].face0;
@@ -1280,27 +1416,21 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
         tst[f0 + k] = face_st[f];
         tdir[f0 + k] = face_dir[f];
         for (int k2 = 0; k2 < D - 1; ++k2) tvs[(f0 + k) * (D - 1) + k2] = face_vst[(size_t)f * (D - 1) + k2];
-        slot_tile[f0 + k] = t;
         const int sl = (int)(f0 + k);
         int cur = fslot[f].load(std::memory_order_relaxed);
         while (sl < cur && !fslot[f].compare_exchange_weak(cur, sl, std::memory_order_relaxed)) {
         }
-        fcount[f].fetch_add(1, std::memory_order_relaxed);
       }
     }
   }, 64);
   tface.clear();
   tface.shrink_to_fit();
-  // that first tile face, its tile's block, the tile count (-1 / 0 for a
-  // face no tile names)
-  std::vector<int> face_slot0(F), face_tblk(F), face_ntile(F);
+  // that first tile face, -1 for a face in no list
+  std::vector<int> face_slot0(F);
   host_parallel(F, [&](int lo, int hi) {
     for (int f = lo; f < hi; ++f) {
       const int sl = fslot[f].load(std::memory_order_relaxed);
-      const bool named = sl != INT_MAX;
-      face_slot0[f] = named ? sl : -1;
-      face_tblk[f] = named ? tiles[slot_tile[sl]].blk : -1;
-      face_ntile[f] = fcount[f].load(std::memory_order_relaxed);
+      face_slot0[f] = sl != INT_MAX ? sl : -1;
     }
   });
   c->ntiles = (int)tiles.size();
@@ -1309,6 +1439,24 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
   // the coarse face and its fine faces) and the tile face -> entry map
   std::vector<RfPair> rfp;
   std::vector<int> tmod(tst.size(), -1);
+  std::vector<uint8_t> paired(m->nmdy > 0 ? F : 0, 0);
+  // the one tile that names a face (one of whose cells lists it), -1 when
+  // none or several do
+  auto naming_tile = [&](int df) {
+    int found = -1;
+    for (int dc : {face_st[df].y, face_st[df].z}) {
+      if (dc >= Nn) continue;
+      bool lists = false;
+      for (int q = 0; q < q2; ++q) lists = lists || cfaces[(size_t)dc * q2 + q] == df;
+      if (!lists) continue;
+      const int t = (int)(std::upper_bound(tiles.begin(), tiles.end(), dc,
+                                           [](int v, const TileInfo &x) { return v < x.cell0; }) -
+                          tiles.begin()) - 1;
+      if (found >= 0 && t != found) return -1;
+      found = t;
+    }
+    return found;
+  };
   for (int i = 0; i < m->nmdy; ++i) {
     const int32_t *r = m->mdy + (size_t)i * 6;
     RfPair p{};
@@ -1320,20 +1468,23 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
       const int df = c->fh2d[r[1 + k]];
       // each balanced face lies in exactly one tile (its other cell is a
       // ghost) and in one pair
-      if (df < 0 || face_ntile[df] != 1 || tmod[face_slot0[df]] >= 0) return IBG_ERR_ARG;
-      const int sl = face_slot0[df];
-      tmod[sl] = j * 5 + k;
+      const int t = df < 0 ? -1 : naming_tile(df);
+      if (t < 0 || paired[df]) return IBG_ERR_ARG;
+      paired[df] = 1;
+      const int sl = face_slot0[df];   // -1 in a block tile (only without the balance)
+      if (sl >= 0) tmod[sl] = j * 5 + k;
       if (k == 0) {
         p.cslot = sl;
-        p.cblk = face_tblk[df];
+        p.cblk = tiles[t].blk;
       } else {
-        if (k > 1 && face_tblk[df] != p.fblk) return IBG_ERR_ARG;
+        if (k > 1 && tiles[t].blk != p.fblk) return IBG_ERR_ARG;
         p.fslot[k - 1] = sl;
-        p.fblk = face_tblk[df];
+        p.fblk = tiles[t].blk;
       }
     }
     rfp.push_back(p);
   }
+  if (!c->cfg.reflux) rfp.clear();   // the pairs are checked, and used only with the balance
   c->nrf = (int)rfp.size();
   // ---- domain ghosts: edge entries first, then corners (whose refcell is an
   // edge ghost)
@@ -1476,6 +1627,7 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
   UP(c->nb27, nb27);
   c->hcellblk = cellblk;
   UP(c->tiles, tiles);
+  UP(c->halo, halo);
   UP(c->tst, tst);
   UP(c->tvs, tvs);
   UP(c->rfp, rfp);

@@ -63,8 +63,8 @@ struct PhysR {
   R gm1, ig1;    // gama - 1 and its reciprocal
   R cpR;         // Cv / Rg + 1: enthalpy h = cpR p / roe + |u|^2 / 2
 };
-template <typename R>
-__device__ __forceinline__ PhysR<R> phys_r(const DevPhys &P) {
+template <typename R, class Q>
+__device__ __forceinline__ PhysR<R> phys_r(const Q &P) {
   PhysR<R> ph;
   ph.gama = (R)P.gama; ph.Rg = (R)P.Rg; ph.Cv = (R)P.Cv; ph.Ma = (R)P.Ma;
   ph.gm1 = (R)(P.gama - 1.0); ph.ig1 = (R)P.ig1;
@@ -209,11 +209,12 @@ __device__ __forceinline__ void from_face(double *f, int dir) {
 
 // Flux of an axis-aligned face.  Output: D == 2: (mass, x-mom, y-mom,
 // energy); D == 3: (mass, x, y, z momentum, energy).
-template <int D>
+template <int D, int DIR = -1>
 __device__ __forceinline__ void roe_flux(const Prim<double, D> &t0, const Prim<double, D> &t1,
                                          const Prim<double, D> &t2, const Prim<double, D> &t3,
                                          int dir, double area, const PhysR<double> &ph, int lim,
                                          double *flux) {
+  if (DIR >= 0) dir = DIR;
   roe_normal<D>(to_face<D>(t0, dir), to_face<D>(t1, dir), to_face<D>(t2, dir), to_face<D>(t3, dir),
                 area, ph, lim, flux);
   from_face<D>(flux, dir);
@@ -229,108 +230,137 @@ __device__ __forceinline__ void roe_flux(const Prim<double, D> &t0, const Prim<d
 // |dqi| < 1e-10 |dqii|, where both forms give qi to within 1e-10 dqii).
 // The error of this mode against the FP64 oracle is measured, not assumed.
 
-// van Albada in FP32 through the ratio r (as the reference forms it, with
-// its guards): r > 0 here, phi = (r^2 + r)/(r^2 + 1).  The one-reciprocal
-// form pr (dqi + dqii) / (dqi^2 + dqii^2) overflows in FP32 once both
+// Limited half slope 0.5 a phi(b / a) of FP32 (see half_slope above), as the
+// value q + or - it.  van Albada through the ratio r (as the reference forms
+// it, with its guards): r > 0 here, phi = (r^2 + r)/(r^2 + 1).  The
+// one-reciprocal form pr (a + b) / (a^2 + b^2) overflows in FP32 once both
 // differences fall below ~1e-19 (the square sum below 2^-126).
 __device__ __forceinline__ float fast_albada(float num, float den) {
   float r = num * f_rcp(den);
   if (!(r <= 1.0e10f)) r = (num > 0.0f) ? 1000000.0f : 0.0f;   // also NaN / inf
-  return (r * r + r) * f_rcp(r * r + 1.0f);
+  return fmaf(r, r, r) * f_rcp(fmaf(r, r, 1.0f));
+}
+template <bool kLeft>
+__device__ __forceinline__ float fast_slope(float q, float a, float b, int lim) {
+#pragma clang fp contract(off)
+  const float pr = a * b;
+  if (!(pr > 0.0f)) return q;
+  if (lim == 1) return fmaf(kLeft ? 0.5f * a : -0.5f * a, fast_albada(b, a), q);
+  return fmaf(kLeft ? pr : -pr, f_rcp(a + b), q);
 }
 
-__device__ __forceinline__ float fast_left(float q_i, float qi, float qi1, int lim) {
-  const float dqi = qi - q_i, dqii = qi1 - qi;
-  const float pr = dqi * dqii;
-  if (!(pr > 0.0f)) return qi;
-  if (lim == 1) return qi + 0.5f * dqi * fast_albada(dqii, dqi);
-  return qi + pr * f_rcp(dqi + dqii);
-}
-
-__device__ __forceinline__ float fast_right(float q_i, float qi, float qi1, int lim) {
-  const float dqi = qi - q_i, dqii = qi1 - qi;
-  const float pr = dqi * dqii;
-  if (!(pr > 0.0f)) return qi;
-  if (lim == 1) return qi - 0.5f * dqii * fast_albada(dqi, dqii);
-  return qi - pr * f_rcp(dqi + dqii);
-}
-
-template <int D>
+// DIR: the face's direction where the compiler knows it (block tiles), -1
+// where it is dir.  The fused operations are written out, so that both forms
+// round alike: the terms that a known direction drops are exact zeros and
+// products with one.
+template <int D, int DIR = -1>
 __device__ __forceinline__ void roe_flux(const Prim<float, D> &t0, const Prim<float, D> &t1,
                                          const Prim<float, D> &t2, const Prim<float, D> &t3,
                                          int dir, float area, const PhysR<float> &ph, int lim,
                                          float *flux) {
+#pragma clang fp contract(off)
   const float gama = ph.gama, Rg = ph.Rg, Cv = ph.Cv;
-  const float lr = fast_left(t0.r, t1.r, t2.r, lim), rr = fast_right(t1.r, t2.r, t3.r, lim);
-  const float lu = fast_left(t0.u, t1.u, t2.u, lim), ru = fast_right(t1.u, t2.u, t3.u, lim);
-  const float lvv = fast_left(t0.v, t1.v, t2.v, lim), rvv = fast_right(t1.v, t2.v, t3.v, lim);
-  float lw = 0.0f, rw = 0.0f;
-  if (D == 3) { lw = fast_left(t0.w, t1.w, t2.w, lim); rw = fast_right(t1.w, t2.w, t3.w, lim); }
-  const float lp = fast_left(t0.p, t1.p, t2.p, lim), rp = fast_right(t1.p, t2.p, t3.p, lim);
+  float lr, rr, lu, ru, lvv, rvv, lw = 0.0f, rw = 0.0f, lp, rp;
+  auto muscl32 = [&](float q0, float q1, float q2, float q3, float &l, float &r) {
+    const float d0 = q1 - q0, d1 = q2 - q1, d2 = q3 - q2;
+    l = fast_slope<true>(q1, d0, d1, lim);
+    r = fast_slope<false>(q2, d2, d1, lim);
+  };
+  muscl32(t0.r, t1.r, t2.r, t3.r, lr, rr);
+  muscl32(t0.u, t1.u, t2.u, t3.u, lu, ru);
+  muscl32(t0.v, t1.v, t2.v, t3.v, lvv, rvv);
+  if (D == 3) muscl32(t0.w, t1.w, t2.w, t3.w, lw, rw);
+  muscl32(t0.p, t1.p, t2.p, t3.p, lp, rp);
   const float ilr = f_rcp(lr), irr = f_rcp(rr);
   const float iRg = f_rcp(Rg);
-  const float lT = lp * ilr * iRg, rT = rp * irr * iRg;
-  const float lke = (D == 3) ? 0.5f * (lu * lu + lvv * lvv + lw * lw) : 0.5f * (lu * lu + lvv * lvv);
-  const float rke = (D == 3) ? 0.5f * (ru * ru + rvv * rvv + rw * rw) : 0.5f * (ru * ru + rvv * rvv);
-  const float le = Cv * lT + lke, re = Cv * rT + rke;
-  const float lv = dir == 0 ? lu : (dir == 1 ? lvv : lw);
-  const float rv = dir == 0 ? ru : (dir == 1 ? rvv : rw);
-  const float kx = dir == 0 ? 1.0f : 0.0f, ky = dir == 1 ? 1.0f : 0.0f, kz = dir == 2 ? 1.0f : 0.0f;
+  const float plr = lp * ilr, prr = rp * irr;
+  const float rT = prr * iRg;
+  float lq = fmaf(lu, lu, lvv * lvv), rq = fmaf(ru, ru, rvv * rvv);
+  if (D == 3) { lq = fmaf(lw, lw, lq); rq = fmaf(rw, rw, rq); }
+  const float le = fmaf(0.5f, lq, Cv * (plr * iRg)), re = fmaf(0.5f, rq, Cv * rT);
+  auto pick = [&](float x, float y, float z) {
+    if (DIR >= 0) return DIR == 0 ? x : (DIR == 1 ? y : z);
+    return dir == 0 ? x : (dir == 1 ? y : z);
+  };
+  const float lv = pick(lu, lvv, lw), rv = pick(ru, rvv, rw);
+  const float k0 = dir == 0 ? 1.0f : 0.0f, k1 = dir == 1 ? 1.0f : 0.0f, k2 = dir == 2 ? 1.0f : 0.0f;
+  // k x + y with the direction's k = 0 or 1
+  auto kfma = [&](int d, float k, float x, float y) {
+    if (DIR >= 0) return DIR == d ? x + y : y;
+    return fmaf(k, x, y);
+  };
   // central part 1/2 (F_L + F_R) A
   const float ha = 0.5f * area;
-  const float p0 = (lr * lv + rr * rv) * ha;
-  const float p1 = (lr * lu * lv + lp * kx + rr * ru * rv + rp * kx) * ha;
-  const float p2 = (lr * lvv * lv + lp * ky + rr * rvv * rv + rp * ky) * ha;
-  const float p3 = (lr * lw * lv + lp * kz + rr * rw * rv + rp * kz) * ha;
-  const float p4 = ((lp + le * lr) * lv + (rp + re * rr) * rv) * ha;
+  const float p0 = fmaf(lr, lv, rr * rv);
+  auto mom = [&](int d, float k, float l, float r) {
+    float x;
+    if (DIR >= 0) x = DIR == d ? fmaf(lr * l, lv, lp) : (lr * l) * lv;
+    else x = fmaf(lr * l, lv, lp * k);
+    return kfma(d, k, rp, fmaf(rr * r, rv, x));
+  };
+  const float p1 = mom(0, k0, lu, ru), p2 = mom(1, k1, lvv, rvv);
+  const float p4 = fmaf(fmaf(le, lr, lp), lv, fmaf(re, rr, rp) * rv);
   const float droe = rr - lr, dp = rp - lp;
-  const float du0 = ru - lu, du1 = rvv - lvv, du2 = rw - lw;
   const float dubar = rv - lv;
   // Roe average
   const float r2lroe = f_sqrt(rr * ilr);
   const float r2l0 = f_rcp(1.0f + r2lroe);
-  const float h_left = le + lp * ilr, h_right = re + rp * irr;
+  const float h_left = fmaf(lp, ilr, le), h_right = fmaf(rp, irr, re);
   const float a_roe = f_sqrt(lr * rr);
-  const float a_u = (lu + ru * r2lroe) * r2l0;
-  const float a_v = (lvv + rvv * r2lroe) * r2l0;
-  const float a_w = (D == 3) ? (lw + rw * r2lroe) * r2l0 : 0.0f;
-  const float a_h = (h_left + h_right * r2lroe) * r2l0;
-  const float q2 = (D == 3) ? (a_u * a_u + a_v * a_v + a_w * a_w) : (a_u * a_u + a_v * a_v);
-  const float csquare = (gama - 1.0f) * (a_h - 0.5f * q2);
+  const float a_u = fmaf(ru, r2lroe, lu) * r2l0;
+  const float a_v = fmaf(rvv, r2lroe, lvv) * r2l0;
+  const float a_w = (D == 3) ? fmaf(rw, r2lroe, lw) * r2l0 : 0.0f;
+  const float a_h = fmaf(h_right, r2lroe, h_left) * r2l0;
+  float q2 = fmaf(a_u, a_u, a_v * a_v);
+  if (D == 3) q2 = fmaf(a_w, a_w, q2);
+  const float csquare = (gama - 1.0f) * fmaf(-0.5f, q2, a_h);
   const float a_c = f_sqrt(csquare);
-  const float a_ubar = dir == 0 ? a_u : (dir == 1 ? a_v : a_w);
+  const float a_ubar = pick(a_u, a_v, a_w);
   const float icsq = f_rcp(csquare);
-  const float namda3 = fabsf(a_ubar);
   const float coef12 = 0.5f * icsq * area;
-  const float roe0cxdubar = a_roe * a_c * dubar;
-  const float faa = area * namda3;
-  const float al0 = faa * (droe - dp * icsq);
+  const float rc = a_roe * a_c;
+  const float faa = area * fabsf(a_ubar);
+  const float al0 = faa * fmaf(-dp, icsq, droe);
   // all-speed eigenvalues (NS_Solver.H:66-77)
-  const float T_a = (lT + rT) * 0.5f;
+  const float T_a = fmaf(plr, iRg, rT) * 0.5f;
   const float V_a = (lv + rv) * 0.5f;
   float f_Ma = fabsf(V_a) * f_rcp(f_sqrt(gama * Rg * T_a));
   f_Ma = f_Ma < ph.Ma ? ph.Ma : f_Ma;
   f_Ma = f_Ma > 1.0f ? 1.0f : f_Ma;
   const float s0 = (1.0f - f_Ma) * (1.0f - f_Ma);
-  const float namda0 = f_sqrt(4.0f * csquare * f_Ma + s0 * a_ubar * a_ubar);
-  const float namda1 = fabsf(0.5f * ((1.0f + f_Ma) * a_ubar + namda0));
-  const float namda2 = fabsf(0.5f * ((1.0f + f_Ma) * a_ubar - namda0));
-  const float al1 = coef12 * namda1 * (dp + roe0cxdubar);
-  const float al2 = coef12 * namda2 * (dp - roe0cxdubar);
-  const float al3 = al0 + al1 + al2;
-  const float al4 = a_c * (al1 - al2);
-  const float al5 = faa * (a_roe * (du0 - kx * dubar));
-  const float al6 = faa * (a_roe * (du1 - ky * dubar));
-  const float al7 = (D == 3) ? faa * (a_roe * (du2 - kz * dubar)) : 0.0f;
+  const float namda0 = f_sqrt(fmaf(4.0f * csquare, f_Ma, s0 * a_ubar * a_ubar));
+  const float n1 = coef12 * fabsf(0.5f * fmaf(1.0f + f_Ma, a_ubar, namda0));
+  const float n2 = coef12 * fabsf(0.5f * fmaf(1.0f + f_Ma, a_ubar, -namda0));
+  const float x1 = fmaf(rc, dubar, dp), x2 = fmaf(-rc, dubar, dp);
+  const float al3 = fmaf(n2, x2, fmaf(n1, x1, al0));
+  const float al4 = a_c * fmaf(n1, x1, -(n2 * x2));
+  // tangential jumps: zero along the normal
+  auto jump = [&](int d, float k, float du) {
+    if (DIR >= 0) return DIR == d ? 0.0f : a_roe * du;
+    return a_roe * fmaf(-k, dubar, du);
+  };
+  const float j0 = jump(0, k0, ru - lu), j1 = jump(1, k1, rvv - lvv);
+  const float j2 = (D == 3) ? jump(2, k2, rw - lw) : 0.0f;
+  auto upw = [&](int d, float k, float vel, float j) {
+    float t;
+    if (DIR >= 0) t = DIR == d ? fmaf(vel, al3, al4) : vel * al3;
+    else t = fmaf(vel, al3, k * al4);
+    return (DIR >= 0 && DIR == d) ? t : fmaf(faa, j, t);
+  };
   const float ig1 = f_rcp(gama - 1.0f);
-  flux[0] = p0 - al3;
-  flux[1] = p1 - (a_u * al3 + kx * al4 + al5);
-  flux[2] = p2 - (a_v * al3 + ky * al4 + al6);
+  flux[0] = fmaf(p0, ha, -al3);
+  flux[1] = fmaf(p1, ha, -upw(0, k0, a_u, j0));
+  flux[2] = fmaf(p2, ha, -upw(1, k1, a_v, j1));
+  float en = fmaf(a_h, al3, a_ubar * al4);
+  if (DIR != 0) en = fmaf(a_u, faa * j0, en);
+  if (DIR != 1) en = fmaf(a_v, faa * j1, en);
+  if (D == 3 && DIR != 2) en = fmaf(a_w, faa * j2, en);
+  en = fmaf(-(csquare * ig1), al0, en);
   if (D == 3) {
-    flux[3] = p3 - (a_w * al3 + kz * al4 + al7);
-    flux[4] = p4 - (a_h * al3 + a_ubar * al4 + a_u * al5 + a_v * al6 + a_w * al7 - csquare * ig1 * al0);
+    flux[3] = fmaf(mom(2, k2, lw, rw), ha, -upw(2, k2, a_w, j2));
+    flux[4] = fmaf(p4, ha, -en);
   } else {
-    flux[3] = p4 - (a_h * al3 + a_ubar * al4 + a_u * al5 + a_v * al6 - csquare * ig1 * al0);
+    flux[3] = fmaf(p4, ha, -en);
   }
 }
 
@@ -502,17 +532,70 @@ __device__ __forceinline__ void visc_flux(const VelT<R> &L, const VelT<R> &Rr, R
   }
 }
 
-// The same from the stencil cells' states.
+// The same in 2D FP32 with its fused operations written out, so that the
+// form with a known direction (DIR, block tiles) rounds as the one with a
+// direction from the face list (DIR = -1).  iL, iR: 1 / (roe Rg) of the two
+// cells; tu, tv: the tangential stencil's velocities (its temperatures do
+// not enter: the heat flux is along the normal).
+template <int DIR>
+__device__ __forceinline__ void visc_flux_2d(const Prim<float, 2> &L, const Prim<float, 2> &Rr,
+                                             float iL, float iR, const float *tu, const float *tv,
+                                             int dir, const ViscPhys<float, 2> &vp, float *out,
+                                             bool turb, float nuL, float nuR, float *mflux) {
+#pragma clang fp contract(off)
+  const bool x = DIR >= 0 ? DIR == 0 : dir == 0;
+  const float nu = Rr.u - L.u, nv = Rr.v - L.v;
+  const float au = 0.25f * (tu[0] + tu[1] - tu[2] - tu[3]);
+  const float av = 0.25f * (tv[0] + tv[1] - tv[2] - tv[3]);
+  const float TR = iR * Rr.p;
+  const float nT = fmaf(-iL, L.p, TR), sT = fmaf(iL, L.p, TR);   // TR -+ TL
+  const float ih = x ? vp.ih0 : vp.ih1, area = x ? vp.ar0 : vp.ar1;
+  const float gux = x ? nu : au, guy = x ? au : nu, gvx = x ? nv : av, gvy = x ? av : nv;
+  const float ftemp = 0.5f * sT;
+  float mu0 = f_sqrt(ftemp * ftemp * ftemp) * ((1.0f + vp.SoT) * f_rcp(fmaf(0.5f, sT, vp.SoT)));
+  float qk0 = vp.qk * mu0;
+  if (turb) {
+    const float fvis = (nuL + nuR) * 0.5f;
+    const float froe = (L.r + Rr.r) * 0.5f;
+    const float nul = mu0 * f_rcp(froe);
+    float bigx = fvis * f_rcp(nul);
+    if (bigx < 0.0f) bigx = 0.0f;
+    const float b2 = bigx * bigx;
+    const float rf = froe * (bigx * b2 * f_rcp(fmaf(bigx, b2, (float)SA::cv1three)));
+    qk0 = fmaf(vp.qk, mu0, rf * fvis * vp.iqkt);
+    mu0 = fmaf(rf, fvis, mu0);
+    *mflux = ((fvis + nul) * ((nuR - nuL) * ih)) * c_rcp((float)SA::segma) * area;
+  }
+  const float dvy = gvy * vp.ih1;
+  const float dv3 = fmaf(gux, vp.ih0, dvy) * c_rcp(3.0f);
+  const float dn = x ? gux * vp.ih0 : dvy;
+  const float tnn = 2.0f * mu0 * (dn - dv3) * vp.iRe;   // tauxx or tauyy
+  const float txy = mu0 * vp.iRe * fmaf(gvx, vp.ih0, guy * vp.ih1);
+  const float t1 = x ? tnn : txy, t2 = x ? txy : tnn;
+  const float fu = (L.u + Rr.u) * 0.5f, fv = (L.v + Rr.v) * 0.5f;
+  out[0] = 0.0f;
+  out[1] = t1 * area;
+  out[2] = t2 * area;
+  out[3] = fmaf(qk0, nT * ih, fmaf(fu, t1, fv * t2)) * area;
+}
+
+// The viscous flux from the stencil cells' states.
 template <typename R, int D>
 __device__ __forceinline__ void visc_flux_cells(const Prim<R, D> &L, const Prim<R, D> &Rr,
                                                 const Prim<R, D> *t, int d,
                                                 const ViscPhys<R, D> &vp, R *out, bool turb, R nuL,
                                                 R nuR, R *mflux) {
-  VelT<R> vt[(D == 3) ? 8 : 4];
+  if constexpr (D == 2 && sizeof(R) == 4) {
+    const float tu[4] = {t[0].u, t[1].u, t[2].u, t[3].u}, tv[4] = {t[0].v, t[1].v, t[2].v, t[3].v};
+    visc_flux_2d<-1>(L, Rr, f_rcp(L.r * vp.Rg), f_rcp(Rr.r * vp.Rg), tu, tv, d, vp, out, turb, nuL,
+                     nuR, mflux);
+  } else {
+    VelT<R> vt[(D == 3) ? 8 : 4];
 #pragma unroll
-  for (int k = 0; k < ((D == 3) ? 8 : 4); ++k) vt[k] = vel_t<R, D>(t[k], vp.Rg);
-  visc_flux<R, D>(vel_t<R, D>(L, vp.Rg), vel_t<R, D>(Rr, vp.Rg), L.r, Rr.r, vt, d, vp, out, turb,
-                  nuL, nuR, mflux);
+    for (int k = 0; k < ((D == 3) ? 8 : 4); ++k) vt[k] = vel_t<R, D>(t[k], vp.Rg);
+    visc_flux<R, D>(vel_t<R, D>(L, vp.Rg), vel_t<R, D>(Rr, vp.Rg), L.r, Rr.r, vt, d, vp, out, turb,
+                    nuL, nuR, mflux);
+  }
 }
 
 // exp, x^6 and x^(1/6) of the SA functions.  FP32: (x^2)^3 and the hardware

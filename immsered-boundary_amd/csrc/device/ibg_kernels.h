@@ -7,6 +7,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "ibg_block.h"
 #include "ibg_common.h"
 #include "ibg_flux.h"
 #include "ibg_mlp.h"
@@ -16,6 +17,11 @@
 namespace ibg {
 
 constexpr int kTile = 256;   // cells per workgroup of the tiled kernels (max)
+
+__device__ __forceinline__ TileInfo tile_info(const TileInfo *tiles, int t) {
+  const auto *p = uni(tiles) + t;
+  return TileInfo{p->cell0, p->ncell, p->face0, p->nface, p->blk, p->halo0, 0, 0};
+}
 
 // ------------------------------------------------------------ pack access
 template <typename R, int D>
@@ -98,6 +104,7 @@ struct ViscArgs {
   const int4 *tst;           // L, R from .y, .z
   const int4 *tvs;           // [nface][D-1] tangential stencil
   const int8_t *tdir;
+  const int *halo;           // halo lists of the block tiles
   const uint16_t *slots;
   const BlkInfo *blk;
   const DevPhys *phys;
@@ -113,8 +120,8 @@ struct ViscArgs {
   const R *rbalv;
 };
 
-template <typename R, int D>
-__device__ __forceinline__ ViscPhys<R, D> visc_phys(const BlkInfo &bi, const DevPhys &P) {
+template <typename R, int D, class B, class Q>
+__device__ __forceinline__ ViscPhys<R, D> visc_phys(B &bi, Q &P) {
   ViscPhys<R, D> vp;
   vp.Rg = (R)P.Rg; vp.iRe = std::is_same<R, float>::value ? c_rcp((R)P.Re) : (R)P.iRe; vp.qk = (R)P.qk; vp.SoT = (R)P.SoT;
   vp.ih0 = (R)bi.invh[0]; vp.ih1 = (R)bi.invh[1]; vp.ih2 = (R)bi.invh[2];
@@ -166,8 +173,8 @@ __device__ __forceinline__ void visc_prep_tile(const ViscArgs<R, D> &a, const Ti
   V *fl4 = reinterpret_cast<V *>(smem_raw);
   R *fl1 = reinterpret_cast<R *>(smem_raw + sizeof(V) * (size_t)ti.nface);
   R *mfl = reinterpret_cast<R *>(smem_raw + (sizeof(V) + (D == 3 ? sizeof(R) : 0)) * (size_t)ti.nface);
-  const BlkInfo &bi = a.blk[ti.blk];
-  const DevPhys &P = a.phys[bi.case_id];
+  auto &bi = uni(a.blk)[ti.blk];
+  auto &P = uni(a.phys)[bi.case_id];
   if (a.viscous) {
     const ViscPhys<R, D> vp = visc_phys<R, D>(bi, P);
     for (int f = threadIdx.x; f < ti.nface; f += blockDim.x) {
@@ -229,12 +236,166 @@ __device__ __forceinline__ void visc_prep_tile(const ViscArgs<R, D> &a, const Ti
   if (a.turb) a.mutf[c] = (R)n_div(n_div(tot, bi.vol), P.Re);
 }
 
+// ---------------------------------------------------------- block tiles
+// The LDS of a block tile (ibg_block.h).
+template <typename R>
+struct BlockLds {
+  typename V4<R>::T *fx, *fy;   // fluxes of the x and y faces
+  typename V4<R>::T *S;         // states of the box
+  R *nu, *T;                    // working variable (SA); temperature (FP64) or
+                                // 1 / (roe Rg) (FP32) for the viscous flux
+};
+template <typename R>
+__device__ __forceinline__ BlockLds<R> block_lds(unsigned char *smem, bool turb) {
+  BlockLds<R> b;
+  b.fx = reinterpret_cast<typename V4<R>::T *>(smem);
+  b.fy = b.fx + kFxSlots;
+  b.S = b.fx + kFluxSlots;
+  b.nu = reinterpret_cast<R *>(b.S + kBoxCells);
+  b.T = b.nu + (turb ? kBoxCells : 0);
+  return b;
+}
+template <typename R>
+__device__ __forceinline__ Prim<R, 2> box_prim(const BlockLds<R> &b, int p) {
+  const typename V4<R>::T q = b.S[p];
+  return Prim<R, 2>{q.x, q.y, q.z, R(0), q.w};
+}
+
+// The square and its first nhalo halo entries into LDS (256 threads; the
+// caller syncs).  kT: BlockLds::T too.
+template <typename R, bool kT>
+__device__ __forceinline__ void block_load(const Pack<R, 2> &W, const R *nu, bool turb,
+                                           const int *halo, const TileInfo &ti, int nhalo, R Rg,
+                                           const BlockLds<R> &b) {
+  const int i = threadIdx.x;
+  const int c = ti.cell0 + i;
+  int hc = 0;
+  if (i < nhalo) hc = halo[ti.halo0 + i];
+  auto put = [&](int p, const typename V4<R>::T &q, R n) {
+    if constexpr (kT && sizeof(R) == 4) b.T[p] = f_rcp(q.x * Rg);
+    else if constexpr (kT) b.T[p] = v_div(q.w, q.x * Rg);
+    b.S[p] = q;
+    if (turb) b.nu[p] = n;
+  };
+  int x, y;
+  blk_xy(i, x, y);
+  const typename V4<R>::T q = W.a[c];
+  const R n = turb ? nu[c] : R(0);
+  if (i < nhalo) {
+    const typename V4<R>::T qh = W.a[hc];
+    const R nh = turb ? nu[hc] : R(0);
+    put(halo_pos(i), qh, nh);
+  }
+  put(box_pos(x, y), q, n);
+}
+
+// Face f of a block tile in direction d: f < 256 the low face of cell f,
+// then the high faces of the last row; its high-side cell's coordinates
+template <int d>
+__device__ __forceinline__ void block_face(int f, int &x, int &y) {
+  blk_xy(f & 255, x, y);
+  if (f >= kBlkCells) {
+    x = d == 0 ? kBlkN : f - kBlkCells;
+    y = d == 0 ? f - kBlkCells : kBlkN;
+  }
+}
+
+// Viscous fluxes of the faces of direction d into LDS, the working
+// variable's face flux in the mass slot (the viscous mass flux is zero).
+template <typename R, int d>
+__device__ __forceinline__ void block_visc_faces(const BlockLds<R> &b, const ViscPhys<R, 2> &vp,
+                                                 bool turb) {
+  constexpr int st = d == 0 ? 1 : kBoxP, tt = d == 0 ? kBoxP : 1;
+  // the last row's faces go to another wave in the y pass than in the x pass
+#pragma unroll 1
+  for (int f = (threadIdx.x + (d == 0 ? 0 : 192)) & 255; f < kBlkCells + kBlkN; f += kBlkCells) {
+    int x, y;
+    block_face<d>(f, x, y);
+    const int p = box_pos(x, y), l = p - st;
+    R out[4], mf = R(0);
+    const R nl = turb ? b.nu[l] : R(0), nr = turb ? b.nu[p] : R(0);
+    const int tp[4] = {l + tt, p + tt, l - tt, p - tt};
+    if constexpr (sizeof(R) == 4) {
+      float tu[4], tv[4];
+#pragma unroll
+      for (int k = 0; k < 4; ++k) { tu[k] = b.S[tp[k]].y; tv[k] = b.S[tp[k]].z; }
+      visc_flux_2d<d>(box_prim<R>(b, l), box_prim<R>(b, p), b.T[l], b.T[p], tu, tv, d, vp, out, turb,
+                      nl, nr, &mf);
+    } else {
+      auto cell = [&](int q) {
+        const typename V4<R>::T s = b.S[q];
+        return VelT<R>{s.y, s.z, R(0), b.T[q]};
+      };
+      const VelT<R> t[4] = {cell(tp[0]), cell(tp[1]), cell(tp[2]), cell(tp[3])};
+      visc_flux<R, 2>(cell(l), cell(p), b.S[l].x, b.S[p].x, t, d, vp, out, turb, nl, nr, &mf);
+    }
+    typename V4<R>::T o;
+    o.x = mf; o.y = out[1]; o.z = out[2]; o.w = out[3];
+    (d == 0 ? b.fx : b.fy)[y * kBoxP + x] = o;
+  }
+}
+
+// Rv and the working variable's face term of this thread's cell from the
+// face fluxes in LDS.
+template <typename R, class B, class Q>
+__device__ __forceinline__ void block_visc_cell(const ViscArgs<R, 2> &a, const TileInfo &ti, B &bi,
+                                                Q &P, const BlockLds<R> &b) {
+  using V = typename V4<R>::T;
+  const int c = ti.cell0 + threadIdx.x;
+  int x, y;
+  blk_xy(threadIdx.x, x, y);
+  double s[4] = {0.0, 0.0, 0.0, 0.0}, tot = 0.0;
+  if (a.viscous) {
+    const int k = y * kBoxP + x;
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      const V lo = d == 0 ? b.fx[k] : b.fy[k], hi = d == 0 ? b.fx[k + 1] : b.fy[k + kBoxP];
+      s[1] += (double)hi.y - (double)lo.y;
+      s[2] += (double)hi.z - (double)lo.z;
+      s[3] += (double)hi.w - (double)lo.w;
+      if (a.turb) {
+        tot += -(double)lo.x;
+        tot += (double)hi.x;
+      }
+    }
+  }
+  const R rv[4] = {(R)s[0], (R)s[1], (R)s[2], (R)s[3]};
+  vstore<R, 2>(a.Rv, c, rv);
+  if (a.turb) a.mutf[c] = (R)n_div(n_div(tot, bi.vol), P.Re);
+}
+
+// The viscous pass of a block tile (visc_prep_tile's work).
+template <typename R>
+__device__ __forceinline__ void visc_prep_block(const ViscArgs<R, 2> &a, const TileInfo &ti,
+                                                unsigned char *smem_raw, int *halt, bool herr) {
+  auto &bi = uni(a.blk)[ti.blk];
+  auto &P = uni(a.phys)[bi.case_id];
+  const BlockLds<R> b = block_lds<R>(smem_raw, a.turb);
+  if (a.viscous) {
+    block_load<R, true>(a.W, a.nu, a.turb, a.halo, ti, kHaloC, (R)P.Rg, b);
+    __syncthreads();
+    const ViscPhys<R, 2> vp = visc_phys<R, 2>(bi, P);
+    block_visc_faces<R, 0>(b, vp, a.turb);
+    block_visc_faces<R, 1>(b, vp, a.turb);
+  }
+  if (threadIdx.x == 0) *halt = herr ? 1 : 0;
+  __syncthreads();
+  if (*halt) return;
+  block_visc_cell<R>(a, ti, bi, P, b);
+}
+
 template <typename R, int D>
 __global__ void __launch_bounds__(kTile) k_visc_prep(ViscArgs<R, D> a) {
   extern __shared__ __align__(32) unsigned char smem_raw[];
   __shared__ int halt;
   const bool herr = halted(a.err);
-  const TileInfo ti = a.tiles[dispatch_tile()];
+  const TileInfo ti = tile_info(a.tiles, dispatch_tile());
+  if constexpr (D == 2) {
+    if (ti.halo0 >= 0) {
+      visc_prep_block<R>(a, ti, smem_raw, &halt, herr);
+      return;
+    }
+  }
   visc_prep_tile<R, D>(a, ti, smem_raw, &halt, herr);
 }
 
@@ -243,6 +404,7 @@ struct StageArgs {
   const TileInfo *tiles;
   const int4 *tst;           // tile face stencil LL,L,R,RR
   const int8_t *tdir;        // tile face direction
+  const int *halo;           // halo lists of the block tiles
   const uint16_t *slots;     // [Nn][2D] tile-local face slot of each cell face
   const uint8_t *flags;      // [Nn]
   const BlkInfo *blk;
@@ -380,7 +542,8 @@ __device__ __forceinline__ double wave_slots16(double *v) {
   const bool sum = (lane & 32) != 0;
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
-    const double keep = sum ? v[j + 8] : v[j], send = sum ? v[j] : v[j + 8];
+    const double lo = v[j], hi = v[j + 8];
+    const double keep = sum ? hi : lo, send = sum ? lo : hi;
     const double o = __shfl_xor(send, 32, 64);
     v[j] = sum ? keep + o : fmax(keep, o);
   }
@@ -389,7 +552,8 @@ __device__ __forceinline__ double wave_slots16(double *v) {
     const bool up = (lane & off) != 0;
 #pragma unroll
     for (int j = 0; j < m; ++j) {
-      const double keep = up ? v[j + m] : v[j], send = up ? v[j] : v[j + m];
+      const double lo = v[j], hi = v[j + m];
+      const double keep = up ? hi : lo, send = up ? lo : hi;
       const double o = __shfl_xor(send, off, 64);
       v[j] = sum ? keep + o : fmax(keep, o);
     }
@@ -403,76 +567,135 @@ __device__ __forceinline__ double wave_slots16(double *v) {
   return x;
 }
 
+// Static LDS of a stage workgroup.  halt: the error word is loaded at kernel
+// start, its load in flight while the face phase runs, published by thread 0
+// just before the face phase's barrier and tested after it (the face phase
+// writes only LDS).
+struct StageShared {
+  int halt;
+  unsigned mlc[2];   // learned closure: network / fallback cells of this tile
+  double red[kRpart][kTile / 64];
+};
+
 // One tile.  WRES: the network's weights are resident at a.mlw_off
 // (persistent schedule); otherwise the ML instantiation stages them after
-// the face fluxes, over the face-cell indices (dead by then).
-template <typename R, int D, bool ML, bool WRES>
-__device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, int tile) {
+// the face fluxes, over what is dead by then (a general tile's face-cell
+// indices, a block tile's states).  BLK: a block tile (ibg_block.h).
+template <typename R, int D, bool ML, bool WRES, bool BLK>
+__device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileInfo &ti, int tile,
+                                           bool herr, StageShared &sh) {
   constexpr bool wres = WRES;
   constexpr int NV = D + 2;
   constexpr bool kMixed = std::is_same<R, float>::value;
   using V = typename V4<R>::T;
   extern __shared__ __align__(32) unsigned char smem_raw[];
-  // the error word: loaded here, its load in flight while the face phase
-  // runs, published by thread 0 just before the face phase's barrier and
-  // tested after it (the face phase writes only LDS)
-  __shared__ int halt;
-  __shared__ unsigned mlc[2];   // learned closure: network / fallback cells of this tile
-  const bool herr = halted(a.err);
+  int &halt = sh.halt;
+  unsigned(&mlc)[2] = sh.mlc;
+  auto &red = sh.red;
   if (ML && threadIdx.x == 0) { mlc[0] = 0u; mlc[1] = 0u; }
-  const TileInfo ti = a.tiles[tile];
-  if constexpr (kFuseVisc<R, D>) {
-    if (a.fuse_visc) {
-      // Rv and mutf of this tile's cells from the step-start state (the
-      // buffer this stage reads); each thread reads back only its own
-      // cell's entries in phase 2, so no other workgroup is involved
-      visc_prep_tile<R, D>(a.va, ti, smem_raw, &halt, herr);
-      if (halt) return;  // uniform: read after the barrier in visc_prep_tile
-      __syncthreads();   // the face arrays are reused by phase 1
-    }
-  }
+  auto &bi = uni(a.blk)[ti.blk];
+  auto &P = uni(a.phys)[bi.case_id];
+  const PhysR<R> ph = phys_r<R>(P);
   V *fl4 = reinterpret_cast<V *>(smem_raw);
   R *fl1 = reinterpret_cast<R *>(smem_raw + sizeof(V) * (size_t)ti.nface);   // 3D 5th value
   // SA: the low / high cell of each face; the cell phase gathers their
   // velocity and working variable (cache hits: phase 1 has just read them)
   int *fL = reinterpret_cast<int *>(smem_raw + (sizeof(V) + (D == 3 ? sizeof(R) : 0)) * (size_t)ti.nface);
   int *fR = fL + ti.nface;
-  __shared__ double red[kRpart][kTile / 64];
-
-  const BlkInfo &bi = a.blk[ti.blk];
-  const DevPhys &P = a.phys[bi.case_id];
-  const PhysR<R> ph = phys_r<R>(P);
-  const R areas[3] = {(R)bi.area[0], (R)bi.area[1], (R)bi.area[2]};
-
-  for (int f = threadIdx.x; f < ti.nface; f += blockDim.x) {
-    const int4 st = a.tst[ti.face0 + f];
-    const int dir = a.tdir[ti.face0 + f];
-    const Prim<R, D> q0 = pload<R, D>(a.Win, st.x);
-    const Prim<R, D> q1 = pload<R, D>(a.Win, st.y);
-    const Prim<R, D> q2 = pload<R, D>(a.Win, st.z);
-    const Prim<R, D> q3 = pload<R, D>(a.Win, st.w);
-    R flux[NV];
-    roe_flux<D>(q0, q1, q2, q3, dir, areas[dir], ph, a.limiter, flux);
-    if (a.rbal) {
-      // a coarse/fine face of the optional balance: its balanced flux
-      const int q = a.tmod[ti.face0 + f];
-      if (q >= 0)
-        for (int v = 0; v < NV; ++v) flux[v] = a.rbal[(size_t)q * NV + v];
+  const BlockLds<R> bl = block_lds<R>(smem_raw, a.turb);
+  // this thread's cell in a block tile, formed anew at each use (held across
+  // the network it costs the ML instantiation registers it spills)
+  auto my_xy = [&](int &x, int &y) {
+    int i = threadIdx.x;
+    asm volatile("" : "+v"(i));
+    blk_xy(i, x, y);
+  };
+  if constexpr (BLK) {
+    bool loaded = false;
+    if constexpr (kFuseVisc<R, D>) {
+      if (a.fuse_visc && a.va.viscous) {
+        block_load<R, true>(a.Win, a.nuin, a.turb, a.halo, ti, kHalo, (R)P.Rg, bl);
+        __syncthreads();
+        const ViscPhys<R, 2> vp = visc_phys<R, 2>(bi, P);
+        block_visc_faces<R, 0>(bl, vp, a.turb);
+        block_visc_faces<R, 1>(bl, vp, a.turb);
+        loaded = true;
+      }
+      if (a.fuse_visc) {
+        // each thread reads back only its own cell's entries in phase 2
+        if (threadIdx.x == 0) halt = herr ? 1 : 0;
+        __syncthreads();
+        if (halt) return;
+        block_visc_cell<R>(a.va, ti, bi, P, bl);
+        __syncthreads();   // the face arrays are reused by phase 1
+      }
     }
-    V o;
-    o.x = flux[0]; o.y = flux[1]; o.z = flux[2]; o.w = flux[3];
-    fl4[f] = o;
-    if (D == 3) fl1[f] = flux[4];
-    if (a.turb) {
-      fL[f] = st.y;
-      fR[f] = st.z;
+    if (!loaded) {
+      block_load<R, false>(a.Win, a.nuin, a.turb, a.halo, ti, kHalo, R(0), bl);
+      __syncthreads();
+    }
+    // phase 1: the low face of every cell and the last row's high faces,
+    // which go to another wave in the y pass than in the x pass
+    auto faces = [&](auto dc) {
+      constexpr int d = decltype(dc)::value;
+      constexpr int st = d == 0 ? 1 : kBoxP;
+#pragma unroll 1
+      for (int f = (threadIdx.x + (d == 0 ? 0 : 192)) & 255; f < kBlkCells + kBlkN; f += kBlkCells) {
+        int x, y;
+        block_face<d>(f, x, y);
+        const int p = box_pos(x, y);
+        R flux[4];
+        roe_flux<2, d>(box_prim<R>(bl, p - 2 * st), box_prim<R>(bl, p - st), box_prim<R>(bl, p),
+                       box_prim<R>(bl, p + st), d, (R)bi.area[d], ph, a.limiter, flux);
+        V o;
+        o.x = flux[0]; o.y = flux[1]; o.z = flux[2]; o.w = flux[3];
+        (d == 0 ? bl.fx : bl.fy)[y * kBoxP + x] = o;
+      }
+    };
+    faces(std::integral_constant<int, 0>());
+    faces(std::integral_constant<int, 1>());
+  } else {
+    if constexpr (kFuseVisc<R, D>) {
+      if (a.fuse_visc) {
+        // Rv and mutf of this tile's cells from the step-start state (the
+        // buffer this stage reads); each thread reads back only its own
+        // cell's entries in phase 2, so no other workgroup is involved
+        visc_prep_tile<R, D>(a.va, ti, smem_raw, &halt, herr);
+        if (halt) return;  // uniform: read after the barrier in visc_prep_tile
+        __syncthreads();   // the face arrays are reused by phase 1
+      }
+    }
+    const R ar0 = (R)bi.area[0], ar1 = (R)bi.area[1], ar2 = (R)bi.area[2];
+    for (int f = threadIdx.x; f < ti.nface; f += blockDim.x) {
+      const int4 st = a.tst[ti.face0 + f];
+      const int dir = a.tdir[ti.face0 + f];
+      const Prim<R, D> q0 = pload<R, D>(a.Win, st.x);
+      const Prim<R, D> q1 = pload<R, D>(a.Win, st.y);
+      const Prim<R, D> q2 = pload<R, D>(a.Win, st.z);
+      const Prim<R, D> q3 = pload<R, D>(a.Win, st.w);
+      R flux[NV];
+      roe_flux<D>(q0, q1, q2, q3, dir, dir == 0 ? ar0 : (dir == 1 ? ar1 : ar2), ph, a.limiter, flux);
+      if (a.rbal) {
+        // a coarse/fine face of the optional balance: its balanced flux
+        const int q = a.tmod[ti.face0 + f];
+        if (q >= 0)
+          for (int v = 0; v < NV; ++v) flux[v] = a.rbal[(size_t)q * NV + v];
+      }
+      V o;
+      o.x = flux[0]; o.y = flux[1]; o.z = flux[2]; o.w = flux[3];
+      fl4[f] = o;
+      if (D == 3) fl1[f] = flux[4];
+      if (a.turb) {
+        fL[f] = st.y;
+        fR[f] = st.z;
+      }
     }
   }
   if (threadIdx.x == 0) halt = herr ? 1 : 0;
   __syncthreads();
   if (halt) return;   // uniform: the flag was written before the barrier
 
-  const double level_ts = a.alpha * a.dt[bi.case_id] * bi.step_num;
+  const double level_ts = a.alpha * uni(a.dt)[bi.case_id] * bi.step_num;
   double mx[NV], sq[NV];
 #pragma unroll
   for (int k = 0; k < NV; ++k) { mx[k] = 0.0; sq[k] = 0.0; }
@@ -501,16 +724,26 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, int tile) {
     }
   };
   int sl[2 * D];
-  if (live) load_slots(sl);
+  if (!BLK && live) load_slots(sl);
   // ComptSource: per direction (F_lo - F_hi), plus the frozen viscous
   // residual sum_d (Fv_hi - Fv_lo).  The learned-closure instantiation
   // forms it after the network (slots read again), so that neither the sum
   // nor the slots are held in registers across the network (they spill).
   auto residual = [&]() {
-    if constexpr (ML) load_slots(sl);
+    if constexpr (ML && !BLK) load_slots(sl);
+    int bx = 0, by = 0;
+    if constexpr (BLK) my_xy(bx, by);
 #pragma unroll
     for (int d = 0; d < D; ++d) {
-      const V lo = fl4[sl[2 * d]], hi = fl4[sl[2 * d + 1]];
+      V lo, hi;
+      if constexpr (BLK) {
+        const int k = by * kBoxP + bx;
+        lo = d == 0 ? bl.fx[k] : bl.fy[k];
+        hi = d == 0 ? bl.fx[k + 1] : bl.fy[k + kBoxP];
+      } else {
+        lo = fl4[sl[2 * d]];
+        hi = fl4[sl[2 * d + 1]];
+      }
       s[0] += (double)lo.x - (double)hi.x;
       s[1] += (double)lo.y - (double)hi.y;
       s[2] += (double)lo.z - (double)hi.z;
@@ -528,11 +761,22 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, int tile) {
     // reference never writes mutsource of solid cells)
     if (a.turb && (fg & F_UPDATE) && (fg & F_SA)) {
       sa_on = true;
-      const Prim<R, D> me = pload<R, D>(a.Win, c);
+      Prim<R, D> me;
+      int bx = 0, by = 0;
+      if constexpr (BLK) my_xy(bx, by);
+      if constexpr (BLK) me = box_prim<R>(bl, box_pos(bx, by));
+      else me = pload<R, D>(a.Win, c);
       R nl[3], nr[3], ul[3], ur[3], vl[3], vr[3], wl[3], wr[3];
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        if (d < D) {
+        if (BLK && d < D) {
+          const int p = box_pos(bx, by), st = d == 0 ? 1 : kBoxP;
+          const V lo = bl.S[p - st], hi = bl.S[p + st];
+          ul[d] = lo.y; vl[d] = lo.z; wl[d] = R(0);
+          ur[d] = hi.y; vr[d] = hi.z; wr[d] = R(0);
+          nl[d] = bl.nu[p - st];
+          nr[d] = bl.nu[p + st];
+        } else if (d < D) {
           const int lo = fL[sl[2 * d]], hi = fR[sl[2 * d + 1]];
           uvw_load<R, D>(a.Win, lo, ul[d], vl[d], wl[d]);
           uvw_load<R, D>(a.Win, hi, ur[d], vr[d], wr[d]);
@@ -543,7 +787,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, int tile) {
         }
       }
       const R T = v_div(me.p, me.r * (R)P.Rg);
-      const R nu = a.nuin[c];
+      const R nu = BLK ? bl.nu[box_pos(bx, by)] : a.nuin[c];
       const R sd = kMixed ? (R)a.sd32[c] : (R)a.signdis[c];
       if constexpr (!ML) {
         snu = (double)sa_source<R, D>(me.u, me.v, me.w, T, me.r, nu, sd, nl, nr, ul, ur, vl, vr,
@@ -576,7 +820,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, int tile) {
         // exec-mask branches, one per bound, otherwise)
 #pragma unroll
         for (int k = 0; k < kMlpIn; ++k)
-          ok = ok & (ml_x[k] >= a.mlp.flo[k]) & (ml_x[k] <= a.mlp.fhi[k]);
+          ok = ok & (ml_x[k] >= uni(a.mlp.flo)[k]) & (ml_x[k] <= uni(a.mlp.fhi)[k]);
         use_ml = ok;
         if (!ok) snu = (double)(sa_rest + sa_pointwise<R>(nu, mu0, me.r, sd, olen, Re));
       }
@@ -584,9 +828,10 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, int tile) {
   }
   // ---- learned closure: the network for the cells in its range
   if constexpr (ML) {
-    unsigned char *wbase = smem_raw + (wres ? (size_t)a.mlw_off : ml_smem_offset<R, D>(ti.nface));
+    unsigned char *wbase = smem_raw + (wres ? (size_t)a.mlw_off
+                                       : BLK ? blk_state_offset(sizeof(R)) : ml_smem_offset<R, D>(ti.nface));
     if (!wres) {
-      __syncthreads();   // every phase-2a read of the face-cell indices is done
+      __syncthreads();   // every phase-2a read of what the weights overwrite is done
       ml_fill_weights(a.mlp, wbase);
       __syncthreads();
     }
@@ -598,7 +843,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, int tile) {
     bf16x8_t xf;
 #pragma unroll
     for (int k = 0; k < kMlpIn; ++k)
-      xf[k] = (__bf16)(use_ml ? ((float)ml_x[k] - a.mlp.fmean[k]) * a.mlp.finv[k] : 0.0f);
+      xf[k] = (__bf16)(use_ml ? ((float)ml_x[k] - uni(a.mlp.fmean)[k]) * uni(a.mlp.finv)[k] : 0.0f);
     float yown = 0.0f;
     // one 32-cell block per pass, skipped (wave-uniformly) when none of its
     // cells is on the network; the compiler barrier keeps the weight
@@ -612,7 +857,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, int tile) {
       if ((lane >> 5) == sb) yown = y;
     }
     if (use_ml) {
-      const float z = a.mlp.zst[0] + a.mlp.zst[1] * (yown + a.mlp.b3[0]);
+      const float z = uni(a.mlp.zst)[0] + uni(a.mlp.zst)[1] * (yown + uni(a.mlp.b3)[0]);
       snu = (double)(sa_rest + (R)z * ml_scale);
     }
     if (a.last && a.mlcount) {
@@ -772,8 +1017,20 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, int tile) {
 // Morton neighbours sharing that XCD's L2.
 template <typename R, int D, bool ML, bool P>
 __device__ __forceinline__ void stage_launch(const StageArgs<R, D> &a) {
+  __shared__ StageShared sh;
+  auto one = [&](int tile) {
+    const bool herr = halted(a.err);
+    const TileInfo ti = tile_info(a.tiles, tile);
+    if constexpr (D == 2) {
+      if (ti.halo0 >= 0) {
+        stage_tile<R, D, ML, P, true>(a, ti, tile, herr, sh);
+        return;
+      }
+    }
+    stage_tile<R, D, ML, P, false>(a, ti, tile, herr, sh);
+  };
   if constexpr (!P) {
-    stage_tile<R, D, ML, false>(a, dispatch_tile());
+    one(dispatch_tile());
     return;
   }
   extern __shared__ __align__(32) unsigned char smem_raw[];
@@ -790,7 +1047,7 @@ __device__ __forceinline__ void stage_launch(const StageArgs<R, D> &a) {
     // nothing is hoisted out of the loop: values kept live across the
     // tiles would cost the loop body registers (and occupancy)
     asm volatile("" ::: "memory");
-    stage_tile<R, D, ML, true>(a, t);
+    one(t);
     __syncthreads();   // the next tile rewrites the face arrays
   }
 }
