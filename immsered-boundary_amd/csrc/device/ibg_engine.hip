@@ -2700,15 +2700,23 @@ ibg_status cl_pack(ibg_ctx *c) {
   return IBG_OK;
 }
 
-constexpr size_t kTrainSmem = (size_t)64 * kX * 2 * 2 + (size_t)64 * kH * 2 * 5 + (5 * 64 + 256) * 4;
-
 ibg_status cl_train_launch(ibg_ctx *c, const float *X, const float *Z, long long n, int nwg,
                            int batch, int explicit_rows, uint64_t seed) {
   TrainArgs a;
   a.M = c->mlpdev();
   a.X = X; a.Z = Z; a.n = n; a.batch = batch; a.explicit_rows = explicit_rows; a.seed = seed;
   a.grad = c->cl.grad; a.lossp = c->cl.lossp;
-  hipLaunchKernelGGL(k_closure_train, dim3(nwg), dim3(256), kTrainSmem, c->s, a);
+  hipLaunchKernelGGL(k_closure_train, dim3(nwg), dim3(256), 0, c->s, a);
+  HIPCHK(hipGetLastError());
+  return IBG_OK;
+}
+
+// Adam over the gradients of nwg workgroups, with the new weights packed; in
+// the summing mode (gsum) the summed gradient only
+ibg_status cl_adam_launch(ibg_ctx *c, int nwg, float lr, int step, float *gsum) {
+  hipLaunchKernelGGL(k_closure_adam, dim3(grid(kNParam, kAdamThreads)), dim3(kAdamThreads), 0, c->s,
+                     c->cl.p, c->cl.m, c->cl.v, c->cl.grad, nwg, lr, step, gsum, c->cl.W1t, c->cl.W2t,
+                     c->cl.W2, c->cl.W2p, c->cl.w3, c->cl.b1, c->cl.b2, c->cl.b3);
   HIPCHK(hipGetLastError());
   return IBG_OK;
 }
@@ -2892,10 +2900,7 @@ ibg_status ibg_closure_train(ibg_ctx *c, int32_t steps, int32_t batch, double lr
     ++c->cl.step;
     // cosine decay of the learning rate over the call, down to lr/100
     const double lrk = lr * (0.01 + 0.99 * 0.5 * (1.0 + std::cos(3.141592653589793 * k / std::max(steps, 1))));
-    hipLaunchKernelGGL(k_closure_adam, dim3(grid(kNParam, 256)), dim3(256), 0, c->s, c->cl.p, c->cl.m,
-                       c->cl.v, c->cl.grad, nwg, (float)lrk, c->cl.step, (float *)nullptr);
-    HIPCHK(hipGetLastError());
-    if ((st = cl_pack(c))) return st;
+    if ((st = cl_adam_launch(c, nwg, (float)lrk, c->cl.step, nullptr))) return st;
   }
   if (loss) {
     std::vector<float> h(nwg);
@@ -2994,12 +2999,10 @@ ibg_status ibg_closure_grad(ibg_ctx *c, const float *x, const float *z, int64_t 
   if (e == hipSuccess) st = cl_train_launch(c, dx, dz, n, nwg, (int)n, 1, 0);
   if (e == hipSuccess && !st) {
     // the Adam kernel in its summing mode: the gradient, no update
-    hipLaunchKernelGGL(k_closure_adam, dim3(grid(kNParam, 256)), dim3(256), 0, c->s, c->cl.p, c->cl.m,
-                       c->cl.v, c->cl.grad, nwg, 0.0f, 1, c->cl.gsum);
-    e = hipGetLastError();
-    if (e == hipSuccess) e = hipStreamSynchronize(c->s);
-    if (e == hipSuccess) e = hipMemcpy(grad, c->cl.gsum, sizeof(float) * kNParam, hipMemcpyDeviceToHost);
-    if (e == hipSuccess && loss) {
+    st = cl_adam_launch(c, nwg, 0.0f, 1, c->cl.gsum);
+    if (!st) e = hipStreamSynchronize(c->s);
+    if (!st && e == hipSuccess) e = hipMemcpy(grad, c->cl.gsum, sizeof(float) * kNParam, hipMemcpyDeviceToHost);
+    if (!st && e == hipSuccess && loss) {
       std::vector<float> h(nwg);
       e = hipMemcpy(h.data(), c->cl.lossp, sizeof(float) * nwg, hipMemcpyDeviceToHost);
       double s = 0;

@@ -38,8 +38,8 @@ typedef float floatx4_t __attribute__((ext_vector_type(4)));
 
 constexpr int kMlpIn = 8;
 constexpr int kMlpHid = 64;
-constexpr int kX = 40;     // LDS row stride (bf16) of the padded 32-wide input rows
-constexpr int kH = 72;     // LDS row stride (bf16) of the 64-wide hidden rows
+constexpr int kX = 40;     // row stride (bf16) of W1t, its 8 inputs padded with zeros
+constexpr int kH = 72;     // row stride (bf16) of 64-wide rows (LDS banks, W2, W2t)
 // fp32 parameter vector: W1[8][64] b1[64] W2[64][64] b2[64] w3[64] b3
 constexpr int kOffW1 = 0, kOffB1 = 512, kOffW2 = 576, kOffB2 = 4672, kOffW3 = 4736, kOffB3 = 4800;
 constexpr int kNParam = 4801;
@@ -63,7 +63,6 @@ struct MlpDev {
 // quarter rate) made the learned-closure stage kernel about 20 % slower for
 // the same closure error.
 __device__ __forceinline__ float mlp_act(float z) { return fmaxf(z, 0.0f); }
-__device__ __forceinline__ float mlp_dact(float z) { return z > 0.0f ? 1.0f : 0.0f; }
 // Two units to a bf16 pair with the ReLU applied after the rounding, as a
 // signed 16-bit max against 0 (v_cvt_pk_bf16_f32 + v_pk_max_i16): a
 // negative value rounds to a bf16 with the sign bit set (or -0), a negative
@@ -79,93 +78,9 @@ __device__ __forceinline__ bf16x2_t mlp_act_pk(float a, float b) {
   const s16x2_t m = __builtin_elementwise_max(__builtin_bit_cast(s16x2_t, h), s16x2_t{0, 0});
   return __builtin_bit_cast(bf16x2_t, m);
 }
-__device__ __forceinline__ float bf16r(float x) { return (float)(__bf16)x; }
 
 __device__ __forceinline__ floatx4_t mfma16(bf16x8_t a, bf16x8_t b, floatx4_t c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
-}
-
-// Weights into LDS (cooperative over the workgroup).
-struct MlpLds {
-  __bf16 *W1t;   // [64][kX]
-  __bf16 *W2t;   // [64][kH]
-  float *w3, *b1, *b2;   // [64] each
-};
-
-__device__ __forceinline__ void mlp_load_lds(const MlpDev &M, const MlpLds &S) {
-  for (int i = threadIdx.x; i < 64 * kX; i += blockDim.x) S.W1t[i] = M.W1t[i];
-  for (int i = threadIdx.x; i < 64 * kH; i += blockDim.x) S.W2t[i] = M.W2t[i];
-  for (int i = threadIdx.x; i < 64; i += blockDim.x) {
-    S.w3[i] = M.w3[i];
-    S.b1[i] = M.b1[i];
-    S.b2[i] = M.b2[i];
-  }
-}
-
-// Forward of 16 rows by one wave.  Xs: [16][kX] bf16 rows (inputs in columns
-// 0..7, zeros in 8..31).  Hs: [16][kH] bf16 scratch of the wave.  The
-// pre-activations are optionally kept (Z1s/Z2s [16][kH] as relu' in bf16)
-// and the activations H1/H2 (H1s, H2s) for the backward pass.  Returns
-// y for rows 4*(l/16)+v in yv[v] of the lanes with l%16 == 0 (summed over
-// the 16 lanes of each group), b3 not included.  All 64 lanes must call it
-// together; the barriers are workgroup barriers, so every wave of the
-// workgroup calls it the same number of times.
-__device__ __forceinline__ void mlp_fwd16(const __bf16 *Xs, __bf16 *H1s, __bf16 *H2s,
-                                          __bf16 *S1s, __bf16 *S2s, const MlpLds &W,
-                                          float *yv) {
-  const int lane = threadIdx.x & 63;
-  const int r = lane & 15, q = lane >> 4;
-  // layer 1: [16 x 32] x [32 x 64]
-  floatx4_t acc[4];
-  const bf16x8_t a1 = *reinterpret_cast<const bf16x8_t *>(Xs + r * kX + 8 * q);
-#pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
-    const float bb = W.b1[16 * nt + r];
-    acc[nt] = floatx4_t{bb, bb, bb, bb};
-    const bf16x8_t b = *reinterpret_cast<const bf16x8_t *>(W.W1t + (16 * nt + r) * kX + 8 * q);
-    acc[nt] = mfma16(a1, b, acc[nt]);
-  }
-#pragma unroll
-  for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int row = 4 * q + v, col = 16 * nt + r;
-      H1s[row * kH + col] = (__bf16)mlp_act(acc[nt][v]);
-      if (S1s) S1s[row * kH + col] = (__bf16)mlp_dact(acc[nt][v]);
-    }
-  __syncthreads();
-  // layer 2: [16 x 64] x [64 x 64]
-#pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
-    const float bb = W.b2[16 * nt + r];
-    acc[nt] = floatx4_t{bb, bb, bb, bb};
-  }
-#pragma unroll
-  for (int kt = 0; kt < 2; ++kt) {
-    const bf16x8_t a = *reinterpret_cast<const bf16x8_t *>(H1s + r * kH + 32 * kt + 8 * q);
-#pragma unroll
-    for (int nt = 0; nt < 4; ++nt) {
-      const bf16x8_t b = *reinterpret_cast<const bf16x8_t *>(W.W2t + (16 * nt + r) * kH + 32 * kt + 8 * q);
-      acc[nt] = mfma16(a, b, acc[nt]);
-    }
-  }
-  // layer 3: y = bf16(relu(Z2)) . w3, reduced over the 16 lanes of a group
-#pragma unroll
-  for (int v = 0; v < 4; ++v) yv[v] = 0.0f;
-#pragma unroll
-  for (int nt = 0; nt < 4; ++nt)
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-      const int row = 4 * q + v, col = 16 * nt + r;
-      const __bf16 h = (__bf16)mlp_act(acc[nt][v]);
-      if (H2s) H2s[row * kH + col] = h;
-      if (S2s) S2s[row * kH + col] = (__bf16)mlp_dact(acc[nt][v]);
-      yv[v] += (float)h * W.w3[col];
-    }
-#pragma unroll
-  for (int v = 0; v < 4; ++v)
-    for (int off = 1; off < 16; off <<= 1) yv[v] += __shfl_xor(yv[v], off, 64);
-  __syncthreads();
 }
 
 // Transposed forward with the activations in registers (the stage kernel),
