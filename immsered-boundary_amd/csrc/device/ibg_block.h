@@ -1,23 +1,25 @@
 // ibg_block.h — block tiles: 256 Morton-consecutive cells that fill an
-// aligned 16 x 16 square of their level (2D).
+// aligned 16 x 16 square (2D) or 8 x 8 x 4 box (3D) of their level.
 //
 // The faces of such a tile, their stencils and the cells' face slots follow
-// from the position in the square, so the tile needs no face list: it reads
-// its 256 cells and the indices of its 132 halo cells (two layers on each
-// side, one cell at each corner) and works from LDS.  A general tile reads
+// from the position in the block, so the tile needs no face list: it reads
+// its 256 cells and the indices of its halo cells (132 in 2D: two layers on
+// each side, one cell at each corner; 592 in 3D) and works from LDS.  A general tile reads
 // 17 B per face (33 B in the viscous pass, ~2.2 faces per cell), 8 B of
 // slots per cell, and gathers each state record about nine times from
 // L1/L2; a block tile reads 2 B per cell of halo indices and each record
 // once.  90 % of the cells of the 2.6M-cell section and 80 % of a
 // 4.2M-cell ensemble lie in block tiles; the rest, the ragged rims of the
-// refinement levels, stay in general tiles (a level's square that lacks a
-// cell, or whose stencil is not the regular one, is general; so are all
-// tiles of other sizes than 256 cells and of 3D meshes).  Average launch of
-// the moving 2.6M-cell section, general tiles only -> with block tiles:
-// k_stage FP64 150 -> 134 us, FP32 71 -> 61 us (the learned closure's 97 ->
-// 87 us), k_visc_prep FP32 66 -> 43 us.  The FP32 stage then issues vector
-// instructions for about two thirds of its time (its bytes alone would take
-// 36 us at the copy rate); the FP64 one for most of it.
+// refinement levels, stay in general tiles (as does a block whose stencils
+// are not the regular ones, and every tile of another size than 256 cells).
+//
+// Average launch, general tiles only -> with block tiles.  2D, moving
+// 2.6M-cell section: k_stage FP64 150 -> 134 us, FP32 71 -> 61 us (the
+// learned closure's 97 -> 87 us), k_visc_prep FP32 66 -> 43 us.  3D, 2.7M
+// cells: k_stage FP32 147 -> 124 us, FP64 300 -> 294 us, k_visc_prep FP32
+// 172 -> 75 us, FP64 321 -> 179 us.  The FP32 stages then issue vector
+// instructions for 77 % (3D) to 92 % (2D) of their time (2D: the bytes alone
+// would take 36 us at the copy rate), the FP64 ones for 65 to 77 %.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -65,6 +67,79 @@ __host__ __device__ inline int halo_pos(int h) {
 __host__ __device__ constexpr size_t blk_state_offset(size_t rsize) { return 4 * rsize * kFluxSlots; }
 __host__ __device__ constexpr size_t blk_smem(size_t rsize, bool turb, bool temp) {
   return blk_state_offset(rsize) + (4 * rsize + (turb ? rsize : 0) + (temp ? rsize : 0)) * kBoxCells;
+}
+
+// ------------------------------------------------------------------- 3D
+// 8 x 8 x 4 cells (x, y, z), Morton order x lowest.  LDS records of the stage
+// kernel: the four planes as 12 x 12 boxes (x and y halos in place, plane
+// pitch 152), then the halo planes z = -1, 4, -2, 5 of 8 x 8 cells; the
+// working variable stops before the last two.  The viscous pass keeps the
+// 10 x 10 x 6 box of the first halo layer.  Both pitches put the 4 x 2 x 2
+// cells of 16 consecutive lanes on (nearly) distinct bank groups.  The face
+// fluxes of one direction at a time: with all three the LDS would hold two
+// workgroups less per CU.
+constexpr int kB3X = 8, kB3Y = 8, kB3Z = 4;
+constexpr int kBox3Plane = 152, kBox3Halo = 4 * kBox3Plane;
+constexpr int kBox3Cells = kBox3Halo + 4 * 64, kBox3Nu = kBox3Halo + 2 * 64;
+constexpr int kVBox3P = 10, kVBox3Plane = 100, kVBox3Cells = 6 * kVBox3Plane;
+constexpr int kFlux3 = 320;
+// halo list: layer 1 (x, y, z; low then high side), the edges of the first
+// layer (xy, xz, yz; low/low, high/low, low/high, high/high), layer 2
+constexpr int kHalo3L1 = 256, kHalo3E = kHalo3L1 + 80, kHalo3 = kHalo3E + 256;
+
+__host__ __device__ inline void blk_xyz(int i, int &x, int &y, int &z) {
+  x = (i & 1) | ((i >> 2) & 2) | ((i >> 4) & 4);
+  y = ((i >> 1) & 1) | ((i >> 3) & 2) | ((i >> 5) & 4);
+  z = ((i >> 2) & 1) | ((i >> 4) & 2);
+}
+// coordinates of halo entry h (-2 .. 9, -2 .. 9, -2 .. 5)
+__host__ __device__ inline void halo3_xyz(int h, int &x, int &y, int &z) {
+  if (h >= kHalo3L1 && h < kHalo3E) {
+    int k = h - kHalo3L1;
+    if (k < 16) {
+      z = k & 3; x = (k & 4) ? kB3X : -1; y = (k & 8) ? kB3Y : -1;
+    } else if (k < 48) {
+      k -= 16;
+      y = k & 7; x = (k & 8) ? kB3X : -1; z = (k & 16) ? kB3Z : -1;
+    } else {
+      k -= 48;
+      x = k & 7; y = (k & 8) ? kB3Y : -1; z = (k & 16) ? kB3Z : -1;
+    }
+    return;
+  }
+  const int far = h >= kHalo3E ? 1 : 0, k = far ? h - kHalo3E : h;
+  const int a = k & 7, b = (k >> 3) & 3, side = (k >> 5) & 1;
+  if (k < 64) {
+    x = side ? kB3X + far : -1 - far; y = a; z = b;
+  } else if (k < 128) {
+    y = side ? kB3Y + far : -1 - far; x = a; z = b;
+  } else {
+    x = a; y = (k >> 3) & 7; z = (k & 64) ? kB3Z + far : -1 - far;
+  }
+}
+__host__ __device__ inline int box3_in(int x, int y, int z) { return z * kBox3Plane + (y + 2) * 12 + x + 2; }
+// plane n of the halo planes z = -1, 4, -2, 5
+__host__ __device__ inline int box3_zhalo(int x, int y, int n) { return kBox3Halo + n * 64 + y * 8 + x; }
+__host__ __device__ inline int box3_pos(int x, int y, int z) {
+  if (z >= 0 && z < kB3Z) return box3_in(x, y, z);
+  return box3_zhalo(x, y, z == -1 ? 0 : (z == kB3Z ? 1 : (z < 0 ? 2 : 3)));
+}
+__host__ __device__ constexpr int vbox3_pos(int x, int y, int z) {
+  return (z + 1) * kVBox3Plane + (y + 1) * kVBox3P + x + 1;
+}
+// flux slot of the low face of cell (x, y, z) in direction d and the step to
+// the next face
+__host__ __device__ constexpr int flux3_slot(int d, int x, int y, int z) {
+  return d == 0 ? x + 9 * y + 76 * z : (d == 1 ? x + 8 * y + 76 * z : x + 8 * y + 64 * z);
+}
+__host__ __device__ constexpr int flux3_step(int d) { return d == 0 ? 1 : (d == 1 ? 8 : 64); }
+
+__host__ __device__ constexpr size_t blk3_state_offset(size_t rsize) { return 5 * rsize * kFlux3; }
+__host__ __device__ constexpr size_t blk3_smem(size_t rsize, bool turb) {
+  return blk3_state_offset(rsize) + 5 * rsize * kBox3Cells + (turb ? rsize * kBox3Nu : 0);
+}
+__host__ __device__ constexpr size_t blk3_visc_smem(size_t rsize, bool turb) {
+  return blk3_state_offset(rsize) + (5 * rsize + (turb ? rsize : 0)) * kVBox3Cells;
 }
 
 }  // namespace ibg

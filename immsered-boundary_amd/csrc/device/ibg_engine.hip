@@ -242,7 +242,8 @@ size_t ml_resident_offset(const ibg_ctx *c) {
   size_t per = 4 * sizeof(float) + (c->D == 3 ? sizeof(float) : 0);
   if (c->turb) per += 2 * sizeof(int);
   size_t b = (size_t)c->max_tile_faces * per;
-  if (c->nblock > 0) b = std::max(b, blk_smem(sizeof(float), c->turb, false));
+  if (c->nblock > 0)
+    b = std::max(b, c->D == 2 ? blk_smem(sizeof(float), c->turb, false) : blk3_smem(sizeof(float), c->turb));
   return (b + 15) & ~(size_t)15;
 }
 
@@ -374,16 +375,21 @@ size_t tile_smem(const ibg_ctx *c, size_t rsize, bool stage, bool fused = false)
   size_t per = 4 * rsize + (c->D == 3 ? rsize : 0);
   if (c->turb) per += stage ? std::max<size_t>(2 * sizeof(int), rsize) : rsize;
   size_t b = (size_t)c->max_tile_faces * per;
-  if (c->nblock > 0) b = std::max(b, blk_smem(rsize, c->turb, fused || !stage));
+  if (c->nblock > 0)
+    b = std::max(b, c->D == 2 ? blk_smem(rsize, c->turb, fused || !stage)
+                              : (stage ? blk3_smem(rsize, c->turb) : blk3_visc_smem(rsize, c->turb)));
   if (stage && c->cl.on) {
     // the network's weights: after every face array, resident across the
     // tiles (persistent schedule), or after the face fluxes over the
     // face-cell indices (one workgroup per tile)
-    if (c->cfg.schedule == 1) return ml_resident_offset(c) + kStageMlSmem;
-    size_t m = c->D == 2 ? ml_smem_offset<float, 2>(c->max_tile_faces)
-                         : ml_smem_offset<float, 3>(c->max_tile_faces);
-    if (c->nblock > 0) m = std::max(m, blk_state_offset(rsize));
-    return std::max(b, m + kStageMlSmem);
+    // (the persistent schedule keeps a 3D block's residuals behind them)
+    if (c->cfg.schedule == 1)
+      return ml_resident_offset(c) + kStageMlSmem +
+             (c->D == 3 && c->nblock > 0 ? blk_ml_smem<3>() - blk_ml_offset<3>() - kStageMlSmem : 0);
+    size_t m = (c->D == 2 ? ml_smem_offset<float, 2>(c->max_tile_faces)
+                          : ml_smem_offset<float, 3>(c->max_tile_faces)) + kStageMlSmem;
+    if (c->nblock > 0) m = std::max(m, c->D == 2 ? blk_ml_smem<2>() : blk_ml_smem<3>());
+    return std::max(b, m);
   }
   return b;
 }
@@ -777,18 +783,44 @@ ibg_status read_err(ibg_ctx *c, int64_t *cell, int32_t *code) {
 
 }  // namespace
 
-// The block tiles of an uploaded 2D mesh: isblk[i] for the first device cell
-// i of every run of 256 cells that fills a 16 x 16 square of its (level,
-// case) in Morton order and whose every face has the stencil its position
-// gives (checked face by face, so a block tile computes from the same cells
-// as a general tile over the same run); halo gets kHalo cells per square, in
-// cell order.  With the optional coarse/fine balance, a square with a
-// balanced face stays general (its fluxes come from the pre-pass by face).
+// The block tiles of an uploaded mesh: isblk[i] for the first device cell i
+// of every run of 256 cells that fills a block of its (level, case) in
+// Morton order and whose every face has the stencil its position gives
+// (checked face by face, so a block tile computes from the same cells as a
+// general tile over the same run); halo gets the block's halo cells (kHalo
+// or kHalo3 of them), in cell order.  With the optional coarse/fine balance,
+// a block with a balanced face stays general (its fluxes come from the
+// pre-pass by face).
 namespace {
-template <class FI, class F4v, class FD>
+template <int D>
+struct BlockShape {
+  static constexpr int n[3] = {D == 2 ? kBlkN : kB3X, D == 2 ? kBlkN : kB3Y, D == 2 ? 1 : kB3Z};
+  static constexpr int halo = D == 2 ? kHalo : kHalo3;
+  static void xyz(int i, int *q) {
+    if (D == 2) { blk_xy(i, q[0], q[1]); q[2] = 0; }
+    else blk_xyz(i, q[0], q[1], q[2]);
+  }
+  // position in the box of the block and two halo layers
+  static constexpr int px = n[0] + 4, py = n[1] + 4, pz = D == 2 ? 1 : n[2] + 4;
+  static constexpr int cells = px * py * pz;
+  static int pos(int x, int y, int z) { return ((D == 2 ? 0 : z + 2) * py + y + 2) * px + x + 2; }
+  static int step(int d) { return d == 0 ? 1 : (d == 1 ? px : px * py); }
+  static int halo_at(int h) {
+    if (D == 2) {
+      const int p = halo_pos(h);
+      return pos(p % kBoxP - 2, p / kBoxP - 2, 0);
+    }
+    int x, y, z;
+    halo3_xyz(h, x, y, z);
+    return pos(x, y, z);
+  }
+};
+
+template <int D, class FI, class F4v, class FD>
 void find_blocks(ibg_ctx *c, const ibg_mesh_soa *m, const std::vector<int> &order,
-                       const FI &cfaces, const F4v &face_st, const F4v &face_vst,
-                       const FD &face_dir, std::vector<uint8_t> &isblk, hvec<int> &halo) {
+                 const FI &cfaces, const F4v &face_st, const F4v &face_vst,
+                 const FD &face_dir, std::vector<uint8_t> &isblk, hvec<int> &halo) {
+  using B = BlockShape<D>;
   const int L = c->L, Nn = c->Nn;
   std::vector<uint8_t> bal;
   if (c->cfg.reflux && m->nmdy > 0) {
@@ -799,70 +831,74 @@ void find_blocks(ibg_ctx *c, const ibg_mesh_soa *m, const std::vector<int> &orde
         if (f >= 0 && f < c->F) bal[c->fh2d[f]] = 1;
       }
   }
-  // candidates: the corners' keys first (nearly every start fails there),
+  // candidates: the last cell's key first (nearly every start fails there),
   // then every key
-  auto key = [&](int i, int d) { return m->key[(size_t)order[i] * 3 + d]; };
+  int at[kBlkCells][3];
+  for (int i = 0; i < kBlkCells; ++i) B::xyz(i, at[i]);
+  auto key = [&](int i) { return m->key + (size_t)order[i] * 3; };
+  auto same = [&](int t, const int32_t *k0, int i) {
+    const int32_t *k = key(t + i);
+    return k[0] == k0[0] + at[i][0] && k[1] == k0[1] + at[i][1] && k[2] == k0[2] + at[i][2];
+  };
   std::vector<int> cand;
   int pos = 0;
   for (int l = L - 1; l >= 0; --l)
     for (int cs = 0; cs < c->ncases; ++cs) {
       const int end = pos + m->blk_nnormal[cs * L + l];
       for (int t = pos; t + kBlkCells <= end;) {
-        const int x0 = key(t, 0), y0 = key(t, 1);
-        bool ok = key(t + 255, 0) == x0 + 15 && key(t + 255, 1) == y0 + 15 &&
-                  key(t + 85, 0) == x0 + 15 && key(t + 85, 1) == y0;
-        for (int i = 0; ok && i < kBlkCells; ++i) {
-          int x, y;
-          blk_xy(i, x, y);
-          ok = key(t + i, 0) == x0 + x && key(t + i, 1) == y0 + y && key(t + i, 2) == key(t, 2);
-        }
+        const int32_t *k0 = key(t);
+        bool ok = same(t, k0, kBlkCells - 1);
+        for (int i = 0; ok && i < kBlkCells; ++i) ok = same(t, k0, i);
         if (ok) cand.push_back(t);
         t += ok ? kBlkCells : 1;
       }
       pos = end;
     }
   const int n = (int)cand.size();
-  hvec<int> all((size_t)n * kHalo);
+  hvec<int> all((size_t)n * B::halo);
   std::vector<uint8_t> good(n, 0);
+  constexpr int q2 = 2 * D;
   host_parallel(n, [&](int lo, int hi) {
+    std::vector<int> P(B::cells);
     for (int q = lo; q < hi; ++q) {
       const int t = cand[q];
-      int P[kBoxCells];
-      for (int &v : P) v = -1;
-      int cell[kBlkN][kBlkN];   // [y][x]
-      for (int i = 0; i < kBlkCells; ++i) {
-        int x, y;
-        blk_xy(i, x, y);
-        P[box_pos(x, y)] = cell[y][x] = t + i;
-      }
-      auto face = [&](int x, int y, int s) { return cfaces[(size_t)cell[y][x] * 4 + s]; };
-      for (int k = 0; k < kBlkN; ++k) {
-        const int4 xl = face_st[face(0, k, 0)], xh = face_st[face(kBlkN - 1, k, 1)];
-        const int4 yl = face_st[face(k, 0, 2)], yh = face_st[face(k, kBlkN - 1, 3)];
-        P[box_pos(-2, k)] = xl.x; P[box_pos(-1, k)] = xl.y;
-        P[box_pos(kBlkN, k)] = xh.z; P[box_pos(kBlkN + 1, k)] = xh.w;
-        P[box_pos(k, -2)] = yl.x; P[box_pos(k, -1)] = yl.y;
-        P[box_pos(k, kBlkN)] = yh.z; P[box_pos(k, kBlkN + 1)] = yh.w;
-      }
-      P[box_pos(-1, -1)] = face_vst[face(0, 0, 0)].z;
-      P[box_pos(kBlkN, -1)] = face_vst[face(kBlkN - 1, 0, 1)].w;
-      P[box_pos(-1, kBlkN)] = face_vst[face(0, kBlkN - 1, 0)].x;
-      P[box_pos(kBlkN, kBlkN)] = face_vst[face(kBlkN - 1, kBlkN - 1, 1)].y;
-      bool ok = true;
-      for (int y = 0; ok && y < kBlkN; ++y)
-        for (int x = 0; ok && x < kBlkN; ++x)
-          for (int s = 0; ok && s < 4; ++s) {
-            const int f = face(x, y, s), d = s >> 1;
-            const int st = d == 0 ? 1 : kBoxP, tt = d == 0 ? kBoxP : 1;
-            const int p = box_pos(x, y) + (s & 1) * st;   // the face's high-side cell
-            const int4 a = face_st[f], v = face_vst[f];
-            ok = face_dir[f] == d && a.x == P[p - 2 * st] && a.y == P[p - st] && a.z == P[p] &&
-                 a.w == P[p + st] && v.x == P[p - st + tt] && v.y == P[p + tt] &&
-                 v.z == P[p - st - tt] && v.w == P[p - tt] && (bal.empty() || !bal[f]);
+      std::fill(P.begin(), P.end(), -1);
+      for (int i = 0; i < kBlkCells; ++i) P[B::pos(at[i][0], at[i][1], at[i][2])] = t + i;
+      // the halo from the stencils of the block's outer faces: the layers
+      // from the inviscid one, corners and edges from the viscous one
+      for (int i = 0; i < kBlkCells; ++i)
+        for (int d = 0; d < D; ++d)
+          for (int s = 0; s < 2; ++s) {
+            if (at[i][d] != (s ? B::n[d] - 1 : 0)) continue;
+            const int f = cfaces[(size_t)(t + i) * q2 + 2 * d + s];
+            const int o = B::pos(at[i][0], at[i][1], at[i][2]) + (s ? 1 : -1) * B::step(d);
+            const int4 a = face_st[f];
+            P[o] = s ? a.z : a.y;
+            P[o + (s ? 1 : -1) * B::step(d)] = s ? a.w : a.x;
+            for (int k = 0; k < D - 1; ++k) {
+              const int tax = (k == 0) ? (d == 0 ? 1 : 0) : (d == 2 ? 1 : 2);
+              const int4 v = face_vst[(size_t)f * (D - 1) + k];
+              if (at[i][tax] == 0) P[o - B::step(tax)] = s ? v.w : v.z;
+              if (at[i][tax] == B::n[tax] - 1) P[o + B::step(tax)] = s ? v.y : v.x;
+            }
           }
-      for (int h = 0; ok && h < kHalo; ++h) {
-        const int v = P[halo_pos(h)];
-        all[(size_t)q * kHalo + h] = v;
+      bool ok = true;
+      for (int i = 0; ok && i < kBlkCells; ++i)
+        for (int s = 0; ok && s < q2; ++s) {
+          const int f = cfaces[(size_t)(t + i) * q2 + s], d = s >> 1, st = B::step(d);
+          const int p = B::pos(at[i][0], at[i][1], at[i][2]) + (s & 1) * st;   // the high-side cell
+          const int4 a = face_st[f];
+          ok = face_dir[f] == d && a.x == P[p - 2 * st] && a.y == P[p - st] && a.z == P[p] &&
+               a.w == P[p + st] && (bal.empty() || !bal[f]);
+          for (int k = 0; ok && k < D - 1; ++k) {
+            const int tt = B::step((k == 0) ? (d == 0 ? 1 : 0) : (d == 2 ? 1 : 2));
+            const int4 v = face_vst[(size_t)f * (D - 1) + k];
+            ok = v.x == P[p - st + tt] && v.y == P[p + tt] && v.z == P[p - st - tt] && v.w == P[p - tt];
+          }
+        }
+      for (int h = 0; ok && h < B::halo; ++h) {
+        const int v = P[B::halo_at(h)];
+        all[(size_t)q * B::halo + h] = v;
         ok = v >= 0 && v < c->N;
       }
       good[q] = ok;
@@ -874,10 +910,11 @@ void find_blocks(ibg_ctx *c, const ibg_mesh_soa *m, const std::vector<int> &orde
     if (!good[q]) continue;
     isblk[cand[q]] = 1;
     if (w != (size_t)q)
-      std::copy(all.begin() + (size_t)q * kHalo, all.begin() + (size_t)(q + 1) * kHalo, all.begin() + w * kHalo);
+      std::copy(all.begin() + (size_t)q * B::halo, all.begin() + (size_t)(q + 1) * B::halo,
+                all.begin() + w * B::halo);
     ++w;
   }
-  all.resize(w * kHalo);
+  all.resize(w * B::halo);
   halo.swap(all);
 }
 }  // namespace
@@ -1302,14 +1339,17 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
   }
   });
   // ---- tiles over each (level, case) run of normal cells: block tiles
-  // (ibg_block.h) where 256 consecutive cells fill a square, general tiles
+  // (ibg_block.h) where 256 consecutive cells fill a block, general tiles
   // over the runs between them.  A general tile's face list is the faces of
   // its cells in first-occurrence order (cells in order, each cell's faces
   // low/high per direction); the lists are formed per tile in parallel,
   // placed by a prefix sum, then filled in parallel.
-  std::vector<uint8_t> isblk;      // by device cell: the first cell of a square
+  std::vector<uint8_t> isblk;      // by device cell: the first cell of a block
   hvec<int> halo;
-  if (D == 2 && c->tile == kBlkCells) find_blocks(c, m, order, cfaces, face_st, face_vst, face_dir, isblk, halo);
+  if (c->tile == kBlkCells) {
+    if (D == 2) find_blocks<2>(c, m, order, cfaces, face_st, face_vst, face_dir, isblk, halo);
+    else find_blocks<3>(c, m, order, cfaces, face_st, face_vst, face_dir, isblk, halo);
+  }
   std::vector<TileInfo> tiles;
   std::vector<int> case_tiles((size_t)nc * L * 2, 0);   // [case][level] = {first, end}
   c->tile_end.assign(L, 0);
@@ -1337,7 +1377,7 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
         for (int t = pos; !isblk.empty() && t + kBlkCells <= pos + n;) {
           if (!isblk[t]) { ++t; continue; }
           flush(t);
-          emit(t, kBlkCells, kHalo * c->nblock++);
+          emit(t, kBlkCells, (D == 2 ? kHalo : kHalo3) * c->nblock++);
           t += kBlkCells;
           run = t;
         }

@@ -7,6 +7,8 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <type_traits>
+
 #include "ibg_common.h"
 
 namespace ibg {
@@ -16,44 +18,38 @@ __device__ __forceinline__ float r_abs(float x) { return fabsf(x); }
 
 // Reciprocal, quotient and square root of the flux arithmetic.  FP32: the
 // hardware v_rcp_f32 / v_sqrt_f32 (~1 ulp).  FP64: the hardware estimate
-// refined by two Newton steps, and Markstein's fused quotient (the residual
-// n - x q is exact): the IEEE sequence without its range scaling and fixup,
-// 8 instructions instead of 11 with the same value in the normal range, 5
-// for a reciprocal.  A zero, denormal or infinite operand gives NaN, so the
-// few places that meet one in earnest divide with '/'.
+// refined.  A zero, denormal or infinite operand gives NaN, so the few places
+// that meet one in earnest divide with '/'.
 __device__ __forceinline__ float f_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ float f_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 __device__ __forceinline__ float n_div(float n, float x) { return n * f_rcp(x); }
-__device__ __forceinline__ double n_rcp(double x) {
+// FP64 quotient: two Newton steps and Markstein's fused residual, the IEEE
+// sequence without its range scaling and fixup: the same value in the normal
+// range.
+__device__ __forceinline__ double n_div(double n, double x) {
   double y = __builtin_amdgcn_rcp(x);
   y = fma(fma(-x, y, 1.0), y, y);
-  return fma(fma(-x, y, 1.0), y, y);
-}
-__device__ __forceinline__ double n_div(double n, double x) {
-  const double y = n_rcp(x), q = n * y;
+  y = fma(fma(-x, y, 1.0), y, y);
+  const double q = n * y;
   return fma(fma(-x, q, n), y, q);
 }
-// coupled Newton (Goldschmidt) iteration on g -> sqrt(x), h -> 1/(2 sqrt(x))
-__device__ __forceinline__ void n_root(double x, double &g, double &h) {
-  const double y = __builtin_amdgcn_rsq(x);
-  g = x * y;
-  h = 0.5 * y;
-  double r = fma(-h, g, 0.5);
-  g = fma(g, r, g);
-  h = fma(h, r, h);
-  r = fma(-h, g, 0.5);
-  h = fma(h, r, h);
-  g = fma(fma(-g, g, x), h, g);
+// FP64 reciprocal and roots to a unit in the last place: v_rcp_f64 and
+// v_rsq_f64 are good to 2^-24 (measured on gfx950: 2^-24.4 and 2^-24.2), so
+// one step of third order (e + e^2, e/2 + 3/8 e^2) reaches 2^-72.
+__device__ __forceinline__ double n_rcp(double x) {
+  const double y = __builtin_amdgcn_rcp(x);
+  const double e = fma(-x, y, 1.0);
+  return fma(y, fma(e, e, e), y);
 }
 __device__ __forceinline__ double n_sqrt(double x) {   // x > 0
-  double g, h;
-  n_root(x, g, h);
-  return g;
+  const double y = __builtin_amdgcn_rsq(x), g = x * y;
+  const double e = fma(-g, y, 1.0);
+  return fma(g * e, fma(e, 0.375, 0.5), g);
 }
 __device__ __forceinline__ double n_rsqrt(double x) {   // x > 0
-  double g, h;
-  n_root(x, g, h);
-  return h + h;
+  const double y = __builtin_amdgcn_rsq(x);
+  const double e = fma(-x * y, y, 1.0);
+  return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
 // Physical constants of one case in the arithmetic type of the kernel.
@@ -86,23 +82,40 @@ struct Prim {
 // and 0 otherwise (the reference forms r and phi with a division each).
 // The reference's guard, |r| > 1e10 or NaN: r becomes 1e6 for b > 0, else
 // -1, so phi is 1e6's or 0 whatever the sign of a.
-__device__ __forceinline__ double half_slope(double a, double b, int lim) {
+// fixed_slope is the value where the guard holds.  That needs a jump beside
+// a difference 1e10 times smaller, flow uniform but for rounding: the waves
+// that meet one take a second pass over the limiters (muscl_guarded).
+template <bool ALBADA>
+__device__ __forceinline__ double half_slope(double a, double b) {
   const double pr = a * b;
   const bool pos = pr > 0.0;
-  const double big = (lim == 1) ? (1.0e12 + 1.0e6) / (1.0e12 + 1.0) : 2.0e6 / (1.0 + 1.0e6);
   double x;
-  if (lim == 1) x = n_div(0.5 * pr * (a + b), pos ? a * a + b * b : 1.0);
-  else x = n_div(pr, pos ? a + b : 1.0);
-  x = pos ? x : pr * 0.0;   // 0, or NaN from a NaN or infinite difference
-  const double g = (b > 0.0) ? 0.5 * a * big : 0.0;
-  return (r_abs(b) > 1.0e10 * r_abs(a)) ? g : x;
+  if (ALBADA) x = 0.5 * pr * (a + b) * n_rcp(fma(a, a, b * b));
+  else x = pr * n_rcp(a + b);
+  return pos ? x : pr * 0.0;   // 0, or NaN from a NaN or infinite difference
 }
-
-__device__ __forceinline__ void muscl(double t0, double t1, double t2, double t3, int lim,
-                                      double &left, double &right) {
-  const double d0 = t1 - t0, d1 = t2 - t1, d2 = t3 - t2;
-  left = t1 + half_slope(d0, d1, lim);
-  right = t2 - half_slope(d2, d1, lim);
+template <bool ALBADA>
+__device__ __forceinline__ double fixed_slope(double a, double b) {
+  const double phi = ALBADA ? (1.0e12 + 1.0e6) / (1.0e12 + 1.0) : 2.0e6 / (1.0 + 1.0e6);
+  return (b > 0.0) ? 0.5 * a * phi : 0.0;
+}
+__device__ __forceinline__ bool slope_guard(double a, double b) { return r_abs(b) > 1.0e10 * r_abs(a); }
+// Left and right values of one variable; guard: whether the reference's
+// guard holds on either side.
+template <bool ALBADA>
+__device__ __forceinline__ void muscl(double q0, double q1, double q2, double q3, double &left,
+                                      double &right, bool &guard) {
+  const double d0 = q1 - q0, d1 = q2 - q1, d2 = q3 - q2;
+  left = q1 + half_slope<ALBADA>(d0, d1);
+  right = q2 - half_slope<ALBADA>(d2, d1);
+  guard = guard | slope_guard(d0, d1) | slope_guard(d2, d1);
+}
+template <bool ALBADA>
+__device__ __forceinline__ void muscl_guarded(double q0, double q1, double q2, double q3,
+                                              double &left, double &right) {
+  const double d0 = q1 - q0, d1 = q2 - q1, d2 = q3 - q2;
+  if (slope_guard(d0, d1)) left = q1 + fixed_slope<ALBADA>(d0, d1);
+  if (slope_guard(d2, d1)) right = q2 - fixed_slope<ALBADA>(d2, d1);
 }
 
 // All-speed Roe flux of one face from the 4-cell stencil (t0,t1 | t2,t3),
@@ -119,22 +132,37 @@ __device__ __forceinline__ void muscl(double t0, double t1, double t2, double t3
 // in FP64 each a chain of 10 to 15 instructions, and the kernels were bound
 // by their FP64 issue.  With the SA functions below and constant divisors as
 // products: 128 steps of the moving 2.6M-cell 2D section 127.7 -> 99.4 ms,
-// 32 steps of the 2.7M-cell 3D section 70.2 -> 57.0 ms.  Error of the 2D flux
-// against 80-bit arithmetic
-// over jumps of 1e-1 .. 1e-6: rms 0.96e-16 (26-division form 0.98e-16).
+// 32 steps of the 2.7M-cell 3D section 70.2 -> 57.0 ms; with third-order
+// reciprocals and roots and the guard out of the common path the stage
+// launches go from 134 to 118 us (2D) and from 294 to 242 us (3D, both with
+// block tiles).  Error of the 2D flux against 80-bit arithmetic over jumps of
+// 1e-1 .. 1e-6: rms 0.97e-16 (26-division form 0.98e-16).
 // Output: (mass, normal, tangential momenta, energy).
 template <int D>
 __device__ __forceinline__ void roe_normal(const Prim<double, D> &t0, const Prim<double, D> &t1,
                                            const Prim<double, D> &t2, const Prim<double, D> &t3, double area,
                                            const PhysR<double> &ph, int lim, double *flux) {
   double lr, rr, lu, ru, lv, rv, lw = 0.0, rw = 0.0, lp, rp;
-  muscl(t0.r, t1.r, t2.r, t3.r, lim, lr, rr);
-  muscl(t0.u, t1.u, t2.u, t3.u, lim, lu, ru);
-  muscl(t0.v, t1.v, t2.v, t3.v, lim, lv, rv);
-  if (D == 3) muscl(t0.w, t1.w, t2.w, t3.w, lim, lw, rw);
-  muscl(t0.p, t1.p, t2.p, t3.p, lim, lp, rp);
+  auto reconstruct = [&](auto albada) {
+    constexpr bool A = decltype(albada)::value;
+    bool guard = false;
+    muscl<A>(t0.r, t1.r, t2.r, t3.r, lr, rr, guard);
+    muscl<A>(t0.u, t1.u, t2.u, t3.u, lu, ru, guard);
+    muscl<A>(t0.v, t1.v, t2.v, t3.v, lv, rv, guard);
+    if (D == 3) muscl<A>(t0.w, t1.w, t2.w, t3.w, lw, rw, guard);
+    muscl<A>(t0.p, t1.p, t2.p, t3.p, lp, rp, guard);
+    if (__any(guard)) {
+      muscl_guarded<A>(t0.r, t1.r, t2.r, t3.r, lr, rr);
+      muscl_guarded<A>(t0.u, t1.u, t2.u, t3.u, lu, ru);
+      muscl_guarded<A>(t0.v, t1.v, t2.v, t3.v, lv, rv);
+      if (D == 3) muscl_guarded<A>(t0.w, t1.w, t2.w, t3.w, lw, rw);
+      muscl_guarded<A>(t0.p, t1.p, t2.p, t3.p, lp, rp);
+    }
+  };
+  if (lim == 1) reconstruct(std::true_type());   // lim is uniform: one branch a face
+  else reconstruct(std::false_type());
   const double ilr = n_rcp(lr);
-  const double plr = lp * ilr, prr = n_div(rp, rr);
+  const double plr = lp * ilr, prr = rp * n_rcp(rr);
   const double lke = (D == 3) ? 0.5 * (lu * lu + lv * lv + lw * lw) : 0.5 * (lu * lu + lv * lv);
   const double rke = (D == 3) ? 0.5 * (ru * ru + rv * rv + rw * rw) : 0.5 * (ru * ru + rv * rv);
   const double hl = ph.cpR * plr + lke, hr = ph.cpR * prr + rke;
@@ -240,6 +268,18 @@ __device__ __forceinline__ float fast_albada(float num, float den) {
   if (!(r <= 1.0e10f)) r = (num > 0.0f) ? 1000000.0f : 0.0f;   // also NaN / inf
   return fmaf(r, r, r) * f_rcp(fmaf(r, r, 1.0f));
 }
+// The same without branches, for the 2D block tiles: a wave's lanes mostly
+// have both signs, so the branches only cost (stage 60.6 -> 56.4 us on the
+// 2.6M-cell section).  In 3D the extra live values spill (123.5 -> 126 us),
+// and in general tiles they cost the learned closure its occupancy.
+template <bool kLeft, bool ALBADA>
+__device__ __forceinline__ float flat_slope(float q, float a, float b) {
+#pragma clang fp contract(off)
+  const float pr = a * b;
+  const float x = ALBADA ? fmaf(kLeft ? 0.5f * a : -0.5f * a, fast_albada(b, a), q)
+                         : fmaf(kLeft ? pr : -pr, f_rcp(a + b), q);
+  return pr > 0.0f ? x : q;
+}
 template <bool kLeft>
 __device__ __forceinline__ float fast_slope(float q, float a, float b, int lim) {
 #pragma clang fp contract(off)
@@ -261,16 +301,31 @@ __device__ __forceinline__ void roe_flux(const Prim<float, D> &t0, const Prim<fl
 #pragma clang fp contract(off)
   const float gama = ph.gama, Rg = ph.Rg, Cv = ph.Cv;
   float lr, rr, lu, ru, lvv, rvv, lw = 0.0f, rw = 0.0f, lp, rp;
-  auto muscl32 = [&](float q0, float q1, float q2, float q3, float &l, float &r) {
-    const float d0 = q1 - q0, d1 = q2 - q1, d2 = q3 - q2;
-    l = fast_slope<true>(q1, d0, d1, lim);
-    r = fast_slope<false>(q2, d2, d1, lim);
+  auto reconstruct = [&](auto m) {
+    m(t0.r, t1.r, t2.r, t3.r, lr, rr);
+    m(t0.u, t1.u, t2.u, t3.u, lu, ru);
+    m(t0.v, t1.v, t2.v, t3.v, lvv, rvv);
+    if (D == 3) m(t0.w, t1.w, t2.w, t3.w, lw, rw);
+    m(t0.p, t1.p, t2.p, t3.p, lp, rp);
   };
-  muscl32(t0.r, t1.r, t2.r, t3.r, lr, rr);
-  muscl32(t0.u, t1.u, t2.u, t3.u, lu, ru);
-  muscl32(t0.v, t1.v, t2.v, t3.v, lvv, rvv);
-  if (D == 3) muscl32(t0.w, t1.w, t2.w, t3.w, lw, rw);
-  muscl32(t0.p, t1.p, t2.p, t3.p, lp, rp);
+  auto flat = [&](auto albada) {
+    constexpr bool A = decltype(albada)::value;
+    reconstruct([&](float q0, float q1, float q2, float q3, float &l, float &r) {
+      const float d0 = q1 - q0, d1 = q2 - q1, d2 = q3 - q2;
+      l = flat_slope<true, A>(q1, d0, d1);
+      r = flat_slope<false, A>(q2, d2, d1);
+    });
+  };
+  if constexpr (D == 2 && DIR >= 0) {
+    if (lim == 1) flat(std::true_type());   // lim is uniform: one branch a face
+    else flat(std::false_type());
+  } else {
+    reconstruct([&](float q0, float q1, float q2, float q3, float &l, float &r) {
+      const float d0 = q1 - q0, d1 = q2 - q1, d2 = q3 - q2;
+      l = fast_slope<true>(q1, d0, d1, lim);
+      r = fast_slope<false>(q2, d2, d1, lim);
+    });
+  }
   const float ilr = f_rcp(lr), irr = f_rcp(rr);
   const float iRg = f_rcp(Rg);
   const float plr = lp * ilr, prr = rp * irr;
@@ -579,6 +634,73 @@ __device__ __forceinline__ void visc_flux_2d(const Prim<float, 2> &L, const Prim
   out[3] = fmaf(qk0, nT * ih, fmaf(fu, t1, fv * t2)) * area;
 }
 
+// The same in 3D (the fused operations are those of the 3D kernels).  t[8]:
+// the tangential stencil, t1 then t2.
+template <int DIR>
+__device__ __forceinline__ void visc_flux_3d(const Prim<float, 3> &L, const Prim<float, 3> &Rr,
+                                             float iL, float iR, const Prim<float, 3> *t, int dir,
+                                             const ViscPhys<float, 3> &vp, float *out, bool turb,
+                                             float nuL, float nuR, float *mflux) {
+#pragma clang fp contract(off)
+  const int d = DIR >= 0 ? DIR : dir;
+  const bool x = d == 0, y = d == 1;
+  auto pf = [](float a, float b, float c, float e) { return 0.25f * (a + b - c - e); };
+  const float n[3] = {Rr.u - L.u, Rr.v - L.v, Rr.w - L.w};
+  const float a[3] = {pf(t[0].u, t[1].u, t[2].u, t[3].u), pf(t[0].v, t[1].v, t[2].v, t[3].v),
+                      pf(t[0].w, t[1].w, t[2].w, t[3].w)};
+  const float b[3] = {pf(t[4].u, t[5].u, t[6].u, t[7].u), pf(t[4].v, t[5].v, t[6].v, t[7].v),
+                      pf(t[4].w, t[5].w, t[6].w, t[7].w)};
+  // gradient of component k along x, y, z: the normal difference along d,
+  // the tangential ones on the other two axes in order
+  float gx[3], gy[3], gz[3];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    gx[k] = x ? n[k] : a[k];
+    gy[k] = y ? n[k] : (x ? a[k] : b[k]);
+    gz[k] = (x || y) ? b[k] : n[k];
+  }
+  const float TL = iL * L.p, TR = iR * Rr.p;
+  const float nT = fmaf(iR, Rr.p, -TL), sT = TL + TR;
+  // (exact; written as sums so that no per-lane table is built)
+  auto axis = [&](float v0, float v1, float v2) {
+    if (DIR >= 0) return DIR == 0 ? v0 : (DIR == 1 ? v1 : v2);
+    return (x ? 1.0f : 0.0f) * v0 + (y ? 1.0f : 0.0f) * v1 + ((x || y) ? 0.0f : 1.0f) * v2;
+  };
+  const float ih = axis(vp.ih0, vp.ih1, vp.ih2), area = axis(vp.ar0, vp.ar1, vp.ar2);
+  const float ftemp = 0.5f * sT;
+  float mu0 = f_sqrt(ftemp * (ftemp * ftemp)) * ((1.0f + vp.SoT) * f_rcp(fmaf(0.5f, sT, vp.SoT)));
+  float qk0 = vp.qk * mu0;
+  if (turb) {
+    const float fvis = (nuL + nuR) * 0.5f;
+    const float froe = (L.r + Rr.r) * 0.5f;
+    const float ir = f_rcp(froe);
+    float bigx = fvis * f_rcp(mu0 * ir);
+    if (bigx < 0.0f) bigx = 0.0f;
+    const float b2 = bigx * bigx;
+    const float rf = froe * (bigx * b2 * f_rcp(fmaf(bigx, b2, (float)SA::cv1three)));
+    *mflux = (fmaf(ir, mu0, fvis) * ((nuR - nuL) * ih)) * c_rcp((float)SA::segma) * area;
+    qk0 = fmaf(vp.qk, mu0, rf * fvis * vp.iqkt);
+    mu0 = fmaf(rf, fvis, mu0);
+  }
+  const float mur = mu0 * vp.iRe, mu2 = 2.0f * mu0;
+  const float dvy = gy[1] * vp.ih1;
+  const float dv3 = fmaf(gz[2], vp.ih2, fmaf(gx[0], vp.ih0, dvy)) * c_rcp(3.0f);
+  const float dn = x ? gx[0] * vp.ih0 : (y ? dvy : gz[2] * vp.ih2);
+  const float tnn = mu2 * (dn - dv3) * vp.iRe;
+  const float txy = mur * fmaf(gy[0], vp.ih1, gx[1] * vp.ih0);
+  const float txz = mur * fmaf(gx[2], vp.ih0, gz[0] * vp.ih2);
+  const float tyz = mur * fmaf(gy[2], vp.ih1, gz[1] * vp.ih2);
+  const float t1 = x ? tnn : (y ? txy : txz), t2 = x ? txy : (y ? tnn : tyz);
+  const float t3 = x ? txz : (y ? tyz : tnn);
+  const float fu = (L.u + Rr.u) * 0.5f, fv = (L.v + Rr.v) * 0.5f, fw = (L.w + Rr.w) * 0.5f;
+  const float uv = x ? fmaf(fv, t2, fu * t1) : fmaf(fu, t1, fv * t2);
+  out[0] = 0.0f;
+  out[1] = t1 * area;
+  out[2] = t2 * area;
+  out[3] = t3 * area;
+  out[4] = fmaf(qk0, nT * ih, fmaf(fw, t3, uv)) * area;
+}
+
 // The viscous flux from the stencil cells' states.
 template <typename R, int D>
 __device__ __forceinline__ void visc_flux_cells(const Prim<R, D> &L, const Prim<R, D> &Rr,
@@ -589,6 +711,9 @@ __device__ __forceinline__ void visc_flux_cells(const Prim<R, D> &L, const Prim<
     const float tu[4] = {t[0].u, t[1].u, t[2].u, t[3].u}, tv[4] = {t[0].v, t[1].v, t[2].v, t[3].v};
     visc_flux_2d<-1>(L, Rr, f_rcp(L.r * vp.Rg), f_rcp(Rr.r * vp.Rg), tu, tv, d, vp, out, turb, nuL,
                      nuR, mflux);
+  } else if constexpr (sizeof(R) == 4) {
+    visc_flux_3d<-1>(L, Rr, f_rcp(L.r * vp.Rg), f_rcp(Rr.r * vp.Rg), t, d, vp, out, turb, nuL, nuR,
+                     mflux);
   } else {
     VelT<R> vt[(D == 3) ? 8 : 4];
 #pragma unroll

@@ -384,17 +384,170 @@ __device__ __forceinline__ void visc_prep_block(const ViscArgs<R, 2> &a, const T
   block_visc_cell<R>(a, ti, bi, P, b);
 }
 
+// ---- 3D
+template <typename R>
+struct Block3Lds {
+  typename V4<R>::T *F;   // fluxes of one direction: values 0..3
+  R *Fe;                  // value 4
+  typename V4<R>::T *S;   // states (roe, u, v, w)
+  R *e, *nu;              // pressure (viscous pass, FP64: temperature); SA
+};
+template <typename R>
+__device__ __forceinline__ Block3Lds<R> block3_lds(unsigned char *smem, int cells) {
+  Block3Lds<R> b;
+  b.F = reinterpret_cast<typename V4<R>::T *>(smem);
+  b.Fe = reinterpret_cast<R *>(b.F + kFlux3);
+  b.S = reinterpret_cast<typename V4<R>::T *>(smem + blk3_state_offset(sizeof(R)));
+  b.e = reinterpret_cast<R *>(b.S + cells);
+  b.nu = b.e + cells;
+  return b;
+}
+template <typename R>
+__device__ __forceinline__ Prim<R, 3> box3_prim(const Block3Lds<R> &b, int p) {
+  const typename V4<R>::T q = b.S[p];
+  return Prim<R, 3>{q.x, q.y, q.z, q.w, b.e[p]};
+}
+
+// The block and its halo into LDS (the caller syncs).  VISC: layer 1 and the
+// edges into the viscous pass's box; otherwise layers 1 and 2.
+template <typename R, bool VISC>
+__device__ __forceinline__ void block3_load(const Pack<R, 3> &W, const R *nu, bool turb,
+                                            const int *halo, const TileInfo &ti, R Rg,
+                                            const Block3Lds<R> &b) {
+  const int i = threadIdx.x;
+  // second entry of this thread: an edge (80 of them) or a cell of layer 2
+  const bool has1 = !VISC || i < kHalo3E - kHalo3L1;
+  const int h1 = VISC ? kHalo3L1 + i : kHalo3E + i;
+  const int c0 = halo[ti.halo0 + i];
+  const int c1 = has1 ? halo[ti.halo0 + h1] : 0;
+  auto put = [&](int x, int y, int z, const typename V4<R>::T &q, R p, bool n, R nv) {
+    const int k = VISC ? vbox3_pos(x, y, z) : box3_pos(x, y, z);
+    b.S[k] = q;
+    b.e[k] = (VISC && sizeof(R) == 8) ? v_div(p, q.x * Rg) : p;
+    if (n) b.nu[k] = nv;
+  };
+  const int c = ti.cell0 + i;
+  const typename V4<R>::T q = W.a[c], q0 = W.a[c0];
+  const R p = W.e[c], p0 = W.e[c0];
+  const R n = turb ? nu[c] : R(0), n0 = turb ? nu[c0] : R(0);
+  int x, y, z;
+  if (has1) {
+    const typename V4<R>::T q1 = W.a[c1];
+    const R p1 = W.e[c1];
+    halo3_xyz(h1, x, y, z);
+    put(x, y, z, q1, p1, false, R(0));
+  }
+  halo3_xyz(i, x, y, z);
+  put(x, y, z, q0, p0, turb, n0);
+  blk_xyz(i, x, y, z);
+  put(x, y, z, q, p, turb, n);
+}
+
+// Face f of a block in direction d: f < 256 the low face of cell f, then the
+// high faces of the last layer; its high-side cell's coordinates
+template <int d>
+__device__ __forceinline__ void block3_face(int f, int &x, int &y, int &z) {
+  if (f < kBlkCells) {
+    blk_xyz(f, x, y, z);
+    return;
+  }
+  const int e = f - kBlkCells, a = e & 7, b = e >> 3;
+  x = d == 0 ? kB3X : a;
+  y = d == 0 ? a : (d == 1 ? kB3Y : b);
+  z = d == 2 ? kB3Z : b;
+}
+template <int d> constexpr int kBlock3Faces = kBlkCells + (d == 2 ? 64 : 32);
+
+// The viscous pass of a 3D block tile (visc_prep_tile's work), one direction
+// at a time.
+template <typename R>
+__device__ __forceinline__ void visc_prep_block3(const ViscArgs<R, 3> &a, const TileInfo &ti,
+                                                 unsigned char *smem_raw, int *halt, bool herr) {
+  using V = typename V4<R>::T;
+  auto &bi = uni(a.blk)[ti.blk];
+  auto &P = uni(a.phys)[bi.case_id];
+  const Block3Lds<R> b = block3_lds<R>(smem_raw, kVBox3Cells);
+  if (threadIdx.x == 0) *halt = herr ? 1 : 0;
+  int cx, cy, cz;
+  blk_xyz(threadIdx.x, cx, cy, cz);
+  double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, tot = 0.0;
+  if (a.viscous) {
+    block3_load<R, true>(a.W, a.nu, a.turb, a.halo, ti, (R)P.Rg, b);
+    const ViscPhys<R, 3> vp = visc_phys<R, 3>(bi, P);
+    __syncthreads();
+    auto direction = [&](auto dc) {
+      constexpr int d = decltype(dc)::value;
+      constexpr int st[3] = {1, kVBox3P, kVBox3Plane};
+      constexpr int sn = st[d], s1 = st[d == 0 ? 1 : 0], s2 = st[d == 2 ? 1 : 2];
+#pragma unroll 1
+      for (int f = (threadIdx.x - 64 * d) & 255; f < kBlock3Faces<d>; f += kBlkCells) {
+        int x, y, z;
+        block3_face<d>(f, x, y, z);
+        const int p = vbox3_pos(x, y, z), l = p - sn;
+        const int tp[8] = {l + s1, p + s1, l - s1, p - s1, l + s2, p + s2, l - s2, p - s2};
+        const R nl = a.turb ? b.nu[l] : R(0), nr = a.turb ? b.nu[p] : R(0);
+        R out[5], mf = R(0);
+        if constexpr (sizeof(R) == 4) {
+          Prim<R, 3> t[8];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) t[k] = box3_prim<R>(b, tp[k]);
+          const Prim<R, 3> L = box3_prim<R>(b, l), Rr = box3_prim<R>(b, p);
+          visc_flux_3d<d>(L, Rr, f_rcp(L.r * vp.Rg), f_rcp(Rr.r * vp.Rg), t, d, vp, out, a.turb, nl, nr, &mf);
+        } else {
+          auto cell = [&](int q) {
+            const V v = b.S[q];
+            return VelT<R>{v.y, v.z, v.w, b.e[q]};
+          };
+          VelT<R> t[8];
+#pragma unroll
+          for (int k = 0; k < 8; ++k) t[k] = cell(tp[k]);
+          visc_flux<R, 3>(cell(l), cell(p), b.S[l].x, b.S[p].x, t, d, vp, out, a.turb, nl, nr, &mf);
+        }
+        V o;
+        o.x = mf; o.y = out[1]; o.z = out[2]; o.w = out[3];
+        const int k = flux3_slot(d, x, y, z);
+        b.F[k] = o;
+        b.Fe[k] = out[4];
+      }
+      __syncthreads();
+      const int k = flux3_slot(d, cx, cy, cz), h = k + flux3_step(d);
+      const V lo = b.F[k], hi = b.F[h];
+      s[1] += (double)hi.y - (double)lo.y;
+      s[2] += (double)hi.z - (double)lo.z;
+      s[3] += (double)hi.w - (double)lo.w;
+      s[4] += (double)b.Fe[h] - (double)b.Fe[k];
+      if (a.turb) {
+        tot += -(double)lo.x;
+        tot += (double)hi.x;
+      }
+      if (d < 2) __syncthreads();   // the next direction rewrites the fluxes
+    };
+    direction(std::integral_constant<int, 0>());
+    direction(std::integral_constant<int, 1>());
+    direction(std::integral_constant<int, 2>());
+  } else {
+    __syncthreads();
+  }
+  if (*halt) return;   // uniform: written before the barriers
+  const int c = ti.cell0 + threadIdx.x;
+  const R rv[5] = {(R)s[0], (R)s[1], (R)s[2], (R)s[3], (R)s[4]};
+  vstore<R, 3>(a.Rv, c, rv);
+  if (a.turb) a.mutf[c] = (R)n_div(n_div(tot, bi.vol), P.Re);
+}
+
+// (waves per SIMD as the LDS of its block tiles allows; the 3D FP64 form
+// takes 184 registers unless held to three)
 template <typename R, int D>
-__global__ void __launch_bounds__(kTile) k_visc_prep(ViscArgs<R, D> a) {
+__global__ void __launch_bounds__(kTile, ((D == 3 && sizeof(R) == 8) ? 3 : 1))
+k_visc_prep(ViscArgs<R, D> a) {
   extern __shared__ __align__(32) unsigned char smem_raw[];
   __shared__ int halt;
   const bool herr = halted(a.err);
   const TileInfo ti = tile_info(a.tiles, dispatch_tile());
-  if constexpr (D == 2) {
-    if (ti.halo0 >= 0) {
-      visc_prep_block<R>(a, ti, smem_raw, &halt, herr);
-      return;
-    }
+  if (ti.halo0 >= 0) {
+    if constexpr (D == 2) visc_prep_block<R>(a, ti, smem_raw, &halt, herr);
+    else visc_prep_block3<R>(a, ti, smem_raw, &halt, herr);
+    return;
   }
   visc_prep_tile<R, D>(a, ti, smem_raw, &halt, herr);
 }
@@ -470,6 +623,16 @@ constexpr int kMlSlots = 64, kMlSlotStride = 16;
 // 16-byte chunks XOR-swizzled by the row, see mlp_fwd_reg), b1, b2 and the
 // bf16 w3.
 constexpr size_t kStageMlSmem = (size_t)64 * 8 * 2 + (size_t)64 * 64 * 2 + 2 * 64 * 4 + 64 * 2;
+// byte offset of that region in a block tile: over its states; in 3D the
+// cells' residuals follow it
+template <int D>
+__host__ __device__ constexpr size_t blk_ml_offset() {
+  return D == 2 ? blk_state_offset(sizeof(float)) : blk3_state_offset(sizeof(float));
+}
+template <int D>
+__host__ __device__ constexpr size_t blk_ml_smem() {
+  return blk_ml_offset<D>() + kStageMlSmem + (D == 3 ? (size_t)kTile * 5 * sizeof(double) : 0);
+}
 // byte offset of that region for a tile of nface faces (16-byte aligned)
 template <typename R, int D>
 __host__ __device__ constexpr size_t ml_smem_offset(int nface) {
@@ -610,7 +773,60 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
     asm volatile("" : "+v"(i));
     blk_xy(i, x, y);
   };
-  if constexpr (BLK) {
+  const Block3Lds<R> b3 = block3_lds<R>(smem_raw, kBox3Cells);
+  double s[NV];   // residual of the cell
+#pragma unroll
+  for (int k = 0; k < NV; ++k) s[k] = 0.0;
+  if constexpr (BLK && D == 3) {
+    if (threadIdx.x == 0) halt = herr ? 1 : 0;
+    block3_load<R, false>(a.Win, a.nuin, a.turb, a.halo, ti, R(0), b3);
+    __syncthreads();
+    // phase 1, one direction at a time: the low face of every cell and the
+    // last layer's high faces (each direction's by another wave), then the
+    // direction's part of the cells' residuals
+    auto direction = [&](auto dc) {
+      constexpr int d = decltype(dc)::value;
+#pragma unroll 1
+      for (int f = (threadIdx.x - 64 * d) & 255; f < kBlock3Faces<d>; f += kBlkCells) {
+        int x, y, z;
+        block3_face<d>(f, x, y, z);
+        int q[4];
+        const int p = box3_in(x, y, z);
+        if constexpr (d < 2) {
+          constexpr int st = d == 0 ? 1 : 12;
+          q[0] = p - 2 * st; q[1] = p - st; q[2] = p; q[3] = p + st;
+        } else {
+          const int hz = box3_zhalo(x, y, 0);   // planes -1, 4, -2, 5 follow, 64 apart
+          q[0] = z >= 2 ? p - 2 * kBox3Plane : hz + (z == 1 ? 0 : 128);
+          q[1] = z >= 1 ? p - kBox3Plane : hz;
+          q[2] = z <= 3 ? p : hz + 64;
+          q[3] = z <= 2 ? p + kBox3Plane : hz + (z == 3 ? 64 : 192);
+        }
+        R flux[5];
+        roe_flux<3, d>(box3_prim<R>(b3, q[0]), box3_prim<R>(b3, q[1]), box3_prim<R>(b3, q[2]),
+                       box3_prim<R>(b3, q[3]), d, (R)bi.area[d], ph, a.limiter, flux);
+        V o;
+        o.x = flux[0]; o.y = flux[1]; o.z = flux[2]; o.w = flux[3];
+        const int k = flux3_slot(d, x, y, z);
+        b3.F[k] = o;
+        b3.Fe[k] = flux[4];
+      }
+      __syncthreads();
+      int x, y, z;
+      blk_xyz(threadIdx.x, x, y, z);
+      const int k = flux3_slot(d, x, y, z), h = k + flux3_step(d);
+      const V lo = b3.F[k], hi = b3.F[h];
+      s[0] += (double)lo.x - (double)hi.x;
+      s[1] += (double)lo.y - (double)hi.y;
+      s[2] += (double)lo.z - (double)hi.z;
+      s[3] += (double)lo.w - (double)hi.w;
+      s[NV - 1] += (double)b3.Fe[k] - (double)b3.Fe[h];
+      if (d < 2) __syncthreads();   // the next direction rewrites the fluxes
+    };
+    direction(std::integral_constant<int, 0>());
+    direction(std::integral_constant<int, 1>());
+    direction(std::integral_constant<int, 2>());
+  } else if constexpr (BLK) {
     bool loaded = false;
     if constexpr (kFuseVisc<R, D>) {
       if (a.fuse_visc && a.va.viscous) {
@@ -691,23 +907,18 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
       }
     }
   }
-  if (threadIdx.x == 0) halt = herr ? 1 : 0;
-  __syncthreads();
+  if constexpr (!(BLK && D == 3)) {
+    if (threadIdx.x == 0) halt = herr ? 1 : 0;
+    __syncthreads();
+  }
   if (halt) return;   // uniform: the flag was written before the barrier
 
   const double level_ts = a.alpha * uni(a.dt)[bi.case_id] * bi.step_num;
-  double mx[NV], sq[NV];
-#pragma unroll
-  for (int k = 0; k < NV; ++k) { mx[k] = 0.0; sq[k] = 0.0; }
-  double nmx = 0.0, nsq = 0.0;
   const int i = threadIdx.x;
-  const bool live = i < ti.ncell;
+  const bool live = BLK || i < ti.ncell;
   const int c = ti.cell0 + (live ? i : 0);
   const uint8_t fg = live ? a.flags[c] : 0;
   // ---- phase 2a: residual of the cell, the SA terms
-  double s[NV];
-#pragma unroll
-  for (int k = 0; k < NV; ++k) s[k] = 0.0;
   double snu = 0.0;
   bool sa_on = false;
   bool use_ml = false;
@@ -732,9 +943,9 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
   auto residual = [&]() {
     if constexpr (ML && !BLK) load_slots(sl);
     int bx = 0, by = 0;
-    if constexpr (BLK) my_xy(bx, by);
+    if constexpr (BLK && D == 2) my_xy(bx, by);
 #pragma unroll
-    for (int d = 0; d < D; ++d) {
+    for (int d = 0; d < ((BLK && D == 3) ? 0 : D); ++d) {
       V lo, hi;
       if constexpr (BLK) {
         const int k = by * kBoxP + bx;
@@ -762,14 +973,29 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
     if (a.turb && (fg & F_UPDATE) && (fg & F_SA)) {
       sa_on = true;
       Prim<R, D> me;
-      int bx = 0, by = 0;
-      if constexpr (BLK) my_xy(bx, by);
-      if constexpr (BLK) me = box_prim<R>(bl, box_pos(bx, by));
-      else me = pload<R, D>(a.Win, c);
+      int bx = 0, by = 0, bz = 0;
+      if constexpr (BLK && D == 2) {
+        my_xy(bx, by);
+        me = box_prim<R>(bl, box_pos(bx, by));
+      } else if constexpr (BLK) {
+        blk_xyz(threadIdx.x, bx, by, bz);
+        me = box3_prim<R>(b3, box3_in(bx, by, bz));
+      } else {
+        me = pload<R, D>(a.Win, c);
+      }
       R nl[3], nr[3], ul[3], ur[3], vl[3], vr[3], wl[3], wr[3];
 #pragma unroll
       for (int d = 0; d < 3; ++d) {
-        if (BLK && d < D) {
+        if (BLK && D == 3) {
+          const int p = box3_in(bx, by, bz), hz = box3_zhalo(bx, by, 0);
+          const int lp = d == 0 ? p - 1 : (d == 1 ? p - 12 : (bz > 0 ? p - kBox3Plane : hz));
+          const int rp = d == 0 ? p + 1 : (d == 1 ? p + 12 : (bz < 3 ? p + kBox3Plane : hz + 64));
+          const V lo = b3.S[lp], hi = b3.S[rp];
+          ul[d] = lo.y; vl[d] = lo.z; wl[d] = lo.w;
+          ur[d] = hi.y; vr[d] = hi.z; wr[d] = hi.w;
+          nl[d] = b3.nu[lp];
+          nr[d] = b3.nu[rp];
+        } else if (BLK && d < D) {
           const int p = box_pos(bx, by), st = d == 0 ? 1 : kBoxP;
           const V lo = bl.S[p - st], hi = bl.S[p + st];
           ul[d] = lo.y; vl[d] = lo.z; wl[d] = R(0);
@@ -787,7 +1013,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
         }
       }
       const R T = v_div(me.p, me.r * (R)P.Rg);
-      const R nu = BLK ? bl.nu[box_pos(bx, by)] : a.nuin[c];
+      const R nu = !BLK ? a.nuin[c] : (D == 2 ? bl.nu[box_pos(bx, by)] : b3.nu[box3_in(bx, by, bz)]);
       const R sd = kMixed ? (R)a.sd32[c] : (R)a.signdis[c];
       if constexpr (!ML) {
         snu = (double)sa_source<R, D>(me.u, me.v, me.w, T, me.r, nu, sd, nl, nr, ul, ur, vl, vr,
@@ -829,9 +1055,16 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
   // ---- learned closure: the network for the cells in its range
   if constexpr (ML) {
     unsigned char *wbase = smem_raw + (wres ? (size_t)a.mlw_off
-                                       : BLK ? blk_state_offset(sizeof(R)) : ml_smem_offset<R, D>(ti.nface));
+                                       : BLK ? blk_ml_offset<D>() : ml_smem_offset<R, D>(ti.nface));
+    // a 3D block's residual waits in LDS behind the weights (in registers it
+    // spills across the network)
+    double *keep = reinterpret_cast<double *>(smem_raw + (wres ? (size_t)a.mlw_off : blk_ml_offset<D>()) + kStageMlSmem);
+    if (!wres) __syncthreads();   // every phase-2a read of what the weights overwrite is done
+    if constexpr (BLK && D == 3) {
+#pragma unroll
+      for (int k = 0; k < NV; ++k) keep[k * kTile + threadIdx.x] = s[k];
+    }
     if (!wres) {
-      __syncthreads();   // every phase-2a read of what the weights overwrite is done
       ml_fill_weights(a.mlp, wbase);
       __syncthreads();
     }
@@ -869,7 +1102,11 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
         atomicAdd(&mlc[1], (unsigned)__popcll(nf));
       }
     }
-    if (live) residual();   // the face fluxes are still in LDS
+    if constexpr (BLK && D == 3) {
+#pragma unroll
+      for (int k = 0; k < NV; ++k) s[k] = keep[k * kTile + threadIdx.x];
+    }
+    if (live) residual();   // (2D and general tiles) the face fluxes are still in LDS
   }
   // ---- phase 2b: update
   if (live) {
@@ -953,13 +1190,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
       if (fg & F_RESID) {
         bool nan = (snu != snu);
 #pragma unroll
-        for (int k = 0; k < NV; ++k) {
-          mx[k] = fabs(s[k]);
-          sq[k] = s[k] * s[k];
-          nan = nan || (s[k] != s[k]);
-        }
-        nmx = fabs(snu);
-        nsq = snu * snu;
+        for (int k = 0; k < NV; ++k) nan = nan || (s[k] != s[k]);
         // a NaN residual aborts the march (ResinDomain, NS_Solver.H:355-375)
         if (nan) report_error(a.err, c, 268);
       }
@@ -968,11 +1199,13 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
   if (a.last) {
     // the wave's partials as 16 slots: maxima (|s_k|, then |snu|) in 0..7,
     // sums of squares in the same order in 8..15, zeros in the rest
+    const bool counted = live && (fg & F_RESID);
     double v[16];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
-      v[j] = j < NV ? mx[j < NV ? j : 0] : (j == NV ? nmx : 0.0);
-      v[8 + j] = j < NV ? sq[j < NV ? j : 0] : (j == NV ? nsq : 0.0);
+      const double x = counted ? (j < NV ? s[j < NV ? j : 0] : (j == NV ? snu : 0.0)) : 0.0;
+      v[j] = fabs(x);
+      v[8 + j] = x * x;
     }
     const double r = wave_slots16(v);
     const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -1021,11 +1254,9 @@ __device__ __forceinline__ void stage_launch(const StageArgs<R, D> &a) {
   auto one = [&](int tile) {
     const bool herr = halted(a.err);
     const TileInfo ti = tile_info(a.tiles, tile);
-    if constexpr (D == 2) {
-      if (ti.halo0 >= 0) {
-        stage_tile<R, D, ML, P, true>(a, ti, tile, herr, sh);
-        return;
-      }
+    if (ti.halo0 >= 0) {
+      stage_tile<R, D, ML, P, true>(a, ti, tile, herr, sh);
+      return;
     }
     stage_tile<R, D, ML, P, false>(a, ti, tile, herr, sh);
   };
@@ -1052,8 +1283,13 @@ __device__ __forceinline__ void stage_launch(const StageArgs<R, D> &a) {
   }
 }
 
+// Waves per SIMD the stage kernels are compiled for (the LDS of their block
+// tiles allows as many)
+template <typename R, int D>
+constexpr int kStageWaves = sizeof(R) == 4 ? (D == 2 ? 8 : 6) : (D == 2 ? 4 : 3);
+
 template <typename R, int D, bool ML, bool P = false>
-__global__ void __launch_bounds__(kTile) k_stage(StageArgs<R, D> a) {
+__global__ void __launch_bounds__(kTile, (P ? 1 : kStageWaves<R, D>)) k_stage(StageArgs<R, D> a) {
   stage_launch<R, D, ML, P>(a);
 }
 

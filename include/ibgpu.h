@@ -385,7 +385,7 @@ ibg_status ibg_last_timing(ibg_ctx *ctx, double *total_ms,
  * kernel of step ts, stage subt, reps times back to back on the context
  * stream between two HIP events.  avg_ms = elapsed / reps; cells and faces
  * are the normal cells one launch processes and the faces it takes from face
- * lists (square tiles of 2D meshes list none).  The state is
+ * lists (block tiles list none).  The state is
  * advanced by the repeated stages (use it after the run being measured).   */
 ibg_status ibg_bench_stage(ibg_ctx *ctx, int32_t ts, int32_t subt, int32_t reps,
                            double *avg_ms, int64_t *cells, int64_t *faces);

@@ -1,7 +1,8 @@
-"""Block tiles (16 x 16 squares of cells processed without face lists, used
-with the default tile of 256 cells) against general tiles over the same
-cells (a tile of 128 cells has none): the same state after a sub-cycling
-period, bit for bit in the mixed mode, to rounding in FP64."""
+"""Block tiles (16 x 16 squares, in 3D 8 x 8 x 4 boxes of cells processed
+without face lists, used with the default tile of 256 cells) against general
+tiles over the same cells (a tile of 128 cells has none): the same state
+after a sub-cycling period, bit for bit in the mixed mode, to rounding in
+FP64."""
 import numpy as np
 import pytest
 
@@ -11,10 +12,10 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.fixture(scope="module")
-def mesh():
-    # ragged base: squares, general runs between them and partial tiles on
-    # every level
-    return ibgpu.Mesh(ibgpu.config2(levels=5, base=90))
+def meshes():
+    # ragged bases: blocks, general runs between them and partial tiles on
+    # every level; spans of 3, 6 and 12 cells
+    return {2: ibgpu.Mesh(ibgpu.config2(levels=5, base=90)), 3: ibgpu.Mesh(ibgpu.config3(levels=4, base=42, nz=3))}
 
 
 def flow(mesh):
@@ -23,6 +24,8 @@ def flow(mesh):
     fv[:, 0] *= 1.0 + 0.01 * np.sin(3.0 * x[:, 0] + x[:, 1])
     fv[:, 1] *= 1.0 - 0.8 * np.exp(-d / 0.05)
     fv[:, 2] += 0.02 * np.cos(2.0 * x[:, 1] - x[:, 0])
+    if mesh.dim == 3:
+        fv[:, 3] += 0.01 * np.sin(60.0 * x[:, 2] + x[:, 0])
     fv[:, 4] *= 1.0 + 0.01 * np.cos(x[:, 0] * 2.0)
     nut = mesh.phys[0].nut_inf * (1.0 - 0.9 * np.exp(-d / 0.1))
     return fv, nut
@@ -38,10 +41,12 @@ CASES = [
 ]
 
 
+@pytest.mark.parametrize("dim", [2, 3])
 @pytest.mark.parametrize("mode,closure,opt", CASES)
-def test_block_tiles_equal_general_tiles(mesh, mode, closure, opt):
+def test_block_tiles_equal_general_tiles(meshes, dim, mode, closure, opt):
+    mesh = meshes[dim]
     fv, nut = flow(mesh)
-    steps = 16 if opt.get("temporal_refine", True) else 2
+    steps = 1 << (mesh.nlevels - 1) if opt.get("temporal_refine", True) else 2
     if opt.get("nstage", 3) == 1:
         steps = 1
     got = {}
