@@ -194,29 +194,37 @@ __global__ void k_closure_pack(const float *p, __bf16 *W1t, __bf16 *W2t, __bf16 
 
 // Stand-alone inference over raw feature rows: z = zmean + zstd * y, with
 // the register forward of the stage kernel (mlp_fwd_reg): 64 rows per wave,
-// one row per lane.
+// one row per lane.  X and Z may be pinned host memory: a row is two 16-byte
+// loads and a wave's 64 results one 256-byte store, so the rows cross the
+// link as the kernel runs (16384 rows in 13.6 us, 43 GB/s: the link bounds
+// it).  The weights go to LDS in 16-byte chunks.
 __global__ void __launch_bounds__(256) k_closure_infer(MlpDev M, const float *X, float *Zout, long long n) {
-  __shared__ __align__(16) __bf16 sW1t[64 * kX];
-  __shared__ __align__(16) __bf16 sW2p[64 * 64];
-  __shared__ __align__(16) float sb1[64], sb2[64];
-  __shared__ __align__(16) __bf16 sw3[64];
-  for (int i = threadIdx.x; i < 64 * kX; i += blockDim.x) sW1t[i] = M.W1t[i];
-  for (int i = threadIdx.x; i < 64 * 64; i += blockDim.x) sW2p[i] = M.W2p[i];
-  for (int i = threadIdx.x; i < 64; i += blockDim.x) { sw3[i] = (__bf16)M.w3[i]; sb1[i] = M.b1[i]; sb2[i] = M.b2[i]; }
-  __syncthreads();
+  __shared__ __align__(16) unsigned char smem[kStageMlSmem];
   const long long row = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+  float x[kMlpIn] = {};
+  if (row < n) {
+    const float4 x0 = *reinterpret_cast<const float4 *>(X + row * kMlpIn);
+    const float4 x1 = *reinterpret_cast<const float4 *>(X + row * kMlpIn + 4);
+    x[0] = x0.x; x[1] = x0.y; x[2] = x0.z; x[3] = x0.w;
+    x[4] = x1.x; x[5] = x1.y; x[6] = x1.z; x[7] = x1.w;
+  }
+  ml_fill_weights(M, smem);
+  __syncthreads();
+  const __bf16 *sW1t = reinterpret_cast<const __bf16 *>(smem), *sW2p = sW1t + 64 * 8;
+  const float *sb1 = reinterpret_cast<const float *>(sW2p + 64 * 64), *sb2 = sb1 + 64;
+  const __bf16 *sw3 = reinterpret_cast<const __bf16 *>(sb2 + 64);
   bf16x8_t xf;
 #pragma unroll
   for (int k = 0; k < kMlpIn; ++k)
-    xf[k] = (__bf16)(row < n ? (X[row * kMlpIn + k] - M.fmean[k]) * M.finv[k] : 0.0f);
+    xf[k] = (__bf16)(row < n ? (x[k] - uni(M.fmean)[k]) * uni(M.finv)[k] : 0.0f);
   const int lane = threadIdx.x & 63;
   float yown = 0.0f;
 #pragma unroll 1
   for (int sb = 0; sb < 2; ++sb) {
-    const float y = mlp_fwd_reg(xf, sb, sW1t, sW2p, sb1, sb2, sw3);
+    const float y = mlp_fwd_reg<8>(xf, sb, sW1t, sW2p, sb1, sb2, sw3);
     if ((lane >> 5) == sb) yown = y;
   }
-  if (row < n) Zout[row] = M.zst[0] + M.zst[1] * (yown + M.b3[0]);
+  if (row < n) Zout[row] = uni(M.zst)[0] + uni(M.zst)[1] * (yown + uni(M.b3)[0]);
 }
 
 // Forward + backward of 64 rows per workgroup (4 waves x 16 rows), loss
