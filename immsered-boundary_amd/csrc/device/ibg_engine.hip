@@ -117,7 +117,10 @@ struct ibg_ctx {
   int4 *dmg = nullptr;
   DmgWall *dmgw = nullptr;      // wall ghosts (BC -81), parallel to dmg; null without walls
   double *dist_dm = nullptr;    // [N] distance to the domain walls; null without walls
-  int *res_ci = nullptr, *res_fi = nullptr, *pro_ci = nullptr, *pro_fi = nullptr;
+  int2 *res_cc = nullptr, *pro_cc = nullptr;   // (coarse cell, case) per pair
+  int4 *res_fi = nullptr;                      // [pairs][2] the sons
+  int *pro_fi = nullptr, *pro_nb = nullptr;    // [pairs][8] sons; [6][pairs] neighbours
+  int npro = 0;
   // optional coarse/fine flux balance: pairs, tile face -> balanced-flux
   // entry, the balanced inviscid / viscous fluxes [nrf][5][NV] (R-typed)
   int nrf = 0;
@@ -181,7 +184,7 @@ struct ibg_ctx {
       }
     }
   } infer;
-  double *dt = nullptr, *cflpart = nullptr, *rpart = nullptr, *resid = nullptr, *probe = nullptr;
+  double *dt = nullptr, *cflpart = nullptr, *rpart = nullptr, *probe = nullptr;
   unsigned long long *err = nullptr;
   unsigned long long *err2 = nullptr;   // error word of the next step's move, run ahead
   int last_ntiles = 0;
@@ -198,6 +201,10 @@ struct ibg_ctx {
   int64_t last_stage_launches = 0, last_updates = 0;
   std::vector<void *> allocs;
   std::string errmsg;
+  // pinned words that kernels write their results to (a copy command per
+  // result otherwise): march end [2], residual or force [cases][kRpart]
+  unsigned long long *hword = nullptr;
+  double *hres = nullptr;
   void *hstage = nullptr;      // pinned host staging of the state boundary
   size_t hstage_bytes = 0;
 
@@ -603,9 +610,9 @@ ibg_status launch_exchange(ibg_ctx *c, int ts) {
     if (!transfer_due(c, l, ts)) continue;
     const int n = c->res_off[l + 1] - c->res_off[l];
     if (n > 0) {
-      hipLaunchKernelGGL((k_restrict<D>), dim3(grid(n, 256)), dim3(256), 0, c->s, n,
-                         c->res_ci + c->res_off[l], c->res_fi + (size_t)8 * c->res_off[l],
-                         c->sout<D>(), c->blk_twod[l + 1], c->phys, c->cellcase);
+      hipLaunchKernelGGL((k_restrict<D>), dim3(grid(n, 64)), dim3(64), 0, c->s, n,
+                         c->res_cc + c->res_off[l], c->res_fi + (size_t)2 * c->res_off[l],
+                         c->sout<D>(), c->blk_twod[l + 1], c->phys);
       HIPCHK(hipGetLastError());
     }
   }
@@ -613,9 +620,10 @@ ibg_status launch_exchange(ibg_ctx *c, int ts) {
     if (!transfer_due(c, l, ts)) continue;
     const int n = c->pro_off[l + 1] - c->pro_off[l];
     if (n > 0) {
-      hipLaunchKernelGGL((k_prolong<D>), dim3(grid(n, 256)), dim3(256), 0, c->s, n,
-                         c->pro_ci + c->pro_off[l], c->pro_fi + (size_t)8 * c->pro_off[l],
-                         c->nb27, c->sout<D>(), c->blk_twod[l + 1], c->phys, c->cellcase);
+      const int nt = n * (c->blk_twod[l + 1] ? 4 : 8);
+      hipLaunchKernelGGL((k_prolong<D>), dim3(grid(nt, 64)), dim3(64), 0, c->s, n,
+                         c->pro_cc + c->pro_off[l], c->pro_fi + (size_t)8 * c->pro_off[l],
+                         c->pro_nb + c->pro_off[l], c->npro, c->sout<D>(), c->blk_twod[l + 1], c->phys);
       HIPCHK(hipGetLastError());
     }
   }
@@ -781,8 +789,7 @@ ibg_status run_step(ibg_ctx *c, int ts, bool joined, bool ahead) {
 }
 
 ibg_status reset_err(ibg_ctx *c) {
-  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, c->s, c->err, 1, ~0ull);
-  hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, c->s, c->err2, 1, ~0ull);
+  hipLaunchKernelGGL(k_march_begin, dim3(1), dim3(64), 0, c->s, c->err, c->err2, (unsigned long long *)nullptr, 0);
   HIPCHK(hipGetLastError());
   return IBG_OK;
 }
@@ -1146,6 +1153,12 @@ ibg_status ibg_create(const ibg_config *cfg, ibg_ctx **out) {
   }
   (void)hipEventCreate(&c->ev0);
   (void)hipEventCreate(&c->ev1);
+  if (hipHostMalloc((void **)&c->hword, 2 * sizeof(unsigned long long) + sizeof(double) * IBG_MAX_CASES * kRpart,
+                    hipHostMallocDefault) != hipSuccess) {
+    ibg_destroy(c);
+    return IBG_ERR_HIP;
+  }
+  c->hres = (double *)(c->hword + 2);
   *out = c;
   return IBG_OK;
 }
@@ -1164,6 +1177,7 @@ ibg_status ibg_destroy(ibg_ctx *c) {
   if (c->s) (void)hipStreamDestroy(c->s);
   if (c->hstage) (void)hipHostFree(c->hstage);
   c->infer.release();
+  if (c->hword) (void)hipHostFree(c->hword);
   delete c;
   return IBG_OK;
 }
@@ -1574,31 +1588,44 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
     c->ndmg_corner = (int)corner.size();
   }
   // ---- pairs grouped by coarse level
-  std::vector<int> res_ci, res_fi, pro_ci, pro_fi;
+  std::vector<int2> res_cc, pro_cc;
+  std::vector<int> res_son, pro_fi;
   c->res_off.assign(L + 1, 0);
   c->pro_off.assign(L + 1, 0);
   for (int l = 0; l < L; ++l) {
-    c->res_off[l] = (int)res_ci.size();
+    c->res_off[l] = (int)res_cc.size();
     for (int i = 0; i < m->nres; ++i) {
       if (m->res_blk[i] % L != l) continue;
-      res_ci.push_back(h2d[m->res_ci[i]]);
+      res_cc.push_back(make_int2(h2d[m->res_ci[i]], hblk[m->res_ci[i]] / L));
       for (int q = 0; q < 8; ++q) {
         const int a = m->res_fi[(size_t)i * 8 + q];
-        res_fi.push_back(a < 0 ? -1 : h2d[a]);
+        res_son.push_back(a < 0 ? -1 : h2d[a]);
       }
     }
-    c->pro_off[l] = (int)pro_ci.size();
+    c->pro_off[l] = (int)pro_cc.size();
     for (int i = 0; i < m->npro; ++i) {
       if (m->pro_blk[i] % L != l) continue;
-      pro_ci.push_back(h2d[m->pro_ci[i]]);
+      pro_cc.push_back(make_int2(h2d[m->pro_ci[i]], hblk[m->pro_ci[i]] / L));
       for (int q = 0; q < 8; ++q) {
         const int a = m->pro_fi[(size_t)i * 8 + q];
         pro_fi.push_back(a < 0 ? -1 : h2d[a]);
       }
     }
   }
-  c->res_off[L] = (int)res_ci.size();
-  c->pro_off[L] = (int)pro_ci.size();
+  c->res_off[L] = (int)res_cc.size();
+  c->pro_off[L] = (int)pro_cc.size();
+  c->npro = (int)pro_cc.size();
+  std::vector<int4> res_fi(res_cc.size() * 2);
+  for (size_t i = 0; i < res_fi.size(); ++i)
+    res_fi[i] = make_int4(res_son[4 * i], res_son[4 * i + 1], res_son[4 * i + 2], res_son[4 * i + 3]);
+  // the six face neighbours of each prolonged cell (cneib TwoLevelOp.H:352)
+  std::vector<int> pro_nb((size_t)c->npro * 6);
+  for (int i = 0; i < c->npro; ++i)
+    for (int q = 0; q < 6; ++q) {
+      const int o = (q & 1) ? 1 : -1;
+      pro_nb[(size_t)q * c->npro + i] =
+          nbo(pro_cc[i].x, q / 2 == 0 ? o : 0, q / 2 == 1 ? o : 0, q / 2 == 2 ? o : 0);
+    }
   // ---- IB
   const int nib = m->nib;
   c->nib = nib;
@@ -1709,7 +1736,8 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
     for (int i = 0; i < N; ++i) ddm[i] = m->dist_dm[order[i]];
     UP(c->dist_dm, ddm);
   }
-  UP(c->res_ci, res_ci); UP(c->res_fi, res_fi); UP(c->pro_ci, pro_ci); UP(c->pro_fi, pro_fi);
+  UP(c->res_cc, res_cc); UP(c->res_fi, res_fi); UP(c->pro_cc, pro_cc); UP(c->pro_fi, pro_fi);
+  UP(c->pro_nb, pro_nb);
   UP(c->ib_cell, ib_cell); UP(c->ib_intp, ib_intp); UP(c->ib_body, ib_body); UP(c->ib_case, ib_case);
   UP(c->ib_coef, ib_coef); UP(c->ib_hgdis, ib_hgdis); UP(c->ib_attach, ib_att); UP(c->ib_nv, ib_nvh);
   UP(c->signdis, sd);
@@ -1729,7 +1757,6 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
   AL(c->err, 1);
   AL(c->err2, 1);
   AL(c->rpart, (size_t)std::max(c->ntiles, 1) * kRpart);
-  AL(c->resid, (size_t)nc * kRpart);
   AL(c->probe, (size_t)std::max(N, F) * 5);
 #undef UP
 #undef AL
@@ -2020,18 +2047,17 @@ ibg_status ibg_time_march(ibg_ctx *c, int32_t ts0, int32_t nsteps, int32_t use_g
   if (!c || !c->have_mesh) return IBG_ERR_STATE;
   if (nsteps < 0) return IBG_ERR_ARG;
   ibg_status st;
-  if ((st = reset_err(c))) return st;
+  // (with the law the moving-body masks change every step: the updates are
+  // counted on the device)
+  const int nupd = kUpdSlots * kUpdSlotStride;
+  hipLaunchKernelGGL(k_march_begin, dim3(c->mv.law ? grid(nupd, 256) : 1), dim3(256), 0, c->s, c->err, c->err2,
+                     c->mv.law ? c->mv.upd : (unsigned long long *)nullptr, nupd);
+  HIPCHK(hipGetLastError());
   c->have_motion = c->mv.law ? 1 : 0;
   const int P = c->cfg.temporal_refine ? (1 << (c->L - 1)) : 1;
   int64_t upd = 0;
   for (int k = 0; k < nsteps; ++k) upd += c->upd_per_lmin[lmin_of(c, ts0 + k)] * c->cfg.nstage;
   c->last_updates = upd;
-  if (c->mv.law) {
-    // the moving-body masks change every step: counted on the device
-    hipLaunchKernelGGL(k_fill_u64, dim3(grid(kUpdSlots * kUpdSlotStride, 256)), dim3(256), 0, c->s,
-                       c->mv.upd, kUpdSlots * kUpdSlotStride, 0ull);
-    HIPCHK(hipGetLastError());
-  }
   HIPCHK(hipEventRecord(c->ev0, c->s));
   int ts = ts0;
   const int end = ts0 + nsteps;
@@ -2046,34 +2072,27 @@ ibg_status ibg_time_march(ibg_ctx *c, int32_t ts0, int32_t nsteps, int32_t use_g
     ts += r.n;
   }
   HIPCHK(hipEventRecord(c->ev1, c->s));
-  HIPCHK(hipEventSynchronize(c->ev1));
+  static_assert(kUpdSlots == 64, "k_march_end sums one slot per lane");
+  hipLaunchKernelGGL(k_march_end, dim3(1), dim3(64), 0, c->s, (const unsigned long long *)c->err,
+                     c->mv.law ? (const unsigned long long *)c->mv.upd : (const unsigned long long *)nullptr,
+                     kUpdSlotStride, c->hword);
+  HIPCHK(hipGetLastError());
+  HIPCHK(hipStreamSynchronize(c->s));
   float ms = 0.f;
   HIPCHK(hipEventElapsedTime(&ms, c->ev0, c->ev1));
   c->last_total_ms = ms;
-  if (c->mv.law) {
-    std::vector<unsigned long long> u((size_t)kUpdSlots * kUpdSlotStride);
-    HIPCHK(hipMemcpyAsync(u.data(), c->mv.upd, sizeof(unsigned long long) * u.size(),
-                          hipMemcpyDeviceToHost, c->s));
-    HIPCHK(hipStreamSynchronize(c->s));
-    unsigned long long sum = 0;
-    for (int k = 0; k < kUpdSlots; ++k) sum += u[(size_t)k * kUpdSlotStride];
-    c->last_updates = (int64_t)sum;
-  }
-  int64_t cell;
-  int32_t code;
-  if ((st = read_err(c, &cell, &code))) return st;
-  if (code) return (ibg_status)code;
+  if (c->mv.law) c->last_updates = (int64_t)c->hword[1];
+  if (c->hword[0] != ~0ull) return (ibg_status)(int32_t)(c->hword[0] & 0xffff);
   return IBG_OK;
 }
 
 ibg_status ibg_residual(ibg_ctx *c, double *linf, double *l2) {
   if (!c || !c->have_mesh) return IBG_ERR_STATE;
   hipLaunchKernelGGL(k_resid_final, dim3(c->ncases), dim3(256), 0, c->s, c->last_ntiles, c->L,
-                     c->case_tiles, c->rpart, c->resid, c->ncases);
+                     c->case_tiles, c->rpart, c->hres, c->ncases);
   HIPCHK(hipGetLastError());
-  std::vector<double> h((size_t)c->ncases * kRpart);
-  HIPCHK(hipMemcpyAsync(h.data(), c->resid, h.size() * 8, hipMemcpyDeviceToHost, c->s));
   HIPCHK(hipStreamSynchronize(c->s));
+  const double *h = c->hres;
   for (int cs = 0; cs < c->ncases; ++cs)
     for (int k = 0; k < 5; ++k) {
       if (linf) linf[cs * 5 + k] = h[cs * kRpart + k];
@@ -2086,11 +2105,10 @@ ibg_status ibg_residual_nut(ibg_ctx *c, double *linf, double *l2) {
   if (!c || !c->have_mesh) return IBG_ERR_STATE;
   if (!c->turb) return IBG_ERR_STATE;
   hipLaunchKernelGGL(k_resid_final, dim3(c->ncases), dim3(256), 0, c->s, c->last_ntiles, c->L,
-                     c->case_tiles, c->rpart, c->resid, c->ncases);
+                     c->case_tiles, c->rpart, c->hres, c->ncases);
   HIPCHK(hipGetLastError());
-  std::vector<double> h((size_t)c->ncases * kRpart);
-  HIPCHK(hipMemcpyAsync(h.data(), c->resid, h.size() * 8, hipMemcpyDeviceToHost, c->s));
   HIPCHK(hipStreamSynchronize(c->s));
+  const double *h = c->hres;
   for (int cs = 0; cs < c->ncases; ++cs) {
     if (linf) linf[cs] = h[cs * kRpart + 10];
     if (l2) l2[cs] = h[cs * kRpart + 11];
@@ -2123,14 +2141,14 @@ ibg_status ibg_forces(ibg_ctx *c, const ibg_body_motion *mo, double *out) {
   if (c->D == 2)
     hipLaunchKernelGGL((k_forces<2>), dim3(c->ncases), dim3(256), 0, c->s, c->npatch, c->pat_case,
                        c->pat_intp, c->pat_coef, c->pat_hgdis, c->pat_nv, c->pat_pc, c->pat_area,
-                       c->case_center, mp, hm, c->w64<2>(), c->phys, (int)c->turb, c->resid);
+                       c->case_center, mp, hm, c->w64<2>(), c->phys, (int)c->turb, c->hres);
   else
     hipLaunchKernelGGL((k_forces<3>), dim3(c->ncases), dim3(256), 0, c->s, c->npatch, c->pat_case,
                        c->pat_intp, c->pat_coef, c->pat_hgdis, c->pat_nv, c->pat_pc, c->pat_area,
-                       c->case_center, mp, hm, c->w64<3>(), c->phys, (int)c->turb, c->resid);
+                       c->case_center, mp, hm, c->w64<3>(), c->phys, (int)c->turb, c->hres);
   HIPCHK(hipGetLastError());
-  HIPCHK(hipMemcpyAsync(out, c->resid, sizeof(double) * 6 * c->ncases, hipMemcpyDeviceToHost, c->s));
   HIPCHK(hipStreamSynchronize(c->s));
+  std::memcpy(out, c->hres, sizeof(double) * 6 * c->ncases);
   return IBG_OK;
 }
 

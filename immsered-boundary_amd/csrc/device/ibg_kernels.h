@@ -1325,11 +1325,13 @@ template <int D>
 __global__ void k_bc(int n, const int4 *dmg, const DmgWall *wall, StateOut<D> o,
                      const DevPhys *phys) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || halted(o.err)) return;
+  if (i >= n) return;
+  const bool stop = halted(o.err);   // in flight with the entry
   const int4 e = dmg[i];
   const int g = e.x, ty = e.z;
   const DevPhys &P = phys[e.w];
   const Prim<double, D> q = pload<double, D>(o.m, e.y);
+  if (stop) return;
   if (ty == -81) {
     // the wall of the TURBULENCE build (BCValues.H:89-125); nothing in the
     // laminar build, where the branch does not exist
@@ -1383,96 +1385,115 @@ __global__ void k_bc(int n, const int4 *dmg, const DmgWall *wall, StateOut<D> o,
   }
 }
 
+// The ghost fills below run on a few thousand entries: a chain of memory
+// latencies each, so every load that does not depend on another is issued at
+// once (the error word with the list entry, the case index with the cell's)
+// and the word is tested before the writes.
+
 // PairRestriction[_2d] TwoLevelOp.H:217-231 with AverageCell[_2d] :45-87
-// (the SA variant :129-179 averages the working variable without weights)
+// (the SA variant :129-179 averages the working variable without weights).
+// cc: (coarse cell, case).
 template <int D>
-__global__ void k_restrict(int n, const int *ci, const int *fi, StateOut<D> o, int twod,
-                           const DevPhys *phys, const int *cellcase) {
+__global__ void k_restrict(int n, const int2 *cc, const int4 *fi, StateOut<D> o, int twod,
+                           const DevPhys *phys) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || halted(o.err)) return;
-  const int c = ci[i];
-  const DevPhys &P = phys[cellcase[c]];
+  if (i >= n) return;
+  const bool stop = halted(o.err);
+  const int2 c = cc[i];
+  const int4 f0 = fi[2 * (size_t)i], f1 = fi[2 * (size_t)i + 1];
+  const int son[8] = {f0.x, f0.y, f0.z, f0.w, f1.x, f1.y, f1.z, f1.w};
+  const DevPhys &P = phys[c.y];
   double r = 0, ru = 0, rv = 0, rw = 0, re = 0, nu = 0;
-  for (int q = 0; q < 8; ++q) {
-    if (twod && (q & 1)) continue;
-    const int a = fi[(size_t)i * 8 + q];
-    const Prim<double, D> s = pload<double, D>(o.m, a);
+  auto add = [&](const Prim<double, D> &s, double nv) {
     const double T = s.p / (s.r * P.Rg);
-    const double e = P.Cv * T + ((D == 3) ? 0.5 * (s.u * s.u + s.v * s.v + s.w * s.w) : 0.5 * (s.u * s.u + s.v * s.v));
+    const double q2 = (D == 3) ? s.u * s.u + s.v * s.v + s.w * s.w : s.u * s.u + s.v * s.v;
+    const double e = fma(0.5, q2, P.Cv * T);
     r += s.r;
     ru += s.u * s.r;
     rv += s.v * s.r;
     rw += s.w * s.r;
     re += e * s.r;
-    if (o.nm) nu += o.nm[a];
-  }
-  const double u = ru / r, v = rv / r, w = rw / r, e = re / r;
+    nu += nv;
+  };
+  // the sons of the low z half first, all in flight, then (a level refined
+  // in z too) the others: sums in son order either way
+  Prim<double, D> s[8];
+  double nv[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    if (!(twod && (q & 1))) {
+      s[q] = pload<double, D>(o.m, son[q]);
+      nv[q] = o.nm ? o.nm[son[q]] : 0.0;
+    }
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    if (!(twod && (q & 1))) add(s[q], nv[q]);
+  if (stop) return;
+  const double u = ru / r, v = rv / r, w = (D == 3) ? rw / r : 0.0, e = re / r;
   const double rho = r * (twod ? 0.25 : 0.125);
   const double ke = (D == 3) ? 0.5 * (u * u + v * v + w * w) : 0.5 * (u * u + v * v);
   const double p = (e - ke) * (P.gama - 1.0) * rho;
-  put_all<D>(o, c, rho, u, v, w, p);
-  if (o.nm) put_nu<D>(o, c, nu * (twod ? 0.25 : 0.125));
+  put_all<D>(o, c.x, rho, u, v, w, p);
+  if (o.nm) put_nu<D>(o, c.x, nu * (twod ? 0.25 : 0.125));
 }
 
 // PairProlongation[_2d] TwoLevelOp.H:183-215: central gradients of the
 // conserved variables over the 6 face neighbours (cneib, :352-358), sons at
 // +-1/4 (fincrem); the SA variant (:91-127) does the same for the working
-// variable.
+// variable.  One thread per son; cc: (coarse cell, case), nb[6][stride]: the
+// cell's neighbours x low, x high, y, z, both listed per pair.  For the 4.4K
+// pairs of a level of the moving section 10.5 -> 6.5 us (one thread per
+// pair, the neighbours from the cell's row of 27).
 template <int D>
-__global__ void k_prolong(int n, const int *ci, const int *fi, const int *nb27, StateOut<D> o,
-                          int twod, const DevPhys *phys, const int *cellcase) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || halted(o.err)) return;
-  const int c = ci[i];
-  const DevPhys &P = phys[cellcase[c]];
-  const int *nb = nb27 + (size_t)c * 27;
-  auto cons = [&](int a, double *U) {
-    const Prim<double, D> q = pload<double, D>(o.m, a);
+__global__ void k_prolong(int n, const int2 *cc, const int *fi, const int *nb, int stride,
+                          StateOut<D> o, int twod, const DevPhys *phys) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  const int ns = twod ? 4 : 8;
+  const int i = t / ns, sn = t - i * ns;
+  if (i >= n) return;
+  const bool stop = halted(o.err);
+  const int2 c = cc[i];
+  const int si = twod ? sn >> 1 : sn >> 2, sj = twod ? sn & 1 : (sn >> 1) & 1, sk = twod ? 0 : sn & 1;
+  const int f = fi[(size_t)i * 8 + si * 4 + sj * 2 + sk];
+  const int ax0 = nb[i], ax1 = nb[stride + i], ay0 = nb[2 * stride + i], ay1 = nb[3 * stride + i];
+  const int az0 = twod ? 0 : nb[4 * stride + i], az1 = twod ? 0 : nb[5 * stride + i];
+  const DevPhys &P = phys[c.y];
+  auto cons = [&](const Prim<double, D> &q, double *U) {
     const double T = q.p / (q.r * P.Rg);
-    const double e = P.Cv * T + ((D == 3) ? 0.5 * (q.u * q.u + q.v * q.v + q.w * q.w) : 0.5 * (q.u * q.u + q.v * q.v));
+    const double q2 = (D == 3) ? q.u * q.u + q.v * q.v + q.w * q.w : q.u * q.u + q.v * q.v;
+    const double e = fma(P.Cv, T, 0.5 * q2);
     U[0] = q.r; U[1] = q.r * q.u; U[2] = q.r * q.v; U[3] = q.r * q.w; U[4] = q.r * e;
   };
-  const int ax0 = nb[0 * 9 + 1 * 3 + 1], ax1 = nb[2 * 9 + 1 * 3 + 1];
-  const int ay0 = nb[1 * 9 + 0 * 3 + 1], ay1 = nb[1 * 9 + 2 * 3 + 1];
-  const int az0 = nb[1 * 9 + 1 * 3 + 0], az1 = nb[1 * 9 + 1 * 3 + 2];
-  double Uc[5], Ux0[5], Ux1[5], Uy0[5], Uy1[5], Uz0[5], Uz1[5];
-  cons(c, Uc);
-  cons(ax0, Ux0); cons(ax1, Ux1);
-  cons(ay0, Uy0); cons(ay1, Uy1);
-  cons(az0, Uz0); cons(az1, Uz1);
-  double gx[5], gy[5], gz[5];
-  for (int t = 0; t < 5; ++t) {
-    gx[t] = (Ux1[t] - Ux0[t]) * 0.5;
-    gy[t] = (Uy1[t] - Uy0[t]) * 0.5;
-    gz[t] = (Uz1[t] - Uz0[t]) * 0.5;
-  }
+  const Prim<double, D> qc = pload<double, D>(o.m, c.x);
+  const Prim<double, D> qx0 = pload<double, D>(o.m, ax0), qx1 = pload<double, D>(o.m, ax1);
+  const Prim<double, D> qy0 = pload<double, D>(o.m, ay0), qy1 = pload<double, D>(o.m, ay1);
+  Prim<double, D> qz0 = qc, qz1 = qc;
+  if (!twod) { qz0 = pload<double, D>(o.m, az0); qz1 = pload<double, D>(o.m, az1); }
   double nc = 0, ngx = 0, ngy = 0, ngz = 0;
   if (o.nm) {
-    nc = o.nm[c];
+    nc = o.nm[c.x];
     ngx = (o.nm[ax1] - o.nm[ax0]) * 0.5;
     ngy = (o.nm[ay1] - o.nm[ay0]) * 0.5;
-    ngz = (o.nm[az1] - o.nm[az0]) * 0.5;
+    if (!twod) ngz = (o.nm[az1] - o.nm[az0]) * 0.5;
   }
-  const double fincrem[2] = {-0.25, 0.25};
-  for (int si = 0; si < 2; ++si)
-    for (int sj = 0; sj < 2; ++sj)
-      for (int sk = 0; sk < (twod ? 1 : 2); ++sk) {
-        const int f = fi[(size_t)i * 8 + si * 4 + sj * 2 + sk];
-        double U[5];
-        for (int t = 0; t < 5; ++t) {
-          if (twod) U[t] = Uc[t] + fincrem[si] * gx[t] + fincrem[sj] * gy[t];
-          else U[t] = Uc[t] + fincrem[si] * gx[t] + fincrem[sj] * gy[t] + fincrem[sk] * gz[t];
-        }
-        const double r = U[0], u = U[1] / U[0], v = U[2] / U[0], w = U[3] / U[0], e = U[4] / U[0];
-        const double ke = (D == 3) ? 0.5 * (u * u + v * v + w * w) : 0.5 * (u * u + v * v);
-        const double p = (e - ke) * (P.gama - 1.0) * r;
-        put_all<D>(o, f, r, u, v, w, p);
-        if (o.nm) {
-          const double nf = twod ? nc + fincrem[si] * ngx + fincrem[sj] * ngy
-                                 : nc + fincrem[si] * ngx + fincrem[sj] * ngy + fincrem[sk] * ngz;
-          put_nu<D>(o, f, nf);
-        }
-      }
+  double Uc[5], Ux0[5], Ux1[5], Uy0[5], Uy1[5], Uz0[5], Uz1[5];
+  cons(qc, Uc);
+  cons(qx0, Ux0); cons(qx1, Ux1);
+  cons(qy0, Uy0); cons(qy1, Uy1);
+  if (!twod) { cons(qz0, Uz0); cons(qz1, Uz1); }
+  const double ix = si ? 0.25 : -0.25, iy = sj ? 0.25 : -0.25, iz = sk ? 0.25 : -0.25;
+  double U[5];
+  for (int t2 = 0; t2 < 5; ++t2) {
+    const double gx = (Ux1[t2] - Ux0[t2]) * 0.5, gy = (Uy1[t2] - Uy0[t2]) * 0.5;
+    if (twod) U[t2] = Uc[t2] + ix * gx + iy * gy;
+    else U[t2] = Uc[t2] + ix * gx + iy * gy + iz * ((Uz1[t2] - Uz0[t2]) * 0.5);
+  }
+  if (stop) return;
+  const double r = U[0], u = U[1] / r, v = U[2] / r, w = (D == 3) ? U[3] / r : 0.0, e = U[4] / r;
+  const double ke = (D == 3) ? 0.5 * (u * u + v * v + w * w) : 0.5 * (u * u + v * v);
+  const double p = (e - ke) * (P.gama - 1.0) * r;
+  put_all<D>(o, f, r, u, v, w, p);
+  if (o.nm) put_nu<D>(o, f, twod ? nc + ix * ngx + iy * ngy : nc + ix * ngx + iy * ngy + iz * ngz);
 }
 
 // Body::IBConditions_Image Body.cpp:1366-1496: image state from the
@@ -1492,14 +1513,31 @@ __global__ void k_ib(int n, const int *ndev, const int *cell, const int *intp, c
   // n: list length, or its capacity when the length lives on the device
   // (moving bodies rebuild the list every step)
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= n || (ndev && i >= ndev[0]) || halted(err)) return;
-  const DevPhys &P = phys[ibcase[i]];
+  if (i >= n) return;
+  // the entry (its arrays hold n), the list length and the error word at once
+  const int nlist = ndev ? ndev[0] : n;
+  const bool stop = halted(err);
+  const int4 a0 = *reinterpret_cast<const int4 *>(intp + (size_t)i * 8);
+  const int4 a1 = *reinterpret_cast<const int4 *>(intp + (size_t)i * 8 + 4);
+  const int cs = ibcase[i], c = cell[i];
+  const double hg = hgdis[i];
+  double cf[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q) cf[q] = coef[(size_t)i * 8 + q];
+  if (i >= nlist || stop) return;
+  const double sd = signdis[c];
+  const DevPhys &P = phys[cs];
+  const int at8[8] = {a0.x, a0.y, a0.z, a0.w, a1.x, a1.y, a1.z, a1.w};
   double T = 0, p = 0, u = 0, v = 0, w = 0;
+  Prim<double, D> img[8];
+#pragma unroll
+  for (int q = 0; q < 8; ++q)
+    if (at8[q] >= 0) img[q] = pload<double, D>(o.m, at8[q]);
+#pragma unroll
   for (int q = 0; q < 8; ++q) {
-    const int a = intp[(size_t)i * 8 + q];
-    if (a < 0) continue;
-    const double cq = coef[(size_t)i * 8 + q];
-    const Prim<double, D> s = pload<double, D>(o.m, a);
+    if (at8[q] < 0) continue;
+    const double cq = cf[q];
+    const Prim<double, D> &s = img[q];
     T += cq * (s.p / (s.r * P.Rg));
     p += cq * s.p;
     u += cq * s.u;
@@ -1515,15 +1553,13 @@ __global__ void k_ib(int n, const int *ndev, const int *cell, const int *intp, c
     pv[1] = M.tra[1] + (M.rot[2] * r1[0] - M.rot[0] * r1[2]);
     pv[2] = M.tra[2] + (M.rot[0] * r1[1] - M.rot[1] * r1[0]);
   }
-  const int c = cell[i];
-  const double sd = signdis[c];
   if (T < 0.0) report_error(err, c, 1050);
   if (!o.nm) {
     double ou, ov, ow;
     if (sd < 0.0) {
       ou = 2.0 * pv[0] - u; ov = 2.0 * pv[1] - v; ow = 2.0 * pv[2] - w;
     } else {
-      const double rt = sd + hgdis[i];
+      const double rt = sd + hg;
       const double r0 = sd / rt;
       ou = pv[0] + (u - pv[0]) * r0;
       ov = pv[1] + (v - pv[1]) * r0;
@@ -1540,7 +1576,7 @@ __global__ void k_ib(int n, const int *ndev, const int *cell, const int *intp, c
   // ImageViseddy
   const double *nm = nvec + (size_t)i * 3;
   const double rho_hg = p / (P.Rg * T);
-  const double rt0 = hgdis[i] + sd;
+  const double rt0 = hg + sd;
   const double ib_rdis = sd / rt0;
   const double hvn = u * nm[0] + v * nm[1] + w * nm[2];
   const double hn[3] = {hvn * nm[0], hvn * nm[1], hvn * nm[2]};
@@ -1609,18 +1645,19 @@ __global__ void k_dt_final(int L, const int *ct, const double *cflpart, double *
                            const DevPhys *phys, int ncases, const unsigned long long *err) {
   const int cs = blockIdx.x;
   if (cs >= ncases) return;
-  __shared__ double red[256];
+  __shared__ double red[4];
   if (wg_halted(err)) return;
   double m = 10000.0;
   for (int l = 0; l < L; ++l) {
     const int a = ct[(cs * L + l) * 2], b = ct[(cs * L + l) * 2 + 1];
     for (int t = a + (int)threadIdx.x; t < b; t += blockDim.x) m = fmin(m, cflpart[t]);
   }
-  red[threadIdx.x] = m;
+  for (int off = 32; off > 0; off >>= 1) m = fmin(m, __shfl_xor(m, off, 64));
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = m;
   __syncthreads();
   if (threadIdx.x == 0) {
     double v = red[0];
-    for (int k = 1; k < (int)blockDim.x; ++k) v = fmin(v, red[k]);
+    for (int k = 1; k < (int)((blockDim.x + 63) >> 6); ++k) v = fmin(v, red[k]);
     const double d = dt[cs] * phys[cs].dt_ratio;
     dt[cs] = (v < d) ? v : d;
   }
@@ -1642,6 +1679,22 @@ template <typename R>
 __global__ void k_fill_nu_from_master(int n, const double *src, R *dst) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i < n) dst[i] = (R)src[i];
+}
+
+// The start of a march: both error words clear, the update counters zero.
+__global__ void k_march_begin(unsigned long long *err, unsigned long long *err2,
+                              unsigned long long *upd, int n) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (upd && i < n) upd[i] = 0ull;
+  if (i == 0) { *err = ~0ull; *err2 = ~0ull; }
+}
+// Its end: the error word and the sum of the update counters (one wave, 64
+// slots of the given stride) into pinned host memory.
+__global__ void k_march_end(const unsigned long long *err, const unsigned long long *upd, int stride,
+                            unsigned long long *out) {
+  unsigned long long s = upd ? upd[(size_t)threadIdx.x * stride] : 0ull;
+  for (int off = 32; off > 0; off >>= 1) s += __shfl_xor(s, off, 64);
+  if (threadIdx.x == 0) { out[0] = *err; out[1] = s; }
 }
 
 __global__ void k_fill_u64(unsigned long long *p, int n, unsigned long long v) {
@@ -1730,11 +1783,17 @@ __global__ void k_forces(int npatch, const int *pcase, const int *intp, const do
   }
   for (int k = 0; k < 12; ++k) acc[threadIdx.x][k] = s[k];
   __syncthreads();
+  // twelve threads, one sum each in thread order (one thread for all of them
+  // took 50 us of LDS latency)
+  __shared__ double t[12];
+  if (threadIdx.x < 12) {
+    double x = 0.0;
+#pragma unroll 16
+    for (int j = 0; j < 256; ++j) x += acc[j][threadIdx.x];
+    t[threadIdx.x] = x;
+  }
+  __syncthreads();
   if (threadIdx.x == 0) {
-    double t[12];
-    for (int k = 0; k < 12; ++k) t[k] = 0.0;
-    for (int j = 0; j < (int)blockDim.x; ++j)
-      for (int k = 0; k < 12; ++k) t[k] += acc[j][k];
     for (int k = 0; k < 3; ++k) {
       // the SA build scales the wall shear by p_ref*area_ref (Body.cpp:547-553)
       const double sr = turb ? P.p_ref_area : P.shear_ref_area;
@@ -1767,16 +1826,16 @@ __global__ void k_resid_final(int ntiles, int L, const int *ct, const double *rp
   }
   for (int k = 0; k < 6; ++k) { red[k][threadIdx.x] = m[k]; red[6 + k][threadIdx.x] = q[k]; }
   __syncthreads();
-  if (threadIdx.x == 0) {
-    for (int k = 0; k < 6; ++k) {
-      double mm = 0.0, qq = 0.0;
-      for (int w = 0; w < (int)blockDim.x; ++w) { mm = fmax(mm, red[k][w]); qq += red[6 + k][w]; }
-      m[k] = mm;
-      q[k] = qq;
-    }
-    for (int k = 0; k < 5; ++k) { out[cs * kRpart + k] = m[k]; out[cs * kRpart + 5 + k] = sqrt(q[k]); }
-    out[cs * kRpart + 10] = m[5];
-    out[cs * kRpart + 11] = sqrt(q[5]);
+  // twelve threads, one entry each in thread order (one thread for all of
+  // them took 25 us of LDS latency)
+  const int j = threadIdx.x;
+  if (j < kRpart) {
+    double x = 0.0;
+    const bool sum = j >= 6;
+#pragma unroll 16
+    for (int w = 0; w < 256; ++w) x = sum ? x + red[j][w] : fmax(x, red[j][w]);
+    const int k = sum ? j - 6 : j;
+    out[cs * kRpart + (k < 5 ? (sum ? 5 + k : k) : (sum ? 11 : 10))] = sum ? sqrt(x) : x;
   }
 }
 
