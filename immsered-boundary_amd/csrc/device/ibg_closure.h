@@ -78,11 +78,11 @@ __global__ void __launch_bounds__(kTile) k_closure_sample(const TileInfo *tiles,
     const double T = me.p / (me.r * P.Rg);
     const double mu0 = sqrt(T * T * T) * ((1.0 + P.SoT) / (T + P.SoT));
     const VelGrad<double> g = cell_grad<D>(W, nb27, c, bi);
-    const double olen = sa_olen<double>(g);
+    const double olen = sa_olen<double>(g, sa_phys(P));
     double scale;
     keep = sa_features<double>(me.u, me.v, me.w, me.r, me.p, mu0, nu[c], signdis[c], g, olen,
                                P.Re, P.init[4], x, scale);
-    if (keep) z = sa_pointwise<double>(nu[c], mu0, me.r, signdis[c], olen, P.Re) / scale;
+    if (keep) z = sa_pointwise<double>(nu[c], mu0, me.r, signdis[c], olen, sa_phys(P)) / scale;
   }
   // rank of the kept cell within the tile: wave prefix + earlier waves
   const unsigned long long bal = __ballot(keep);

@@ -105,6 +105,18 @@ struct BlkInfo {
   int case_id, level, finest, pad;
 };
 
+// What the FP32 kernels need of a (case, level), in FP32: the constants of
+// BlkInfo and DevPhys rounded, and their reciprocals and root as the hardware
+// forms them (k_flow32 fills the table on the device).  Formed per wave they
+// are ~25 conversions, reciprocals and roots, the latter at a quarter of the
+// vector rate.
+struct Flow32 {
+  float area[3], invh[3];
+  float gama, Rg, Cv, Ma, gm1, ig1, iRg, cpR;   // gm1 = gama - 1 in FP32, ig1 and iRg reciprocals
+  float SoT, SoT1, Re, iRe, qk, iqkt, sqrt2;    // SoT1 = 1 + SoT
+  float pad;
+};
+
 // halo0: first entry of a block tile's halo list, -1 for a general tile
 // (whose faces are [face0, face0 + nface) of the tile face lists)
 struct TileInfo {

@@ -113,6 +113,7 @@ struct ibg_ctx {
   int8_t *face_dir = nullptr;
   int16_t *face_blk = nullptr;
   BlkInfo *blk = nullptr;
+  Flow32 *flow = nullptr;       // [blocks] the FP32 constants of each
   DevPhys *phys = nullptr;
   int4 *dmg = nullptr;
   DmgWall *dmgw = nullptr;      // wall ghosts (BC -81), parallel to dmg; null without walls
@@ -434,7 +435,7 @@ ViscArgs<R, D> visc_args(ibg_ctx *c) {
   ViscArgs<R, D> a;
   a.tiles = c->tiles; a.tst = c->tst; a.tvs = c->tvs; a.tdir = c->tdir; a.slots = c->slots;
   a.halo = c->halo;
-  a.blk = c->blk; a.phys = c->phys;
+  a.blk = c->blk; a.phys = c->phys; a.flow = c->flow;
   a.W = c->sbuf<R, D>(0);
   a.Rv = c->rv<R, D>();
   a.nu = c->nubuf<R>(0);
@@ -455,7 +456,7 @@ ibg_status launch_stage(ibg_ctx *c, int ntile, int ncell, int subt, bool last, d
   stage_bufs(c->cfg.nstage, subt, &bin, &bout);
   StageArgs<R, D> a;
   a.tiles = c->tiles; a.tst = c->tst; a.tdir = c->tdir; a.slots = c->slots; a.halo = c->halo;
-  a.flags = c->flags; a.blk = c->blk; a.phys = c->phys; a.dt = c->dt;
+  a.flags = c->flags; a.blk = c->blk; a.phys = c->phys; a.flow = c->flow; a.dt = c->dt;
   a.Win = c->sbuf<R, D>(bin);
   a.Wout = c->sbuf<R, D>(bout);
   a.W64 = c->w64<D>();
@@ -1758,6 +1759,7 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
   AL(c->err2, 1);
   AL(c->rpart, (size_t)std::max(c->ntiles, 1) * kRpart);
   AL(c->probe, (size_t)std::max(N, F) * 5);
+  AL(c->flow, (size_t)nblk);
 #undef UP
 #undef AL
   // cell-stage update count per step, for each lmin (UPDATE cells marched)
@@ -1773,6 +1775,9 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
     }
   }
   HIPCHK(hipDeviceSynchronize());
+  hipLaunchKernelGGL(k_flow32, dim3(grid(nblk, 64)), dim3(64), 0, c->s, nblk, (const BlkInfo *)c->blk,
+                     (const DevPhys *)c->phys, c->flow);
+  HIPCHK(hipGetLastError());
   if ((st = reset_err(c))) return st;
   HIPCHK(hipStreamSynchronize(c->s));
   c->have_mesh = true;
@@ -2543,7 +2548,7 @@ void launch_probes(ibg_ctx *c, bool visc) {
   if (F <= 0) return;
   if (visc)
     hipLaunchKernelGGL((k_visc_probe<R, D>), dim3(grid(F, 256)), dim3(256), 0, c->s, F, c->face_st,
-                       c->face_vst, c->face_dir, c->face_blk, c->wstencil<R, D>(), c->blk, c->phys,
+                       c->face_vst, c->face_dir, c->face_blk, c->wstencil<R, D>(), c->blk, c->phys, c->flow,
                        c->turb ? c->nubuf<R>(0) : (const R *)nullptr, c->probe, c->mprobe);
   else
     hipLaunchKernelGGL((k_face_probe<R, D>), dim3(grid(F, 256)), dim3(256), 0, c->s, F, c->face_st,

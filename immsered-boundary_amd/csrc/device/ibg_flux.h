@@ -57,15 +57,25 @@ template <typename R>
 struct PhysR {
   R gama, Rg, Cv, Ma;
   R gm1, ig1;    // gama - 1 and its reciprocal
+  R iRg;         // 1 / Rg (FP32 only)
   R cpR;         // Cv / Rg + 1: enthalpy h = cpR p / roe + |u|^2 / 2
 };
 template <typename R, class Q>
 __device__ __forceinline__ PhysR<R> phys_r(const Q &P) {
   PhysR<R> ph;
   ph.gama = (R)P.gama; ph.Rg = (R)P.Rg; ph.Cv = (R)P.Cv; ph.Ma = (R)P.Ma;
-  ph.gm1 = (R)(P.gama - 1.0); ph.ig1 = (R)P.ig1;
   ph.cpR = (R)P.cpR;
+  if constexpr (sizeof(R) == 4) {
+    ph.gm1 = ph.gama - 1.0f; ph.ig1 = f_rcp(ph.gm1); ph.iRg = f_rcp(ph.Rg);
+  } else {
+    ph.gm1 = P.gama - 1.0; ph.ig1 = P.ig1; ph.iRg = 0.0;
+  }
   return ph;
+}
+// the same from the table of the FP32 constants
+template <class Q>
+__device__ __forceinline__ PhysR<float> phys_r32(const Q &F) {
+  return PhysR<float>{F.gama, F.Rg, F.Cv, F.Ma, F.gm1, F.ig1, F.iRg, F.cpR};
 }
 
 template <typename R, int D>
@@ -237,7 +247,7 @@ __device__ __forceinline__ void from_face(double *f, int dir) {
 
 // Flux of an axis-aligned face.  Output: D == 2: (mass, x-mom, y-mom,
 // energy); D == 3: (mass, x, y, z momentum, energy).
-template <int D, int DIR = -1>
+template <int D, int DIR = -1, bool FLAT = false>
 __device__ __forceinline__ void roe_flux(const Prim<double, D> &t0, const Prim<double, D> &t1,
                                          const Prim<double, D> &t2, const Prim<double, D> &t3,
                                          int dir, double area, const PhysR<double> &ph, int lim,
@@ -293,7 +303,8 @@ __device__ __forceinline__ float fast_slope(float q, float a, float b, int lim) 
 // where it is dir.  The fused operations are written out, so that both forms
 // round alike: the terms that a known direction drops are exact zeros and
 // products with one.
-template <int D, int DIR = -1>
+// FLAT: the limiter without branches.
+template <int D, int DIR = -1, bool FLAT = (D == 2 && DIR >= 0)>
 __device__ __forceinline__ void roe_flux(const Prim<float, D> &t0, const Prim<float, D> &t1,
                                          const Prim<float, D> &t2, const Prim<float, D> &t3,
                                          int dir, float area, const PhysR<float> &ph, int lim,
@@ -316,7 +327,7 @@ __device__ __forceinline__ void roe_flux(const Prim<float, D> &t0, const Prim<fl
       r = flat_slope<false, A>(q2, d2, d1);
     });
   };
-  if constexpr (D == 2 && DIR >= 0) {
+  if constexpr (FLAT) {
     if (lim == 1) flat(std::true_type());   // lim is uniform: one branch a face
     else flat(std::false_type());
   } else {
@@ -327,7 +338,7 @@ __device__ __forceinline__ void roe_flux(const Prim<float, D> &t0, const Prim<fl
     });
   }
   const float ilr = f_rcp(lr), irr = f_rcp(rr);
-  const float iRg = f_rcp(Rg);
+  const float iRg = ph.iRg;
   const float plr = lp * ilr, prr = rp * irr;
   const float rT = prr * iRg;
   float lq = fmaf(lu, lu, lvv * lvv), rq = fmaf(ru, ru, rvv * rvv);
@@ -368,7 +379,7 @@ __device__ __forceinline__ void roe_flux(const Prim<float, D> &t0, const Prim<fl
   const float a_h = fmaf(h_right, r2lroe, h_left) * r2l0;
   float q2 = fmaf(a_u, a_u, a_v * a_v);
   if (D == 3) q2 = fmaf(a_w, a_w, q2);
-  const float csquare = (gama - 1.0f) * fmaf(-0.5f, q2, a_h);
+  const float csquare = ph.gm1 * fmaf(-0.5f, q2, a_h);
   const float a_c = f_sqrt(csquare);
   const float a_ubar = pick(a_u, a_v, a_w);
   const float icsq = f_rcp(csquare);
@@ -402,7 +413,7 @@ __device__ __forceinline__ void roe_flux(const Prim<float, D> &t0, const Prim<fl
     else t = fmaf(vel, al3, k * al4);
     return (DIR >= 0 && DIR == d) ? t : fmaf(faa, j, t);
   };
-  const float ig1 = f_rcp(gama - 1.0f);
+  const float ig1 = ph.ig1;
   flux[0] = fmaf(p0, ha, -al3);
   flux[1] = fmaf(p1, ha, -upw(0, k0, a_u, j0));
   flux[2] = fmaf(p2, ha, -upw(1, k1, a_v, j1));
@@ -455,11 +466,32 @@ template <> __device__ __forceinline__ double v_sqrt<double>(double a) {
   const double g = n_sqrt(a);
   return a == 0.0 ? a : g;
 }
+// The constants of the SA source: S/T_ref of Sutherland's law and 1 + it, the
+// Reynolds number, its reciprocal (FP32) and sqrt(2).
+template <typename R>
+struct SaPhys {
+  R SoT, SoT1, Re, iRe, sqrt2;
+};
+template <class Q>
+__device__ __forceinline__ SaPhys<double> sa_phys(const Q &P) {
+  return SaPhys<double>{P.SoT, 1.0 + P.SoT, P.Re, P.iRe, 1.4142135623730951};
+}
+template <class Q>
+__device__ __forceinline__ SaPhys<float> sa_phys32(const Q &F) {
+  return SaPhys<float>{F.SoT, F.SoT1, F.Re, F.iRe, F.sqrt2};
+}
+__device__ __forceinline__ float over_re(float x, const SaPhys<float> &sp) { return x * sp.iRe; }
+__device__ __forceinline__ double over_re(double x, const SaPhys<double> &sp) { return n_div(x, sp.Re); }
+
 // r = nu / (S~ kappa^2 d^2 Re) of the SA destruction term: S~ vanishes in a
 // uniform stream, where nu / 0 = inf is the reference's value (capped at 10
 // by the caller) and 0 / 0 its NaN, so FP64 divides in full here
-__device__ __forceinline__ float sa_r(float nu, float sd2, float Re) { return v_div(v_div(nu, sd2), Re); }
-__device__ __forceinline__ double sa_r(double nu, double sd2, double Re) { return nu / (sd2 * Re); }
+__device__ __forceinline__ float sa_r(float nu, float sd2, const SaPhys<float> &sp) {
+  return v_div(nu, sd2) * sp.iRe;
+}
+__device__ __forceinline__ double sa_r(double nu, double sd2, const SaPhys<double> &sp) {
+  return nu / (sd2 * sp.Re);
+}
 
 // Viseddy2mut (Turbulence.cpp:23-30): mu_t = roe fv1 nu, X = nu/(mu/roe)
 // clamped at 0, fv1 = X^3/(X^3 + cv1^3).
@@ -772,7 +804,7 @@ template <typename R, int D>
 __device__ __forceinline__ R sa_source(R u, R v, R w, R T, R roe, R nu, R sd, const R *nl,
                                        const R *nr, const R *ul, const R *ur, const R *vl,
                                        const R *vr, const R *wl, const R *wr, R ih0, R ih1, R ih2,
-                                       R SoT, R Re, R mutf) {
+                                       const SaPhys<R> &sp, R mutf) {
   const R h = R(0.5);
   const R dvisx = ((nr[0] - nl[0]) * h) * ih0;
   const R dvisy = ((nr[1] - nl[1]) * h) * ih1;
@@ -787,7 +819,7 @@ __device__ __forceinline__ R sa_source(R u, R v, R w, R T, R roe, R nu, R sd, co
     dwy = ((wr[1] - wl[1]) * h) * ih1;
   }
   const R ox = R(0.5) * (dwy - dvz), oy = R(0.5) * (duz - dwx), oz = R(0.5) * (dvx - duy);
-  const R mu0 = v_sqrt(T * T * T) * v_div(R(1.0) + SoT, T + SoT);
+  const R mu0 = v_sqrt(T * T * T) * v_div(sp.SoT1, T + sp.SoT);
   const R vis0 = v_div(mu0, roe);
   const R bigx = v_div(nu, vis0);
   const R b3 = bigx * bigx * bigx;
@@ -802,11 +834,11 @@ __device__ __forceinline__ R sa_source(R u, R v, R w, R T, R roe, R nu, R sd, co
     vis2d = v_div(nu, sd);
   }
   segdis *= segdis;
-  const R olen = v_sqrt(R(2.0)) * v_sqrt(ox * ox + oy * oy + oz * oz);
-  R bigs = olen + v_div(v_div(nu * fv2, segdis), Re);
+  const R olen = sp.sqrt2 * v_sqrt(ox * ox + oy * oy + oz * oz);
+  R bigs = olen + over_re(v_div(nu * fv2, segdis), sp);
   bigs = (R(0.3) * olen < bigs) ? bigs : R(0.3) * olen;
   const R ft2 = R(SA::ct3) * r_exp(-R(SA::ct4) * bigx * bigx);
-  R rr = sa_r(nu, bigs * segdis, Re);
+  R rr = sa_r(nu, bigs * segdis, sp);
   rr = (R(10.0) < rr) ? R(10.0) : rr;
   const R rsix = r_pow6(rr);
   const R g = rr + R(SA::cw2) * (rsix - rr);
@@ -815,8 +847,8 @@ __device__ __forceinline__ R sa_source(R u, R v, R w, R T, R roe, R nu, R sd, co
   const R fw = g * r_root6(v_div(R(1.0) + cw3six, gsix + cw3six));
   R src = -(u * dvisx + v * dvisy + w * dvisz);
   src += R(SA::cb1) * (R(1.0) - ft2) * bigs * nu;
-  src -= v_div((R(SA::cw1) * fw - v_div(R(SA::cb1) * ft2, R(SA::kappa * SA::kappa))) * (vis2d * vis2d), Re);
-  src += v_div(v_div(R(SA::cb2) * (dvisx * dvisx + dvisy * dvisy + dvisz * dvisz), R(SA::segma)), Re);
+  src -= over_re((R(SA::cw1) * fw - v_div(R(SA::cb1) * ft2, R(SA::kappa * SA::kappa))) * (vis2d * vis2d), sp);
+  src += over_re(v_div(R(SA::cb2) * (dvisx * dvisx + dvisy * dvisy + dvisz * dvisz), R(SA::segma)), sp);
   src += mutf;
   return src;
 }

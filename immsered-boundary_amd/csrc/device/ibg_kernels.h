@@ -34,6 +34,12 @@ __device__ __forceinline__ Prim<R, D> pload(const Pack<R, D> &W, int c) {
   return o;
 }
 
+// the records from cell c0 on
+template <typename R, int D>
+__device__ __forceinline__ Pack<R, D> rebase(const Pack<R, D> &W, int c0) {
+  return Pack<R, D>{W.a + c0, D == 3 ? W.e + c0 : W.e};
+}
+
 // velocity of cell c (the 4-vector only; w = 0 in 2D)
 template <typename R, int D>
 __device__ __forceinline__ void uvw_load(const Pack<R, D> &W, int c, R &u, R &v, R &w) {
@@ -108,6 +114,7 @@ struct ViscArgs {
   const uint16_t *slots;
   const BlkInfo *blk;
   const DevPhys *phys;
+  const Flow32 *flow;        // per block (FP32)
   Pack<R, D> W;              // step-start stencil state
   Pack<R, D> Rv;
   const R *nu;               // SA working variable (turb)
@@ -120,14 +127,48 @@ struct ViscArgs {
   const R *rbalv;
 };
 
-template <typename R, int D, class B, class Q>
-__device__ __forceinline__ ViscPhys<R, D> visc_phys(B &bi, Q &P) {
+template <typename R, int D>
+__device__ __forceinline__ ViscPhys<R, D> visc_phys(const BlkInfo *blks, const DevPhys *phys,
+                                                    const Flow32 *flow, int blk) {
   ViscPhys<R, D> vp;
-  vp.Rg = (R)P.Rg; vp.iRe = std::is_same<R, float>::value ? c_rcp((R)P.Re) : (R)P.iRe; vp.qk = (R)P.qk; vp.SoT = (R)P.SoT;
-  vp.ih0 = (R)bi.invh[0]; vp.ih1 = (R)bi.invh[1]; vp.ih2 = (R)bi.invh[2];
-  vp.ar0 = (R)bi.area[0]; vp.ar1 = (R)bi.area[1]; vp.ar2 = (R)bi.area[2];
-  vp.iqkt = std::is_same<R, float>::value ? c_rcp((R)P.qkt_den) : (R)P.iqkt;
+  if constexpr (sizeof(R) == 4) {
+    const auto &F = uni(flow)[blk];
+    vp.Rg = F.Rg; vp.iRe = F.iRe; vp.qk = F.qk; vp.SoT = F.SoT;
+    vp.ih0 = F.invh[0]; vp.ih1 = F.invh[1]; vp.ih2 = F.invh[2];
+    vp.ar0 = F.area[0]; vp.ar1 = F.area[1]; vp.ar2 = F.area[2];
+    vp.iqkt = F.iqkt;
+  } else {
+    const auto &bi = uni(blks)[blk];
+    const auto &P = uni(phys)[bi.case_id];
+    vp.Rg = P.Rg; vp.iRe = P.iRe; vp.qk = P.qk; vp.SoT = P.SoT;
+    vp.ih0 = bi.invh[0]; vp.ih1 = bi.invh[1]; vp.ih2 = bi.invh[2];
+    vp.ar0 = bi.area[0]; vp.ar1 = bi.area[1]; vp.ar2 = bi.area[2];
+    vp.iqkt = P.iqkt;
+  }
   return vp;
+}
+template <typename R, int D>
+__device__ __forceinline__ ViscPhys<R, D> visc_phys(const ViscArgs<R, D> &a, int blk) {
+  return visc_phys<R, D>(a.blk, a.phys, a.flow, blk);
+}
+
+// The FP32 constants of block b (see Flow32).
+__global__ void k_flow32(int nblk, const BlkInfo *blk, const DevPhys *phys, Flow32 *out) {
+  const int b = blockIdx.x * blockDim.x + threadIdx.x;
+  if (b >= nblk) return;
+  const BlkInfo &B = blk[b];
+  const DevPhys &P = phys[B.case_id];
+  Flow32 F;
+  for (int d = 0; d < 3; ++d) { F.area[d] = (float)B.area[d]; F.invh[d] = (float)B.invh[d]; }
+  const PhysR<float> ph = phys_r<float>(P);
+  F.gama = ph.gama; F.Rg = ph.Rg; F.Cv = ph.Cv; F.Ma = ph.Ma;
+  F.gm1 = ph.gm1; F.ig1 = ph.ig1; F.iRg = ph.iRg; F.cpR = ph.cpR;
+  F.SoT = (float)P.SoT; F.SoT1 = 1.0f + F.SoT;
+  F.Re = (float)P.Re; F.iRe = f_rcp(F.Re);
+  F.qk = (float)P.qk; F.iqkt = f_rcp((float)P.qkt_den);
+  F.sqrt2 = v_sqrt(2.0f);
+  F.pad = 0.0f;
+  out[b] = F;
 }
 
 // The viscous flux (and, with the SA closure, the working variable's face
@@ -176,7 +217,7 @@ __device__ __forceinline__ void visc_prep_tile(const ViscArgs<R, D> &a, const Ti
   auto &bi = uni(a.blk)[ti.blk];
   auto &P = uni(a.phys)[bi.case_id];
   if (a.viscous) {
-    const ViscPhys<R, D> vp = visc_phys<R, D>(bi, P);
+    const ViscPhys<R, D> vp = visc_phys<R, D>(a, ti.blk);
     for (int f = threadIdx.x; f < ti.nface; f += blockDim.x) {
       R out[NV];
       R mf;
@@ -262,56 +303,64 @@ __device__ __forceinline__ Prim<R, 2> box_prim(const BlockLds<R> &b, int p) {
 }
 
 // The square and its first nhalo halo entries into LDS (256 threads; the
-// caller syncs).  kT: BlockLds::T too.
+// caller syncs).  p0: this thread's cell in the box.  kT: BlockLds::T too.
 template <typename R, bool kT>
 __device__ __forceinline__ void block_load(const Pack<R, 2> &W, const R *nu, bool turb,
                                            const int *halo, const TileInfo &ti, int nhalo, R Rg,
-                                           const BlockLds<R> &b) {
-  const int i = threadIdx.x;
-  const int c = ti.cell0 + i;
+                                           const BlockLds<R> &b, int p0) {
+  // arrays from the tile's first entry on: a uniform base and a 32-bit offset
+  const unsigned i = threadIdx.x;
   int hc = 0;
-  if (i < nhalo) hc = halo[ti.halo0 + i];
+  if ((int)i < nhalo) hc = (halo + ti.halo0)[i];
   auto put = [&](int p, const typename V4<R>::T &q, R n) {
     if constexpr (kT && sizeof(R) == 4) b.T[p] = f_rcp(q.x * Rg);
     else if constexpr (kT) b.T[p] = v_div(q.w, q.x * Rg);
     b.S[p] = q;
     if (turb) b.nu[p] = n;
   };
-  int x, y;
-  blk_xy(i, x, y);
-  const typename V4<R>::T q = W.a[c];
-  const R n = turb ? nu[c] : R(0);
-  if (i < nhalo) {
+  const typename V4<R>::T q = (W.a + ti.cell0)[i];
+  const R n = turb ? (nu + ti.cell0)[i] : R(0);
+  if ((int)i < nhalo) {
     const typename V4<R>::T qh = W.a[hc];
     const R nh = turb ? nu[hc] : R(0);
-    put(halo_pos(i), qh, nh);
+    put(halo_pos((int)i), qh, nh);
   }
-  put(box_pos(x, y), q, n);
+  put(p0, q, n);
 }
 
-// Face f of a block tile in direction d: f < 256 the low face of cell f,
-// then the high faces of the last row; its high-side cell's coordinates
-template <int d>
-__device__ __forceinline__ void block_face(int f, int &x, int &y) {
-  blk_xy(f & 255, x, y);
-  if (f >= kBlkCells) {
-    x = d == 0 ? kBlkN : f - kBlkCells;
-    y = d == 0 ? f - kBlkCells : kBlkN;
-  }
+// The faces of a block tile, f(direction or -1, direction, high-side cell in
+// the box): the low faces of this thread's cell (box position p), then the
+// last column's x and the last row's y faces, half a wave together.  That
+// wave is another one from workgroup to workgroup, so that the third pass
+// does not always fall on the same SIMD.
+template <class F>
+__device__ __forceinline__ void block_faces(int p, F f) {
+  f(std::integral_constant<int, 0>(), 0, p);
+  // (no overlap of the two: it would cost the registers of both)
+  asm volatile("" ::: "memory");
+  f(std::integral_constant<int, 1>(), 1, p);
+  asm volatile("" ::: "memory");
+  const int l = threadIdx.x & 63;
+  if (((threadIdx.x >> 6) ^ blockIdx.x) & 3 || l >= 2 * kBlkN) return;
+  const int dir = l >> 4, t = l & (kBlkN - 1);
+  f(std::integral_constant<int, -1>(), dir, dir == 0 ? box_pos(kBlkN, t) : box_pos(t, kBlkN));
+}
+// box position of this thread's cell
+__device__ __forceinline__ int block_cell() {
+  int x, y;
+  blk_xy(threadIdx.x, x, y);
+  return box_pos(x, y);
 }
 
-// Viscous fluxes of the faces of direction d into LDS, the working
-// variable's face flux in the mass slot (the viscous mass flux is zero).
-template <typename R, int d>
+// Viscous fluxes of the faces into LDS, the working variable's face flux in
+// the mass slot (the viscous mass flux is zero).  p: this thread's cell.
+template <typename R>
 __device__ __forceinline__ void block_visc_faces(const BlockLds<R> &b, const ViscPhys<R, 2> &vp,
-                                                 bool turb) {
-  constexpr int st = d == 0 ? 1 : kBoxP, tt = d == 0 ? kBoxP : 1;
-  // the last row's faces go to another wave in the y pass than in the x pass
-#pragma unroll 1
-  for (int f = (threadIdx.x + (d == 0 ? 0 : 192)) & 255; f < kBlkCells + kBlkN; f += kBlkCells) {
-    int x, y;
-    block_face<d>(f, x, y);
-    const int p = box_pos(x, y), l = p - st;
+                                                 bool turb, int p0) {
+  block_faces(p0, [&](auto dc, int dir, int p) {
+    constexpr int d = decltype(dc)::value;
+    const int st = dir == 0 ? 1 : kBoxP, tt = dir == 0 ? kBoxP : 1;
+    const int l = p - st;
     R out[4], mf = R(0);
     const R nl = turb ? b.nu[l] : R(0), nr = turb ? b.nu[p] : R(0);
     const int tp[4] = {l + tt, p + tt, l - tt, p - tt};
@@ -319,7 +368,7 @@ __device__ __forceinline__ void block_visc_faces(const BlockLds<R> &b, const Vis
       float tu[4], tv[4];
 #pragma unroll
       for (int k = 0; k < 4; ++k) { tu[k] = b.S[tp[k]].y; tv[k] = b.S[tp[k]].z; }
-      visc_flux_2d<d>(box_prim<R>(b, l), box_prim<R>(b, p), b.T[l], b.T[p], tu, tv, d, vp, out, turb,
+      visc_flux_2d<d>(box_prim<R>(b, l), box_prim<R>(b, p), b.T[l], b.T[p], tu, tv, dir, vp, out, turb,
                       nl, nr, &mf);
     } else {
       auto cell = [&](int q) {
@@ -327,26 +376,24 @@ __device__ __forceinline__ void block_visc_faces(const BlockLds<R> &b, const Vis
         return VelT<R>{s.y, s.z, R(0), b.T[q]};
       };
       const VelT<R> t[4] = {cell(tp[0]), cell(tp[1]), cell(tp[2]), cell(tp[3])};
-      visc_flux<R, 2>(cell(l), cell(p), b.S[l].x, b.S[p].x, t, d, vp, out, turb, nl, nr, &mf);
+      visc_flux<R, 2>(cell(l), cell(p), b.S[l].x, b.S[p].x, t, dir, vp, out, turb, nl, nr, &mf);
     }
     typename V4<R>::T o;
     o.x = mf; o.y = out[1]; o.z = out[2]; o.w = out[3];
-    (d == 0 ? b.fx : b.fy)[y * kBoxP + x] = o;
-  }
+    (dir == 0 ? b.fx : b.fy)[p - box_pos(0, 0)] = o;
+  });
 }
 
 // Rv and the working variable's face term of this thread's cell from the
 // face fluxes in LDS.
 template <typename R, class B, class Q>
 __device__ __forceinline__ void block_visc_cell(const ViscArgs<R, 2> &a, const TileInfo &ti, B &bi,
-                                                Q &P, const BlockLds<R> &b) {
+                                                Q &P, const BlockLds<R> &b, int p) {
   using V = typename V4<R>::T;
-  const int c = ti.cell0 + threadIdx.x;
-  int x, y;
-  blk_xy(threadIdx.x, x, y);
+  const unsigned c = threadIdx.x;
   double s[4] = {0.0, 0.0, 0.0, 0.0}, tot = 0.0;
   if (a.viscous) {
-    const int k = y * kBoxP + x;
+    const int k = p - box_pos(0, 0);
 #pragma unroll
     for (int d = 0; d < 2; ++d) {
       const V lo = d == 0 ? b.fx[k] : b.fy[k], hi = d == 0 ? b.fx[k + 1] : b.fy[k + kBoxP];
@@ -360,8 +407,8 @@ __device__ __forceinline__ void block_visc_cell(const ViscArgs<R, 2> &a, const T
     }
   }
   const R rv[4] = {(R)s[0], (R)s[1], (R)s[2], (R)s[3]};
-  vstore<R, 2>(a.Rv, c, rv);
-  if (a.turb) a.mutf[c] = (R)n_div(n_div(tot, bi.vol), P.Re);
+  vstore<R, 2>(rebase(a.Rv, ti.cell0), c, rv);
+  if (a.turb) (a.mutf + ti.cell0)[c] = (R)n_div(n_div(tot, bi.vol), P.Re);
 }
 
 // The viscous pass of a block tile (visc_prep_tile's work).
@@ -371,17 +418,16 @@ __device__ __forceinline__ void visc_prep_block(const ViscArgs<R, 2> &a, const T
   auto &bi = uni(a.blk)[ti.blk];
   auto &P = uni(a.phys)[bi.case_id];
   const BlockLds<R> b = block_lds<R>(smem_raw, a.turb);
+  const int p = block_cell();
   if (a.viscous) {
-    block_load<R, true>(a.W, a.nu, a.turb, a.halo, ti, kHaloC, (R)P.Rg, b);
+    block_load<R, true>(a.W, a.nu, a.turb, a.halo, ti, kHaloC, (R)P.Rg, b, p);
     __syncthreads();
-    const ViscPhys<R, 2> vp = visc_phys<R, 2>(bi, P);
-    block_visc_faces<R, 0>(b, vp, a.turb);
-    block_visc_faces<R, 1>(b, vp, a.turb);
+    block_visc_faces<R>(b, visc_phys<R, 2>(a, ti.blk), a.turb, p);
   }
   if (threadIdx.x == 0) *halt = herr ? 1 : 0;
   __syncthreads();
   if (*halt) return;
-  block_visc_cell<R>(a, ti, bi, P, b);
+  block_visc_cell<R>(a, ti, bi, P, b, p);
 }
 
 // ---- 3D
@@ -473,7 +519,7 @@ __device__ __forceinline__ void visc_prep_block3(const ViscArgs<R, 3> &a, const 
   double s[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, tot = 0.0;
   if (a.viscous) {
     block3_load<R, true>(a.W, a.nu, a.turb, a.halo, ti, (R)P.Rg, b);
-    const ViscPhys<R, 3> vp = visc_phys<R, 3>(bi, P);
+    const ViscPhys<R, 3> vp = visc_phys<R, 3>(a, ti.blk);
     __syncthreads();
     auto direction = [&](auto dc) {
       constexpr int d = decltype(dc)::value;
@@ -562,6 +608,7 @@ struct StageArgs {
   const uint8_t *flags;      // [Nn]
   const BlkInfo *blk;
   const DevPhys *phys;
+  const Flow32 *flow;        // per block (FP32)
   const double *dt;          // [ncases]
   Pack<R, D> Win;            // stencil state this stage reads
   Pack<R, D> Wout;           // stencil state this stage writes (another buffer)
@@ -758,7 +805,18 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
   if (ML && threadIdx.x == 0) { mlc[0] = 0u; mlc[1] = 0u; }
   auto &bi = uni(a.blk)[ti.blk];
   auto &P = uni(a.phys)[bi.case_id];
-  const PhysR<R> ph = phys_r<R>(P);
+  const auto &F32 = uni(a.flow)[ti.blk];
+  PhysR<R> ph;
+  R ar0, ar1, ar2, ih0, ih1, ih2;
+  if constexpr (kMixed) {
+    ph = phys_r32(F32);
+    ar0 = F32.area[0]; ar1 = F32.area[1]; ar2 = F32.area[2];
+    ih0 = F32.invh[0]; ih1 = F32.invh[1]; ih2 = F32.invh[2];
+  } else {
+    ph = phys_r<R>(P);
+    ar0 = bi.area[0]; ar1 = bi.area[1]; ar2 = bi.area[2];
+    ih0 = bi.invh[0]; ih1 = bi.invh[1]; ih2 = bi.invh[2];
+  }
   V *fl4 = reinterpret_cast<V *>(smem_raw);
   R *fl1 = reinterpret_cast<R *>(smem_raw + sizeof(V) * (size_t)ti.nface);   // 3D 5th value
   // SA: the low / high cell of each face; the cell phase gathers their
@@ -766,12 +824,16 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
   int *fL = reinterpret_cast<int *>(smem_raw + (sizeof(V) + (D == 3 ? sizeof(R) : 0)) * (size_t)ti.nface);
   int *fR = fL + ti.nface;
   const BlockLds<R> bl = block_lds<R>(smem_raw, a.turb);
-  // this thread's cell in a block tile, formed anew at each use (held across
-  // the network it costs the ML instantiation registers it spills)
-  auto my_xy = [&](int &x, int &y) {
-    int i = threadIdx.x;
+  // this thread's cell in a block tile; after the face phase the ML
+  // instantiation forms it anew at each use (held across the network it costs
+  // registers that spill)
+  const int bp0 = (BLK && D == 2) ? block_cell() : 0;
+  auto my_p = [&]() {
+    if constexpr (!ML) return bp0;
+    int i = threadIdx.x, x, y;
     asm volatile("" : "+v"(i));
     blk_xy(i, x, y);
+    return box_pos(x, y);
   };
   const Block3Lds<R> b3 = block3_lds<R>(smem_raw, kBox3Cells);
   double s[NV];   // residual of the cell
@@ -804,7 +866,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
         }
         R flux[5];
         roe_flux<3, d>(box3_prim<R>(b3, q[0]), box3_prim<R>(b3, q[1]), box3_prim<R>(b3, q[2]),
-                       box3_prim<R>(b3, q[3]), d, (R)bi.area[d], ph, a.limiter, flux);
+                       box3_prim<R>(b3, q[3]), d, d == 0 ? ar0 : (d == 1 ? ar1 : ar2), ph, a.limiter, flux);
         V o;
         o.x = flux[0]; o.y = flux[1]; o.z = flux[2]; o.w = flux[3];
         const int k = flux3_slot(d, x, y, z);
@@ -830,11 +892,9 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
     bool loaded = false;
     if constexpr (kFuseVisc<R, D>) {
       if (a.fuse_visc && a.va.viscous) {
-        block_load<R, true>(a.Win, a.nuin, a.turb, a.halo, ti, kHalo, (R)P.Rg, bl);
+        block_load<R, true>(a.Win, a.nuin, a.turb, a.halo, ti, kHalo, (R)P.Rg, bl, bp0);
         __syncthreads();
-        const ViscPhys<R, 2> vp = visc_phys<R, 2>(bi, P);
-        block_visc_faces<R, 0>(bl, vp, a.turb);
-        block_visc_faces<R, 1>(bl, vp, a.turb);
+        block_visc_faces<R>(bl, visc_phys<R, 2>(a.va, ti.blk), a.turb, bp0);
         loaded = true;
       }
       if (a.fuse_visc) {
@@ -842,34 +902,25 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
         if (threadIdx.x == 0) halt = herr ? 1 : 0;
         __syncthreads();
         if (halt) return;
-        block_visc_cell<R>(a.va, ti, bi, P, bl);
+        block_visc_cell<R>(a.va, ti, bi, P, bl, bp0);
         __syncthreads();   // the face arrays are reused by phase 1
       }
     }
     if (!loaded) {
-      block_load<R, false>(a.Win, a.nuin, a.turb, a.halo, ti, kHalo, R(0), bl);
+      block_load<R, false>(a.Win, a.nuin, a.turb, a.halo, ti, kHalo, R(0), bl, bp0);
       __syncthreads();
     }
-    // phase 1: the low face of every cell and the last row's high faces,
-    // which go to another wave in the y pass than in the x pass
-    auto faces = [&](auto dc) {
+    // phase 1
+    block_faces(bp0, [&](auto dc, int dir, int p) {
       constexpr int d = decltype(dc)::value;
-      constexpr int st = d == 0 ? 1 : kBoxP;
-#pragma unroll 1
-      for (int f = (threadIdx.x + (d == 0 ? 0 : 192)) & 255; f < kBlkCells + kBlkN; f += kBlkCells) {
-        int x, y;
-        block_face<d>(f, x, y);
-        const int p = box_pos(x, y);
-        R flux[4];
-        roe_flux<2, d>(box_prim<R>(bl, p - 2 * st), box_prim<R>(bl, p - st), box_prim<R>(bl, p),
-                       box_prim<R>(bl, p + st), d, (R)bi.area[d], ph, a.limiter, flux);
-        V o;
-        o.x = flux[0]; o.y = flux[1]; o.z = flux[2]; o.w = flux[3];
-        (d == 0 ? bl.fx : bl.fy)[y * kBoxP + x] = o;
-      }
-    };
-    faces(std::integral_constant<int, 0>());
-    faces(std::integral_constant<int, 1>());
+      const int st = dir == 0 ? 1 : kBoxP;
+      R flux[4];
+      roe_flux<2, d, kMixed>(box_prim<R>(bl, p - 2 * st), box_prim<R>(bl, p - st), box_prim<R>(bl, p),
+                             box_prim<R>(bl, p + st), dir, dir == 0 ? ar0 : ar1, ph, a.limiter, flux);
+      V o;
+      o.x = flux[0]; o.y = flux[1]; o.z = flux[2]; o.w = flux[3];
+      (dir == 0 ? bl.fx : bl.fy)[p - box_pos(0, 0)] = o;
+    });
   } else {
     if constexpr (kFuseVisc<R, D>) {
       if (a.fuse_visc) {
@@ -881,7 +932,6 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
         __syncthreads();   // the face arrays are reused by phase 1
       }
     }
-    const R ar0 = (R)bi.area[0], ar1 = (R)bi.area[1], ar2 = (R)bi.area[2];
     for (int f = threadIdx.x; f < ti.nface; f += blockDim.x) {
       const int4 st = a.tst[ti.face0 + f];
       const int dir = a.tdir[ti.face0 + f];
@@ -916,8 +966,11 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
   const double level_ts = a.alpha * uni(a.dt)[bi.case_id] * bi.step_num;
   const int i = threadIdx.x;
   const bool live = BLK || i < ti.ncell;
-  const int c = ti.cell0 + (live ? i : 0);
-  const uint8_t fg = live ? a.flags[c] : 0;
+  // the per-cell arrays from the tile's first cell on, entry c: a uniform base
+  // and a 32-bit offset
+  const int c0 = ti.cell0;
+  const unsigned c = live ? (unsigned)i : 0u;
+  const uint8_t fg = live ? (a.flags + c0)[c] : 0;
   // ---- phase 2a: residual of the cell, the SA terms
   double snu = 0.0;
   bool sa_on = false;
@@ -927,11 +980,11 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
   // the cell's face slots in the tile's face list
   auto load_slots = [&](int *sl) {
     if (D == 2) {
-      const ushort4 s4 = *reinterpret_cast<const ushort4 *>(a.slots + (size_t)c * 4);
+      const ushort4 s4 = reinterpret_cast<const ushort4 *>(a.slots + (size_t)c0 * 4)[c];
       sl[0] = s4.x; sl[1] = s4.y; sl[2] = s4.z; sl[3] = s4.w;
     } else {
 #pragma unroll
-      for (int q = 0; q < 2 * D; ++q) sl[q] = a.slots[(size_t)c * 2 * D + q];
+      for (int q = 0; q < 2 * D; ++q) sl[q] = (a.slots + (size_t)c0 * 2 * D)[c * 2 * D + q];
     }
   };
   int sl[2 * D];
@@ -942,15 +995,14 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
   // nor the slots are held in registers across the network (they spill).
   auto residual = [&]() {
     if constexpr (ML && !BLK) load_slots(sl);
-    int bx = 0, by = 0;
-    if constexpr (BLK && D == 2) my_xy(bx, by);
+    int bp = 0;
+    if constexpr (BLK && D == 2) bp = my_p() - box_pos(0, 0);
 #pragma unroll
     for (int d = 0; d < ((BLK && D == 3) ? 0 : D); ++d) {
       V lo, hi;
       if constexpr (BLK) {
-        const int k = by * kBoxP + bx;
-        lo = d == 0 ? bl.fx[k] : bl.fy[k];
-        hi = d == 0 ? bl.fx[k + 1] : bl.fy[k + kBoxP];
+        lo = d == 0 ? bl.fx[bp] : bl.fy[bp];
+        hi = d == 0 ? bl.fx[bp + 1] : bl.fy[bp + kBoxP];
       } else {
         lo = fl4[sl[2 * d]];
         hi = fl4[sl[2 * d + 1]];
@@ -962,7 +1014,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
       if (D == 3) s[4] += (double)fl1[sl[2 * d]] - (double)fl1[sl[2 * d + 1]];
     }
     R rv[NV];
-    vload<R, D>(a.Rv, c, rv);
+    vload<R, D>(rebase(a.Rv, c0), c, rv);
 #pragma unroll
     for (int k = 0; k < NV; ++k) s[k] += (double)rv[k];
   };
@@ -973,15 +1025,15 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
     if (a.turb && (fg & F_UPDATE) && (fg & F_SA)) {
       sa_on = true;
       Prim<R, D> me;
-      int bx = 0, by = 0, bz = 0;
+      int bp = 0, bx = 0, by = 0, bz = 0;
       if constexpr (BLK && D == 2) {
-        my_xy(bx, by);
-        me = box_prim<R>(bl, box_pos(bx, by));
+        bp = my_p();
+        me = box_prim<R>(bl, bp);
       } else if constexpr (BLK) {
         blk_xyz(threadIdx.x, bx, by, bz);
         me = box3_prim<R>(b3, box3_in(bx, by, bz));
       } else {
-        me = pload<R, D>(a.Win, c);
+        me = pload<R, D>(rebase(a.Win, c0), c);
       }
       R nl[3], nr[3], ul[3], ur[3], vl[3], vr[3], wl[3], wr[3];
 #pragma unroll
@@ -996,7 +1048,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
           nl[d] = b3.nu[lp];
           nr[d] = b3.nu[rp];
         } else if (BLK && d < D) {
-          const int p = box_pos(bx, by), st = d == 0 ? 1 : kBoxP;
+          const int p = bp, st = d == 0 ? 1 : kBoxP;
           const V lo = bl.S[p - st], hi = bl.S[p + st];
           ul[d] = lo.y; vl[d] = lo.z; wl[d] = R(0);
           ur[d] = hi.y; vr[d] = hi.z; wr[d] = R(0);
@@ -1012,16 +1064,19 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
           ul[d] = ur[d] = vl[d] = vr[d] = wl[d] = wr[d] = nl[d] = nr[d] = R(0);
         }
       }
-      const R T = v_div(me.p, me.r * (R)P.Rg);
-      const R nu = !BLK ? a.nuin[c] : (D == 2 ? bl.nu[box_pos(bx, by)] : b3.nu[box3_in(bx, by, bz)]);
-      const R sd = kMixed ? (R)a.sd32[c] : (R)a.signdis[c];
+      const R T = v_div(me.p, me.r * ph.Rg);
+      const R nu = !BLK ? (a.nuin + c0)[c] : (D == 2 ? bl.nu[bp] : b3.nu[box3_in(bx, by, bz)]);
+      const R sd = kMixed ? (R)(a.sd32 + c0)[c] : (R)(a.signdis + c0)[c];
+      const R mutf = (a.mutf + c0)[c];
+      SaPhys<R> sp;
+      if constexpr (kMixed) sp = sa_phys32(F32);
+      else sp = sa_phys(P);
       if constexpr (!ML) {
         snu = (double)sa_source<R, D>(me.u, me.v, me.w, T, me.r, nu, sd, nl, nr, ul, ur, vl, vr,
-                                      wl, wr, (R)bi.invh[0], (R)bi.invh[1], (R)bi.invh[2],
-                                      (R)P.SoT, (R)P.Re, a.mutf[c]);
+                                      wl, wr, ih0, ih1, ih2, sp, mutf);
       } else {
         const R h = R(0.5);
-        const R i0 = (R)bi.invh[0], i1 = (R)bi.invh[1], i2 = (R)bi.invh[2];
+        const R i0 = ih0, i1 = ih1, i2 = ih2;
         VelGrad<R> g;
         g.dux = ((ur[0] - ul[0]) * h) * i0; g.dvx = ((vr[0] - vl[0]) * h) * i0; g.dwx = ((wr[0] - wl[0]) * h) * i0;
         g.duy = ((ur[1] - ul[1]) * h) * i1; g.dvy = ((vr[1] - vl[1]) * h) * i1; g.dwy = ((wr[1] - wl[1]) * h) * i1;
@@ -1032,15 +1087,14 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
         }
         const R dvisx = ((nr[0] - nl[0]) * h) * i0, dvisy = ((nr[1] - nl[1]) * h) * i1;
         const R dvisz = (D == 3) ? ((nr[2] - nl[2]) * h) * i2 : R(0);
-        const R Re = (R)P.Re;
-        const R olen = sa_olen<R>(g);
-        const R mu0 = v_sqrt(T * T * T) * v_div(R(1.0) + (R)P.SoT, T + (R)P.SoT);
+        const R olen = sa_olen<R>(g, sp);
+        const R mu0 = v_sqrt(T * T * T) * v_div(sp.SoT1, T + sp.SoT);
         // derivative terms in their discrete form
         sa_rest = -(me.u * dvisx + me.v * dvisy + me.w * dvisz) +
-                  v_div(v_div(R(SA::cb2) * (dvisx * dvisx + dvisy * dvisy + dvisz * dvisz), R(SA::segma)), Re) +
-                  a.mutf[c];
+                  over_re(v_div(R(SA::cb2) * (dvisx * dvisx + dvisy * dvisy + dvisz * dvisz), R(SA::segma)), sp) +
+                  mutf;
         sa_nu = nu;
-        bool ok = sa_features<R>(me.u, me.v, me.w, me.r, me.p, mu0, nu, sd, g, olen, Re,
+        bool ok = sa_features<R>(me.u, me.v, me.w, me.r, me.p, mu0, nu, sd, g, olen, sp.Re,
                                  (R)P.init[4], ml_x, ml_scale);
         // the range test without short-circuit branches (a chain of
         // exec-mask branches, one per bound, otherwise)
@@ -1048,7 +1102,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
         for (int k = 0; k < kMlpIn; ++k)
           ok = ok & (ml_x[k] >= uni(a.mlp.flo)[k]) & (ml_x[k] <= uni(a.mlp.fhi)[k]);
         use_ml = ok;
-        if (!ok) snu = (double)(sa_rest + sa_pointwise<R>(nu, mu0, me.r, sd, olen, Re));
+        if (!ok) snu = (double)(sa_rest + sa_pointwise<R>(nu, mu0, me.r, sd, olen, sp));
       }
     }
   }
@@ -1118,7 +1172,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
       // e = Cv T + |u|^2/2, T = p/(roe Rg)
       double U[NV];
       {
-        const Prim<double, D> w0 = pload<double, D>(a.W64, c);
+        const Prim<double, D> w0 = pload<double, D>(rebase(a.W64, c0), c);
         const double ke0 = (D == 3) ? 0.5 * (w0.u * w0.u + w0.v * w0.v + w0.w * w0.w)
                                     : 0.5 * (w0.u * w0.u + w0.v * w0.v);
         double re0;
@@ -1133,10 +1187,10 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
       for (int k = 0; k < NV; ++k) U[k] = fma(s[k], sc, U[k]);
       if (a.turb) {
         // viseddy = max(c_vis_old + mutsource * level_ts, 0) (:874-876, :955-957)
-        nu_new = a.nu64[c] + snu * level_ts;
+        nu_new = (a.nu64 + c0)[c] + snu * level_ts;
         nu_new = (nu_new < 0.0) ? 0.0 : nu_new;
       }
-      if (U[0] < 0.0) report_error(a.err, c, (fg & F_FINEST) ? 611 : 523);
+      if (U[0] < 0.0) report_error(a.err, c0 + (int)c, (fg & F_FINEST) ? 611 : 523);
       if (fg & F_PRIM) {
         // Get_Prim_Vars FlowVariables.H:50-57
         wr = U[0];
@@ -1162,7 +1216,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
           wp = (U[D == 3 ? 4 : 3] - ke * wr) * (P.gama - 1.0);
         }
         // T = p/(roe Rg) < 0  (NS_Solver.cpp:55-66), Rg > 0
-        if ((wp < 0.0) != (wr < 0.0)) report_error(a.err, c, 37);
+        if ((wp < 0.0) != (wr < 0.0)) report_error(a.err, c0 + (int)c, 37);
         write = true;
       }
     }
@@ -1173,26 +1227,26 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
       write = true;
     }
     if (write) {
-      pstore<R, D>(a.Wout, c, (R)wr, (R)wu, (R)wv, (R)ww, (R)wp);
-      if (kMixed && a.last) pstore<double, D>(a.W64, c, wr, wu, wv, ww, wp);
+      pstore<R, D>(rebase(a.Wout, c0), c, (R)wr, (R)wu, (R)wv, (R)ww, (R)wp);
+      if (kMixed && a.last) pstore<double, D>(rebase(a.W64, c0), c, wr, wu, wv, ww, wp);
     }
     if (a.turb && ((fg & F_UPDATE) || (fg & F_FREE))) {
-      a.nuout[c] = (R)nu_new;
-      if (kMixed && a.last) a.nu64[c] = nu_new;
+      (a.nuout + c0)[c] = (R)nu_new;
+      if (kMixed && a.last) (a.nu64 + c0)[c] = nu_new;
     }
     if (a.last) {
       if (a.src) {
-        double *o = a.src + (size_t)c * 5;
+        double *o = a.src + (size_t)(c0 + (int)c) * 5;
         o[0] = s[0]; o[1] = s[1]; o[2] = s[2];
         if (D == 3) { o[3] = s[3]; o[4] = s[4]; } else { o[3] = 0.0; o[4] = s[3]; }
       }
-      if (a.nusrc) a.nusrc[c] = snu;
+      if (a.nusrc) (a.nusrc + c0)[c] = snu;
       if (fg & F_RESID) {
         bool nan = (snu != snu);
 #pragma unroll
         for (int k = 0; k < NV; ++k) nan = nan || (s[k] != s[k]);
         // a NaN residual aborts the march (ResinDomain, NS_Solver.H:355-375)
-        if (nan) report_error(a.err, c, 268);
+        if (nan) report_error(a.err, c0 + (int)c, 268);
       }
     }
   }
@@ -1862,13 +1916,12 @@ __global__ void k_face_probe(int nface, const int4 *st, const int8_t *dir, const
 template <typename R, int D>
 __global__ void k_visc_probe(int nface, const int4 *st, const int4 *vst, const int8_t *dir,
                              const int16_t *fblk, Pack<R, D> W, const BlkInfo *blk,
-                             const DevPhys *phys, const R *nu, double *out, double *mout) {
+                             const DevPhys *phys, const Flow32 *flow, const R *nu, double *out,
+                             double *mout) {
   const int f = blockIdx.x * blockDim.x + threadIdx.x;
   if (f >= nface) return;
   constexpr int NV = D + 2;
-  const BlkInfo &bi = blk[fblk[f]];
-  const DevPhys &P = phys[bi.case_id];
-  const ViscPhys<R, D> vp = visc_phys<R, D>(bi, P);
+  const ViscPhys<R, D> vp = visc_phys<R, D>(blk, phys, flow, fblk[f]);
   const int4 s = st[f];
   Prim<R, D> t[(D == 3) ? 8 : 4];
   const int4 v0 = vst[(size_t)f * (D - 1)];

@@ -192,9 +192,9 @@ struct VelGrad {
 
 // |Omega| as the reference forms it: sqrt(2) |curl(u)/2| (NS_Solver.cpp:688-731)
 template <typename R>
-__device__ __forceinline__ R sa_olen(const VelGrad<R> &g) {
+__device__ __forceinline__ R sa_olen(const VelGrad<R> &g, const SaPhys<R> &sp) {
   const R ox = R(0.5) * (g.dwy - g.dvz), oy = R(0.5) * (g.duz - g.dwx), oz = R(0.5) * (g.dvx - g.duy);
-  return v_sqrt(R(2.0)) * v_sqrt(ox * ox + oy * oy + oz * oz);
+  return sp.sqrt2 * v_sqrt(ox * ox + oy * oy + oz * oz);
 }
 
 // Point-wise production - destruction of the SA source for one cell, the
@@ -202,7 +202,8 @@ __device__ __forceinline__ R sa_olen(const VelGrad<R> &g) {
 // (cw1 fw - cb1 ft2/kappa^2)(nu/d)^2/Re), from the working variable, the
 // laminar viscosity mu, roe, the wall distance and |Omega|.
 template <typename R>
-__device__ __forceinline__ R sa_pointwise(R nu, R mu0, R roe, R sd, R olen, R Re) {
+__device__ __forceinline__ R sa_pointwise(R nu, R mu0, R roe, R sd, R olen,
+                                          const SaPhys<R> &sp) {
   const R vis0 = v_div(mu0, roe);
   const R bigx = v_div(nu, vis0);
   const R b3 = bigx * bigx * bigx;
@@ -217,17 +218,17 @@ __device__ __forceinline__ R sa_pointwise(R nu, R mu0, R roe, R sd, R olen, R Re
     vis2d = v_div(nu, sd);
   }
   segdis *= segdis;
-  R bigs = olen + v_div(v_div(nu * fv2, segdis), Re);
+  R bigs = olen + over_re(v_div(nu * fv2, segdis), sp);
   bigs = (R(0.3) * olen < bigs) ? bigs : R(0.3) * olen;
   const R ft2 = R(SA::ct3) * r_exp(-R(SA::ct4) * bigx * bigx);
-  R rr = sa_r(nu, bigs * segdis, Re);
+  R rr = sa_r(nu, bigs * segdis, sp);
   rr = (R(10.0) < rr) ? R(10.0) : rr;
   const R rsix = r_pow6(rr);
   const R g = rr + R(SA::cw2) * (rsix - rr);
   const R gsix = r_pow6(g);
   const R fw = g * r_root6(v_div(R(65.0), gsix + R(64.0)));
   const R prod = R(SA::cb1) * (R(1.0) - ft2) * bigs * nu;
-  const R dest = v_div((R(SA::cw1) * fw - v_div(R(SA::cb1) * ft2, R(SA::kappa * SA::kappa))) * (vis2d * vis2d), Re);
+  const R dest = over_re((R(SA::cw1) * fw - v_div(R(SA::cb1) * ft2, R(SA::kappa * SA::kappa))) * (vis2d * vis2d), sp);
   return prod - dest;
 }
 

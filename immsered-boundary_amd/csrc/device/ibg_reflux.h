@@ -110,8 +110,7 @@ k_balance_visc(ViscArgs<R, D> a, const RfPair *pairs, int n, R *rbalv) {
 #pragma unroll
   for (int k = 0; k <= 4; ++k) {
     if (k > nf) break;
-    const BlkInfo &bi = a.blk[k == 0 ? p.cblk : p.fblk];
-    const ViscPhys<R, D> vp = visc_phys<R, D>(bi, a.phys[bi.case_id]);
+    const ViscPhys<R, D> vp = visc_phys<R, D>(a, k == 0 ? p.cblk : p.fblk);
     R mf;
     visc_face<R, D>(a, vp, k == 0 ? p.cslot : p.fslot[k - 1], F[k], mf);
   }
