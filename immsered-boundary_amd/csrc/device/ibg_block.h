@@ -15,7 +15,8 @@
 //
 // Average launch, general tiles only -> with block tiles.  2D, moving
 // 2.6M-cell section: k_stage FP64 150 -> 134 us, FP32 71 -> 61 us (the
-// learned closure's 97 -> 87 us), k_visc_prep FP32 66 -> 43 us.  3D, 2.7M
+// learned closure's 97 -> 87 us), k_visc_prep FP32 66 -> 43 us (30 with the
+// layout below).  3D, 2.7M
 // cells: k_stage FP32 147 -> 124 us, FP64 300 -> 294 us, k_visc_prep FP32
 // 172 -> 75 us, FP64 321 -> 179 us.  The FP32 stages then issue vector
 // instructions for 77 % (3D) to 92 % (2D) of their time (2D: the bytes alone
@@ -54,17 +55,41 @@ __host__ __device__ inline void blk_xy(int i, int &x, int &y) {
   y = ((i >> 1) & 1) | ((i >> 2) & 2) | ((i >> 3) & 4) | ((i >> 4) & 8);
 }
 
-// box position of halo entry h
-__host__ __device__ inline int halo_pos(int h) {
+// coordinates of halo entry h (-2 .. 17)
+__host__ __device__ inline void halo_xy(int h, int &x, int &y) {
   if (h >= kHaloL1 && h < kHaloC) {
     const int c = h - kHaloL1;
-    return box_pos((c & 1) ? kBlkN : -1, (c & 2) ? kBlkN : -1);
+    x = (c & 1) ? kBlkN : -1;
+    y = (c & 2) ? kBlkN : -1;
+    return;
   }
   const int far = h >= kHaloC ? 1 : 0;
   const int k = far ? h - kHaloC : h;
   const int t = k & (kBlkN - 1), side = k >> 4;
   const int o = (side & 1) ? kBlkN + far : -1 - far;
-  return (side & 2) ? box_pos(t, o) : box_pos(o, t);
+  x = (side & 2) ? t : o;
+  y = (side & 2) ? o : t;
+}
+// box position of halo entry h
+__host__ __device__ inline int halo_pos(int h) {
+  int x, y;
+  halo_xy(h, x, y);
+  return box_pos(x, y);
+}
+
+// The FP32 viscous pass keeps the square and one halo layer as pairs (u, v),
+// (roe, p) and (1 / (roe Rg), working variable): a face reads the velocities
+// of six cells and the rest of two, mostly as two neighbouring records by one
+// instruction for 16 lanes at a time; at pitch 20 their five rows (or five
+// columns) of four 8-byte records lie on distinct banks.  From the stage's
+// 16-byte records the reads of (u, v) alone used half the banks: 325 of the
+// pass's 585 cycles per wave and CU were bank conflicts, 136 of 450 now; with
+// pitch 24 (32 lanes of one record each on distinct banks) 207 of 500.
+// 43 -> 30 us on the moving section.
+constexpr int kViscP = 20, kViscCells = (kBlkN + 2) * kViscP;
+__host__ __device__ constexpr int visc_pos(int x, int y) { return (y + 1) * kViscP + x + 1; }
+__host__ __device__ constexpr size_t blk_visc_smem32() {
+  return 16 * (size_t)kFluxSlots + 3 * 8 * (size_t)kViscCells;
 }
 
 // LDS bytes of a block tile: fluxes, the box's states, with the SA closure

@@ -401,7 +401,7 @@ size_t tile_smem(const ibg_ctx *c, size_t rsize, bool stage, bool fused = false)
   if (c->turb) per += stage ? std::max<size_t>(2 * sizeof(int), rsize) : rsize;
   size_t b = (size_t)c->max_tile_faces * per;
   if (c->nblock > 0)
-    b = std::max(b, c->D == 2 ? blk_smem(rsize, c->turb, fused || !stage)
+    b = std::max(b, c->D == 2 ? (rsize == 4 && !stage ? blk_visc_smem32() : blk_smem(rsize, c->turb, fused || !stage))
                               : (stage ? blk3_smem(rsize, c->turb) : blk3_visc_smem(rsize, c->turb)));
   if (stage && c->cl.on) {
     // the network's weights: after every face array, resident across the

@@ -283,8 +283,8 @@ template <typename R>
 struct BlockLds {
   typename V4<R>::T *fx, *fy;   // fluxes of the x and y faces
   typename V4<R>::T *S;         // states of the box
-  R *nu, *T;                    // working variable (SA); temperature (FP64) or
-                                // 1 / (roe Rg) (FP32) for the viscous flux
+  R *nu, *T;                    // working variable (SA); temperature for the
+                                // viscous flux (FP64)
 };
 template <typename R>
 __device__ __forceinline__ BlockLds<R> block_lds(unsigned char *smem, bool turb) {
@@ -313,8 +313,7 @@ __device__ __forceinline__ void block_load(const Pack<R, 2> &W, const R *nu, boo
   int hc = 0;
   if ((int)i < nhalo) hc = (halo + ti.halo0)[i];
   auto put = [&](int p, const typename V4<R>::T &q, R n) {
-    if constexpr (kT && sizeof(R) == 4) b.T[p] = f_rcp(q.x * Rg);
-    else if constexpr (kT) b.T[p] = v_div(q.w, q.x * Rg);
+    if constexpr (kT) b.T[p] = v_div(q.w, q.x * Rg);
     b.S[p] = q;
     if (turb) b.nu[p] = n;
   };
@@ -328,22 +327,29 @@ __device__ __forceinline__ void block_load(const Pack<R, 2> &W, const R *nu, boo
   put(p0, q, n);
 }
 
-// The faces of a block tile, f(direction or -1, direction, high-side cell in
-// the box): the low faces of this thread's cell (box position p), then the
+// The faces of a block tile, f(direction or -1, direction, x, y of the
+// high-side cell): the low faces of this thread's cell (x, y), then the
 // last column's x and the last row's y faces, half a wave together.  That
 // wave is another one from workgroup to workgroup, so that the third pass
 // does not always fall on the same SIMD.
 template <class F>
-__device__ __forceinline__ void block_faces(int p, F f) {
-  f(std::integral_constant<int, 0>(), 0, p);
+__device__ __forceinline__ void block_faces(int x, int y, F f) {
+  f(std::integral_constant<int, 0>(), 0, x, y);
   // (no overlap of the two: it would cost the registers of both)
   asm volatile("" ::: "memory");
-  f(std::integral_constant<int, 1>(), 1, p);
+  f(std::integral_constant<int, 1>(), 1, x, y);
   asm volatile("" ::: "memory");
   const int l = threadIdx.x & 63;
   if (((threadIdx.x >> 6) ^ blockIdx.x) & 3 || l >= 2 * kBlkN) return;
   const int dir = l >> 4, t = l & (kBlkN - 1);
-  f(std::integral_constant<int, -1>(), dir, dir == 0 ? box_pos(kBlkN, t) : box_pos(t, kBlkN));
+  f(std::integral_constant<int, -1>(), dir, dir == 0 ? kBlkN : t, dir == 0 ? t : kBlkN);
+}
+// the same with the box position of the high-side cell, p that of this thread's
+template <class F>
+__device__ __forceinline__ void block_faces(int p, F f) {
+  block_faces(0, 0, [&](auto dc, int dir, int x, int y) {
+    f(dc, dir, decltype(dc)::value >= 0 ? p : box_pos(x, y));
+  });
 }
 // box position of this thread's cell
 __device__ __forceinline__ int block_cell() {
@@ -352,8 +358,8 @@ __device__ __forceinline__ int block_cell() {
   return box_pos(x, y);
 }
 
-// Viscous fluxes of the faces into LDS, the working variable's face flux in
-// the mass slot (the viscous mass flux is zero).  p: this thread's cell.
+// FP64 viscous fluxes of the faces into LDS, the working variable's face flux
+// in the mass slot (the viscous mass flux is zero).  p: this thread's cell.
 template <typename R>
 __device__ __forceinline__ void block_visc_faces(const BlockLds<R> &b, const ViscPhys<R, 2> &vp,
                                                  bool turb, int p0) {
@@ -364,20 +370,12 @@ __device__ __forceinline__ void block_visc_faces(const BlockLds<R> &b, const Vis
     R out[4], mf = R(0);
     const R nl = turb ? b.nu[l] : R(0), nr = turb ? b.nu[p] : R(0);
     const int tp[4] = {l + tt, p + tt, l - tt, p - tt};
-    if constexpr (sizeof(R) == 4) {
-      float tu[4], tv[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k) { tu[k] = b.S[tp[k]].y; tv[k] = b.S[tp[k]].z; }
-      visc_flux_2d<d>(box_prim<R>(b, l), box_prim<R>(b, p), b.T[l], b.T[p], tu, tv, dir, vp, out, turb,
-                      nl, nr, &mf);
-    } else {
-      auto cell = [&](int q) {
-        const typename V4<R>::T s = b.S[q];
-        return VelT<R>{s.y, s.z, R(0), b.T[q]};
-      };
-      const VelT<R> t[4] = {cell(tp[0]), cell(tp[1]), cell(tp[2]), cell(tp[3])};
-      visc_flux<R, 2>(cell(l), cell(p), b.S[l].x, b.S[p].x, t, dir, vp, out, turb, nl, nr, &mf);
-    }
+    auto cell = [&](int q) {
+      const typename V4<R>::T s = b.S[q];
+      return VelT<R>{s.y, s.z, R(0), b.T[q]};
+    };
+    const VelT<R> t[4] = {cell(tp[0]), cell(tp[1]), cell(tp[2]), cell(tp[3])};
+    visc_flux<R, 2>(cell(l), cell(p), b.S[l].x, b.S[p].x, t, dir, vp, out, turb, nl, nr, &mf);
     typename V4<R>::T o;
     o.x = mf; o.y = out[1]; o.z = out[2]; o.w = out[3];
     (dir == 0 ? b.fx : b.fy)[p - box_pos(0, 0)] = o;
@@ -411,6 +409,51 @@ __device__ __forceinline__ void block_visc_cell(const ViscArgs<R, 2> &a, const T
   if (a.turb) (a.mutf + ti.cell0)[c] = (R)n_div(n_div(tot, bi.vol), P.Re);
 }
 
+// The FP32 viscous pass of a block tile up to the fluxes in LDS (layout:
+// ibg_block.h).  (x, y): this thread's cell.  The halo's first layer only.
+__device__ __forceinline__ void block_visc_faces32(const ViscArgs<float, 2> &a, const TileInfo &ti,
+                                                   unsigned char *smem, const BlockLds<float> &b,
+                                                   int x, int y) {
+  float2 *uv = reinterpret_cast<float2 *>(smem + 16 * (size_t)kFluxSlots);
+  float2 *rp = uv + kViscCells, *in = rp + kViscCells;
+  const ViscPhys<float, 2> vp = visc_phys<float, 2>(a, ti.blk);
+  const unsigned i = threadIdx.x;
+  int hc = 0;
+  if ((int)i < kHaloC) hc = (a.halo + ti.halo0)[i];
+  auto put = [&](int p, const F4 &q, float n) {
+    uv[p] = make_float2(q.y, q.z);
+    rp[p] = make_float2(q.x, q.w);
+    in[p] = make_float2(f_rcp(q.x * vp.Rg), n);
+  };
+  const F4 q = (a.W.a + ti.cell0)[i];
+  const float n = a.turb ? (a.nu + ti.cell0)[i] : 0.0f;
+  if ((int)i < kHaloC) {
+    const F4 qh = a.W.a[hc];
+    const float nh = a.turb ? a.nu[hc] : 0.0f;
+    int hx, hy;
+    halo_xy((int)i, hx, hy);
+    put(visc_pos(hx, hy), qh, nh);
+  }
+  const int p0 = visc_pos(x, y);
+  put(p0, q, n);
+  __syncthreads();
+  block_faces(x, y, [&](auto dc, int dir, int fx, int fy) {
+    constexpr int d = decltype(dc)::value;
+    const int p = d >= 0 ? p0 : visc_pos(fx, fy);
+    const int st = dir == 0 ? 1 : kViscP, tt = dir == 0 ? kViscP : 1;
+    const int l = p - st;
+    const int tp[4] = {l + tt, p + tt, l - tt, p - tt};
+    float tu[4], tv[4], out[4], mf = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) { const float2 v = uv[tp[k]]; tu[k] = v.x; tv[k] = v.y; }
+    const float2 vl = uv[l], vr = uv[p], sl = rp[l], sr = rp[p], il = in[l], ir = in[p];
+    visc_flux_2d<d>(Prim<float, 2>{sl.x, vl.x, vl.y, 0.0f, sl.y},
+                    Prim<float, 2>{sr.x, vr.x, vr.y, 0.0f, sr.y}, il.x, ir.x, tu, tv, dir, vp, out,
+                    a.turb, il.y, ir.y, &mf);
+    (dir == 0 ? b.fx : b.fy)[fy * kBoxP + fx] = F4{mf, out[1], out[2], out[3]};
+  });
+}
+
 // The viscous pass of a block tile (visc_prep_tile's work).
 template <typename R>
 __device__ __forceinline__ void visc_prep_block(const ViscArgs<R, 2> &a, const TileInfo &ti,
@@ -418,11 +461,17 @@ __device__ __forceinline__ void visc_prep_block(const ViscArgs<R, 2> &a, const T
   auto &bi = uni(a.blk)[ti.blk];
   auto &P = uni(a.phys)[bi.case_id];
   const BlockLds<R> b = block_lds<R>(smem_raw, a.turb);
-  const int p = block_cell();
+  int x, y;
+  blk_xy(threadIdx.x, x, y);
+  const int p = box_pos(x, y);
   if (a.viscous) {
-    block_load<R, true>(a.W, a.nu, a.turb, a.halo, ti, kHaloC, (R)P.Rg, b, p);
-    __syncthreads();
-    block_visc_faces<R>(b, visc_phys<R, 2>(a, ti.blk), a.turb, p);
+    if constexpr (sizeof(R) == 4) {
+      block_visc_faces32(a, ti, smem_raw, b, x, y);
+    } else {
+      block_load<R, true>(a.W, a.nu, a.turb, a.halo, ti, kHaloC, P.Rg, b, p);
+      __syncthreads();
+      block_visc_faces<R>(b, visc_phys<R, 2>(a, ti.blk), a.turb, p);
+    }
   }
   if (threadIdx.x == 0) *halt = herr ? 1 : 0;
   __syncthreads();
