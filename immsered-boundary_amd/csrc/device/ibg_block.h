@@ -18,14 +18,14 @@
 // learned closure's 97 -> 87 us), k_visc_prep FP32 66 -> 43 us (30 with the
 // layout below).  3D, 2.7M
 // cells: k_stage FP32 147 -> 124 us, FP64 300 -> 294 us, k_visc_prep FP32
-// 172 -> 75 us, FP64 321 -> 179 us.  The FP32 stages then issue vector
+// 172 -> 74 us, FP64 321 -> 148 us.  The FP32 stages then issue vector
 // instructions for 77 % (3D) to 92 % (2D) of their time (2D: the bytes alone
 // would take 36 us at the copy rate), the FP64 ones for 65 to 77 %.  So the
 // code spends them sparingly: the limiters without branches (2D), one
 // position per thread for every phase, the last column's and row's faces in
 // one pass, FP32 constants from a table (Flow32), uniform bases with 32-bit
 // offsets.  With those and leaner FP64 arithmetic the 2D stages take 53 us
-// (FP32), 81 (learned closure) and 111 (FP64), the 3D ones 122 and 236.
+// (FP32), 81 (learned closure) and 106 (FP64), the 3D ones 122 and 229.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -101,17 +101,25 @@ __host__ __device__ constexpr size_t blk_smem(size_t rsize, bool turb, bool temp
 
 // ------------------------------------------------------------------- 3D
 // 8 x 8 x 4 cells (x, y, z), Morton order x lowest.  LDS records of the stage
-// kernel: the four planes as 12 x 12 boxes (x and y halos in place, plane
-// pitch 152), then the halo planes z = -1, 4, -2, 5 of 8 x 8 cells; the
-// working variable stops before the last two.  The viscous pass keeps the
-// 10 x 10 x 6 box of the first halo layer.  Both pitches put the 4 x 2 x 2
-// cells of 16 consecutive lanes on (nearly) distinct bank groups.  The face
-// fluxes of one direction at a time: with all three the LDS would hold two
-// workgroups less per CU.
+// kernel: the four planes as 12 x 12 boxes (x and y halos in place), then
+// the halo planes z = -1, 4, -2, 5 of 8 x 8 cells; the working variable stops
+// before the last two.  The viscous pass keeps the 10 x 10 x 6 box of the
+// first halo layer.  The face fluxes of one direction at a time: with all
+// three the LDS would hold two workgroups less per CU.
+//
+// Pitches and slots by the bank rule of 16-byte reads, as measured: the LDS
+// serves 16 lanes at a time, lanes 0-3, 12-15, 20-23 and 24-27, then the other
+// half of the 32; they must differ in the record's address modulo 16 (x bit 0,
+// y bit 0 and pairs of z bit 0, x bit 1, y bit 1 of the Morton order).  Both
+// boxes and the three flux layouts satisfy it: 5 cycles per read of 64 lanes;
+// 8 and 12 with the box pitches 12 / 152 and 10 / 100 and fluxes at 9 / 76.
+// FP64 records are two planes of 16-byte halves.  k_visc_prep FP64 179 -> 148
+// us, k_stage FP64 236 -> 229 (2D FP64, for the halves alone, 111 -> 106); in
+// FP32 the reads were not what bounds.
 constexpr int kB3X = 8, kB3Y = 8, kB3Z = 4;
-constexpr int kBox3Plane = 152, kBox3Halo = 4 * kBox3Plane;
+constexpr int kBox3Plane = 144, kBox3Halo = 4 * kBox3Plane;
 constexpr int kBox3Cells = kBox3Halo + 4 * 64, kBox3Nu = kBox3Halo + 2 * 64;
-constexpr int kVBox3P = 10, kVBox3Plane = 100, kVBox3Cells = 6 * kVBox3Plane;
+constexpr int kVBox3P = 12, kVBox3Plane = 128, kVBox3Cells = 6 * kVBox3Plane;
 constexpr int kFlux3 = 320;
 // halo list: layer 1 (x, y, z; low then high side), the edges of the first
 // layer (xy, xz, yz; low/low, high/low, low/high, high/high), layer 2
@@ -157,12 +165,11 @@ __host__ __device__ inline int box3_pos(int x, int y, int z) {
 __host__ __device__ constexpr int vbox3_pos(int x, int y, int z) {
   return (z + 1) * kVBox3Plane + (y + 1) * kVBox3P + x + 1;
 }
-// flux slot of the low face of cell (x, y, z) in direction d and the step to
-// the next face
+// flux slot of the low face of cell (x, y, z) in direction d
 __host__ __device__ constexpr int flux3_slot(int d, int x, int y, int z) {
-  return d == 0 ? x + 9 * y + 76 * z : (d == 1 ? x + 8 * y + 76 * z : x + 8 * y + 64 * z);
+  return d == 0 ? 32 * x + ((y + 8 * z) ^ ((x & 1) << 2))
+                : (d == 1 ? x + 8 * y + 76 * z : 64 * z + ((x + 8 * y) ^ ((z & 1) << 2)));
 }
-__host__ __device__ constexpr int flux3_step(int d) { return d == 0 ? 1 : (d == 1 ? 8 : 64); }
 
 __host__ __device__ constexpr size_t blk3_state_offset(size_t rsize) { return 5 * rsize * kFlux3; }
 __host__ __device__ constexpr size_t blk3_smem(size_t rsize, bool turb) {

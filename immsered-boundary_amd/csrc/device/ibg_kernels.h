@@ -279,20 +279,54 @@ __device__ __forceinline__ void visc_prep_tile(const ViscArgs<R, D> &a, const Ti
 
 // ---------------------------------------------------------- block tiles
 // The LDS of a block tile (ibg_block.h).
+// n 4-vectors in LDS: FP32 whole, FP64 as two planes of 16-byte halves (a
+// 32-byte stride would leave every second group of four banks idle).
+template <typename R>
+struct LdsVec {
+  using V = typename V4<R>::T;
+  V *q;
+  __device__ __forceinline__ V operator[](int p) const { return q[p]; }
+  __device__ __forceinline__ void put(int p, const V &v) const { q[p] = v; }
+  __device__ __forceinline__ LdsVec from(int p) const { return LdsVec{q + p}; }
+};
+template <>
+struct LdsVec<double> {
+  using V = D4;
+  double2 *a, *b;
+  __device__ __forceinline__ D4 operator[](int p) const {
+    const double2 x = a[p], y = b[p];
+    return D4{x.x, x.y, y.x, y.y};
+  }
+  __device__ __forceinline__ void put(int p, const D4 &v) const {
+    a[p] = make_double2(v.x, v.y);
+    b[p] = make_double2(v.z, v.w);
+  }
+  __device__ __forceinline__ LdsVec from(int p) const { return LdsVec{a + p, b + p}; }
+};
+template <typename R>
+__device__ __forceinline__ LdsVec<R> lds_vec(unsigned char *smem, int n) {
+  if constexpr (sizeof(R) == 4) {
+    return LdsVec<R>{reinterpret_cast<typename V4<R>::T *>(smem)};
+  } else {
+    double2 *h = reinterpret_cast<double2 *>(smem);
+    return LdsVec<R>{h, h + n};
+  }
+}
 template <typename R>
 struct BlockLds {
-  typename V4<R>::T *fx, *fy;   // fluxes of the x and y faces
-  typename V4<R>::T *S;         // states of the box
+  LdsVec<R> fx, fy;             // fluxes of the x and y faces
+  LdsVec<R> S;                  // states of the box
   R *nu, *T;                    // working variable (SA); temperature for the
                                 // viscous flux (FP64)
 };
 template <typename R>
 __device__ __forceinline__ BlockLds<R> block_lds(unsigned char *smem, bool turb) {
   BlockLds<R> b;
-  b.fx = reinterpret_cast<typename V4<R>::T *>(smem);
-  b.fy = b.fx + kFxSlots;
-  b.S = b.fx + kFluxSlots;
-  b.nu = reinterpret_cast<R *>(b.S + kBoxCells);
+  b.fx = lds_vec<R>(smem, kFluxSlots);
+  b.fy = b.fx.from(kFxSlots);
+  unsigned char *st = smem + blk_state_offset(sizeof(R));
+  b.S = lds_vec<R>(st, kBoxCells);
+  b.nu = reinterpret_cast<R *>(st + 4 * sizeof(R) * kBoxCells);
   b.T = b.nu + (turb ? kBoxCells : 0);
   return b;
 }
@@ -314,7 +348,7 @@ __device__ __forceinline__ void block_load(const Pack<R, 2> &W, const R *nu, boo
   if ((int)i < nhalo) hc = (halo + ti.halo0)[i];
   auto put = [&](int p, const typename V4<R>::T &q, R n) {
     if constexpr (kT) b.T[p] = v_div(q.w, q.x * Rg);
-    b.S[p] = q;
+    b.S.put(p, q);
     if (turb) b.nu[p] = n;
   };
   const typename V4<R>::T q = (W.a + ti.cell0)[i];
@@ -378,7 +412,7 @@ __device__ __forceinline__ void block_visc_faces(const BlockLds<R> &b, const Vis
     visc_flux<R, 2>(cell(l), cell(p), b.S[l].x, b.S[p].x, t, dir, vp, out, turb, nl, nr, &mf);
     typename V4<R>::T o;
     o.x = mf; o.y = out[1]; o.z = out[2]; o.w = out[3];
-    (dir == 0 ? b.fx : b.fy)[p - box_pos(0, 0)] = o;
+    b.fx.put(p - box_pos(0, 0) + (dir == 0 ? 0 : kFxSlots), o);
   });
 }
 
@@ -450,7 +484,7 @@ __device__ __forceinline__ void block_visc_faces32(const ViscArgs<float, 2> &a, 
     visc_flux_2d<d>(Prim<float, 2>{sl.x, vl.x, vl.y, 0.0f, sl.y},
                     Prim<float, 2>{sr.x, vr.x, vr.y, 0.0f, sr.y}, il.x, ir.x, tu, tv, dir, vp, out,
                     a.turb, il.y, ir.y, &mf);
-    (dir == 0 ? b.fx : b.fy)[fy * kBoxP + fx] = F4{mf, out[1], out[2], out[3]};
+    b.fx.put(fy * kBoxP + fx + (dir == 0 ? 0 : kFxSlots), F4{mf, out[1], out[2], out[3]});
   });
 }
 
@@ -482,18 +516,19 @@ __device__ __forceinline__ void visc_prep_block(const ViscArgs<R, 2> &a, const T
 // ---- 3D
 template <typename R>
 struct Block3Lds {
-  typename V4<R>::T *F;   // fluxes of one direction: values 0..3
+  LdsVec<R> F;            // fluxes of one direction: values 0..3
   R *Fe;                  // value 4
-  typename V4<R>::T *S;   // states (roe, u, v, w)
+  LdsVec<R> S;            // states (roe, u, v, w)
   R *e, *nu;              // pressure (viscous pass, FP64: temperature); SA
 };
 template <typename R>
 __device__ __forceinline__ Block3Lds<R> block3_lds(unsigned char *smem, int cells) {
   Block3Lds<R> b;
-  b.F = reinterpret_cast<typename V4<R>::T *>(smem);
-  b.Fe = reinterpret_cast<R *>(b.F + kFlux3);
-  b.S = reinterpret_cast<typename V4<R>::T *>(smem + blk3_state_offset(sizeof(R)));
-  b.e = reinterpret_cast<R *>(b.S + cells);
+  b.F = lds_vec<R>(smem, kFlux3);
+  b.Fe = reinterpret_cast<R *>(smem + 4 * sizeof(R) * kFlux3);
+  unsigned char *st = smem + blk3_state_offset(sizeof(R));
+  b.S = lds_vec<R>(st, cells);
+  b.e = reinterpret_cast<R *>(st + 4 * sizeof(R) * cells);
   b.nu = b.e + cells;
   return b;
 }
@@ -517,7 +552,7 @@ __device__ __forceinline__ void block3_load(const Pack<R, 3> &W, const R *nu, bo
   const int c1 = has1 ? halo[ti.halo0 + h1] : 0;
   auto put = [&](int x, int y, int z, const typename V4<R>::T &q, R p, bool n, R nv) {
     const int k = VISC ? vbox3_pos(x, y, z) : box3_pos(x, y, z);
-    b.S[k] = q;
+    b.S.put(k, q);
     b.e[k] = (VISC && sizeof(R) == 8) ? v_div(p, q.x * Rg) : p;
     if (n) b.nu[k] = nv;
   };
@@ -601,11 +636,11 @@ __device__ __forceinline__ void visc_prep_block3(const ViscArgs<R, 3> &a, const 
         V o;
         o.x = mf; o.y = out[1]; o.z = out[2]; o.w = out[3];
         const int k = flux3_slot(d, x, y, z);
-        b.F[k] = o;
+        b.F.put(k, o);
         b.Fe[k] = out[4];
       }
       __syncthreads();
-      const int k = flux3_slot(d, cx, cy, cz), h = k + flux3_step(d);
+      const int k = flux3_slot(d, cx, cy, cz), h = flux3_slot(d, cx + (d == 0), cy + (d == 1), cz + (d == 2));
       const V lo = b.F[k], hi = b.F[h];
       s[1] += (double)hi.y - (double)lo.y;
       s[2] += (double)hi.z - (double)lo.z;
@@ -919,13 +954,13 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
         V o;
         o.x = flux[0]; o.y = flux[1]; o.z = flux[2]; o.w = flux[3];
         const int k = flux3_slot(d, x, y, z);
-        b3.F[k] = o;
+        b3.F.put(k, o);
         b3.Fe[k] = flux[4];
       }
       __syncthreads();
       int x, y, z;
       blk_xyz(threadIdx.x, x, y, z);
-      const int k = flux3_slot(d, x, y, z), h = k + flux3_step(d);
+      const int k = flux3_slot(d, x, y, z), h = flux3_slot(d, x + (d == 0), y + (d == 1), z + (d == 2));
       const V lo = b3.F[k], hi = b3.F[h];
       s[0] += (double)lo.x - (double)hi.x;
       s[1] += (double)lo.y - (double)hi.y;
@@ -968,7 +1003,7 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
                              box_prim<R>(bl, p + st), dir, dir == 0 ? ar0 : ar1, ph, a.limiter, flux);
       V o;
       o.x = flux[0]; o.y = flux[1]; o.z = flux[2]; o.w = flux[3];
-      (dir == 0 ? bl.fx : bl.fy)[p - box_pos(0, 0)] = o;
+      bl.fx.put(p - box_pos(0, 0) + (dir == 0 ? 0 : kFxSlots), o);
     });
   } else {
     if constexpr (kFuseVisc<R, D>) {
@@ -1401,7 +1436,7 @@ __global__ void __launch_bounds__(kTile, (P ? 1 : kStageWaves<R, D>)) k_stage(St
 // to scratch and the launch takes 112 instead of 93 us on the 2.6M-cell
 // NACA0015 case).
 template <int D, bool P = false>
-__global__ void __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(7, 8)))
+__global__ void __launch_bounds__(kTile) __attribute__((amdgpu_waves_per_eu(P ? 4 : 7, 8)))
 k_stage_ml(StageArgs<float, D> a) {
   stage_launch<float, D, true, P>(a);
 }
