@@ -1426,8 +1426,16 @@ __device__ __forceinline__ void stage_launch(const StageArgs<R, D> &a) {
 template <typename R, int D>
 constexpr int kStageWaves = sizeof(R) == 4 ? (D == 2 ? 8 : 6) : (D == 2 ? 4 : 3);
 
+// The persistent variants: what the loop keeps live across its tiles costs
+// them registers, and held to more waves they spill and lose (3D FP32 9.7 ms a
+// march of 32 steps at two waves, 7.9 at three, 10.5 at five; 3D FP64 18.5 at
+// one, 14.5 at two).
+template <typename R, int D>
+constexpr int kPersistWaves = sizeof(R) == 4 ? (D == 2 ? 4 : 3) : 2;
+
 template <typename R, int D, bool ML, bool P = false>
-__global__ void __launch_bounds__(kTile, (P ? 1 : kStageWaves<R, D>)) k_stage(StageArgs<R, D> a) {
+__global__ void __launch_bounds__(kTile, (P ? kPersistWaves<R, D> : kStageWaves<R, D>))
+k_stage(StageArgs<R, D> a) {
   stage_launch<R, D, ML, P>(a);
 }
 
