@@ -278,10 +278,11 @@ __device__ __forceinline__ float fast_albada(float num, float den) {
   if (!(r <= 1.0e10f)) r = (num > 0.0f) ? 1000000.0f : 0.0f;   // also NaN / inf
   return fmaf(r, r, r) * f_rcp(fmaf(r, r, 1.0f));
 }
-// The same without branches, for the 2D block tiles: a wave's lanes mostly
-// have both signs, so the branches only cost (stage 60.6 -> 56.4 us on the
-// 2.6M-cell section).  In 3D the extra live values spill (123.5 -> 126 us),
-// and in general tiles they cost the learned closure its occupancy.
+// The same without branches, for the block tiles: a wave's lanes mostly have
+// both signs, so the branches only cost (stage 60.6 -> 56.4 us on the
+// 2.6M-cell section; 3D 117 -> 111.5, once its residual sums leave the
+// registers for it).  In general tiles the extra live values cost the learned
+// closure its occupancy.
 template <bool kLeft, bool ALBADA>
 __device__ __forceinline__ float flat_slope(float q, float a, float b) {
 #pragma clang fp contract(off)
@@ -304,7 +305,7 @@ __device__ __forceinline__ float fast_slope(float q, float a, float b, int lim) 
 // round alike: the terms that a known direction drops are exact zeros and
 // products with one.
 // FLAT: the limiter without branches.
-template <int D, int DIR = -1, bool FLAT = (D == 2 && DIR >= 0)>
+template <int D, int DIR = -1, bool FLAT = false>
 __device__ __forceinline__ void roe_flux(const Prim<float, D> &t0, const Prim<float, D> &t1,
                                          const Prim<float, D> &t2, const Prim<float, D> &t3,
                                          int dir, float area, const PhysR<float> &ph, int lim,
