@@ -50,7 +50,7 @@ HBM_PEAK_GBS = 8000.0   # MI355X HBM3E
 # timed steps), as recorded with the traffic profile of this workload; update it
 # with the kernel.  FETCH_SIZE counts what the L2s fetch from the fabric,
 # last-level-cache (MALL) hits included, so it bounds the HBM bytes from above.
-TRAFFIC_BYTES_PER_CELL = 198.3
+TRAFFIC_BYTES_PER_CELL = 147.8
 
 
 def stage_bytes(mode, dim, turb, cells, faces, last=False, first=False):
@@ -62,8 +62,8 @@ def stage_bytes(mode, dim, turb, cells, faces, last=False, first=False):
     with the SA closure the working variable read and written, its FP64
     master (the old value), the frozen face term and the wall distance
     (FP32 in the mixed mode).  The last stage of a step in mixed mode also
-    writes the FP64 masters.  Per tile face the 4 stencil indices and the
-    direction byte.  The first stage of a 2D FP64 step also computes the
+    writes the FP64 masters.  Per face of a face list (`faces`; a block tile
+    has none) the 4 stencil indices and the direction byte.  The first stage of a 2D FP64 step also computes the
     frozen viscous residual and face term: it writes them instead of reading
     them (same bytes) and reads the tangential viscous stencil (16 B per
     face).
@@ -77,6 +77,15 @@ def stage_bytes(mode, dim, turb, cells, faces, last=False, first=False):
         per_cell += nv * 8 + (8 if turb else 0)
     per_face = 17 + (16 if first and dim == 2 and mode == "fp64" else 0)
     return cells * per_cell + faces * per_face
+
+
+def block_bytes_saved(dim, cells, faces):
+    """Bytes that stage_bytes counts too many for the cells of block tiles:
+    they read the tile's halo list (132 or 592 indices per 256 cells) instead
+    of their face slots.  A face list holds at least `dim` faces per cell of
+    its tiles, so at least cells - faces / dim cells are in block tiles."""
+    halo = {2: 132, 3: 592}[dim] * 4 / 256
+    return max(0.0, cells - faces / dim) * (2 * dim * 2 - halo)
 
 
 def stage_mix(eng, mesh, mode, ts0, nsteps, nstage, reps):
@@ -95,7 +104,8 @@ def stage_mix(eng, mesh, mode, ts0, nsteps, nstage, reps):
         for k in range(nstage):
             ms, nc, nf = eng.bench_stage(ts, k, reps)
             ms_sum += w * ms
-            by_sum += w * stage_bytes(mode, mesh.dim, True, nc, nf, last=(k == nstage - 1), first=(k == 0))
+            by_sum += w * (stage_bytes(mode, mesh.dim, True, nc, nf, last=(k == nstage - 1), first=(k == 0))
+                           - block_bytes_saved(mesh.dim, nc, nf))
             c_sum += w * nc
             n += w
     return ms_sum / n, by_sum / n, c_sum / n

@@ -1432,9 +1432,9 @@ template <typename R, int D>
 constexpr int kStageWaves = sizeof(R) == 4 ? (D == 2 ? 8 : 6) : (D == 2 ? 4 : 3);
 
 // The persistent variants: what the loop keeps live across its tiles costs
-// them registers, and held to more waves they spill and lose (3D FP32 9.7 ms a
-// march of 32 steps at two waves, 7.9 at three, 10.5 at five; 3D FP64 18.5 at
-// one, 14.5 at two).
+// them registers, and held to more waves they spill and lose (0.9M cells in
+// 3D, a march of 32 steps: FP32 9.7 ms at two waves, 7.9 at three, 10.5 at
+// five; FP64 18.5 at one, 14.5 at two).
 template <typename R, int D>
 constexpr int kPersistWaves = sizeof(R) == 4 ? (D == 2 ? 4 : 3) : 2;
 
@@ -1593,7 +1593,7 @@ __global__ void k_restrict(int n, const int2 *cc, const int4 *fi, StateOut<D> o,
 // +-1/4 (fincrem); the SA variant (:91-127) does the same for the working
 // variable.  One thread per son; cc: (coarse cell, case), nb[6][stride]: the
 // cell's neighbours x low, x high, y, z, both listed per pair.  For the 4.4K
-// pairs of a level of the moving section 10.5 -> 6.5 us (one thread per
+// pairs of a level of the moving section 10.5 -> 4.5 us (one thread per
 // pair, the neighbours from the cell's row of 27).
 template <int D>
 __global__ void k_prolong(int n, const int2 *cc, const int *fi, const int *nb, int stride,
