@@ -50,7 +50,7 @@ HBM_PEAK_GBS = 8000.0   # MI355X HBM3E
 # timed steps), as recorded with the traffic profile of this workload; update it
 # with the kernel.  FETCH_SIZE counts what the L2s fetch from the fabric,
 # last-level-cache (MALL) hits included, so it bounds the HBM bytes from above.
-TRAFFIC_BYTES_PER_CELL = 147.8
+TRAFFIC_BYTES_PER_CELL = 147.9
 
 
 def stage_bytes(mode, dim, turb, cells, faces, last=False, first=False):
