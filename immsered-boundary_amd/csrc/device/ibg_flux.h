@@ -86,39 +86,23 @@ struct Prim {
 // Limited half slope 0.5 a phi(r), r = b / a, of SlopeCorrection_Left/Right
 // (Slopelimiter.H:22-58, comptqleft/right NS_Solver.H:21-27): left of a face
 // a = qi - q_i, b = qi1 - qi, added to qi; right of it a = qi1 - qi,
-// b = qi - q_i, subtracted.  With one division, as a product of a weight in
-// [0, 1] and a sum or difference: for a and b of one sign (r > 0)
-//   van Leer   phi = 2r/(1+r):        0.5 a phi = |a| / (|a| + |b|)  b
-//   van Albada phi = (r^2+r)/(r^2+1): 0.5 a phi = a b / (a^2 + b^2)  0.5 (a + b)
+// b = qi - q_i, subtracted.  With one division: for r > 0
+//   van Leer   phi = 2r/(1+r):        0.5 a phi = a b / (a + b)
+//   van Albada phi = (r^2+r)/(r^2+1): 0.5 a phi = 0.5 a b (a + b) / (a^2 + b^2)
 // and 0 otherwise (the reference forms r and phi with a division each).
-// No intermediate leaves the range of a normal number, whatever the size of
-// a and b: the front of a disturbance in a uniform stream decays from cell to
-// cell through differences of 1e-100, 1e-200 and less, whose products and
-// square sums are denormal or zero and whose reciprocal is infinite.  So the
-// signs are compared as such, van Leer's divisor has an addend of 2^-1021
-// (lost in rounding above 2^-967), and van Albada's squares are formed of
-// |a| and |b| scaled to at most one by a power of two.
-// A NaN or infinite difference gives NaN.
 // The reference's guard, |r| > 1e10 or NaN: r becomes 1e6 for b > 0, else
 // -1, so phi is 1e6's or 0 whatever the sign of a.
 // fixed_slope is the value where the guard holds.  That needs a jump beside
 // a difference 1e10 times smaller, flow uniform but for rounding: the waves
 // that meet one take a second pass over the limiters (muscl_guarded).
-struct HalfSlope {
-  double w, d;   // the half slope as a product
-};
 template <bool ALBADA>
-__device__ __forceinline__ HalfSlope half_slope(double a, double b) {
-#pragma clang fp contract(off)
-  const bool same = (__double2hiint(a) ^ __double2hiint(b)) >= 0;
-  const double x = r_abs(a), y = r_abs(b);
-  if (ALBADA) {
-    const int k = -__builtin_amdgcn_frexp_exp(x + y);
-    const double u = __builtin_ldexp(x, k), v = __builtin_ldexp(y, k);
-    const double q = n_rcp(fma(u, u, fma(v, v, 0x1p-1000)));
-    return {0.5 * (u * v * q), same ? a + b : 0.0};
-  }
-  return {x * n_rcp(x + (y + 0x1p-1021)), same ? b : 0.0};
+__device__ __forceinline__ double half_slope(double a, double b) {
+  const double pr = a * b;
+  const bool pos = pr > 0.0;
+  double x;
+  if (ALBADA) x = 0.5 * pr * (a + b) * n_rcp(fma(a, a, b * b));
+  else x = pr * n_rcp(a + b);
+  return pos ? x : pr * 0.0;   // 0, or NaN from a NaN or infinite difference
 }
 template <bool ALBADA>
 __device__ __forceinline__ double fixed_slope(double a, double b) {
@@ -132,9 +116,8 @@ template <bool ALBADA>
 __device__ __forceinline__ void muscl(double q0, double q1, double q2, double q3, double &left,
                                       double &right, bool &guard) {
   const double d0 = q1 - q0, d1 = q2 - q1, d2 = q3 - q2;
-  const HalfSlope l = half_slope<ALBADA>(d0, d1), r = half_slope<ALBADA>(d2, d1);
-  left = fma(l.w, l.d, q1);
-  right = fma(-r.w, r.d, q2);
+  left = q1 + half_slope<ALBADA>(d0, d1);
+  right = q2 - half_slope<ALBADA>(d2, d1);
   guard = guard | slope_guard(d0, d1) | slope_guard(d2, d1);
 }
 template <bool ALBADA>
