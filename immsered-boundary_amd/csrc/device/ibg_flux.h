@@ -27,6 +27,7 @@ __device__ __forceinline__ float n_div(float n, float x) { return n * f_rcp(x); 
 // sequence without its range scaling and fixup: the same value in the normal
 // range.
 __device__ __forceinline__ double n_div(double n, double x) {
+#pragma clang fp contract(off)
   double y = __builtin_amdgcn_rcp(x);
   y = fma(fma(-x, y, 1.0), y, y);
   y = fma(fma(-x, y, 1.0), y, y);
@@ -37,16 +38,19 @@ __device__ __forceinline__ double n_div(double n, double x) {
 // v_rsq_f64 are good to 2^-24 (measured on gfx950: 2^-24.4 and 2^-24.2), so
 // one step of third order (e + e^2, e/2 + 3/8 e^2) reaches 2^-72.
 __device__ __forceinline__ double n_rcp(double x) {
+#pragma clang fp contract(off)
   const double y = __builtin_amdgcn_rcp(x);
   const double e = fma(-x, y, 1.0);
   return fma(y, fma(e, e, e), y);
 }
 __device__ __forceinline__ double n_sqrt(double x) {   // x > 0
+#pragma clang fp contract(off)
   const double y = __builtin_amdgcn_rsq(x), g = x * y;
   const double e = fma(-g, y, 1.0);
   return fma(g * e, fma(e, 0.375, 0.5), g);
 }
 __device__ __forceinline__ double n_rsqrt(double x) {   // x > 0
+#pragma clang fp contract(off)
   const double y = __builtin_amdgcn_rsq(x);
   const double e = fma(-x * y, y, 1.0);
   return fma(y * e, fma(e, 0.375, 0.5), y);
@@ -97,6 +101,7 @@ struct Prim {
 // that meet one take a second pass over the limiters (muscl_guarded).
 template <bool ALBADA>
 __device__ __forceinline__ double half_slope(double a, double b) {
+#pragma clang fp contract(off)
   const double pr = a * b;
   const bool pos = pr > 0.0;
   double x;
@@ -106,6 +111,7 @@ __device__ __forceinline__ double half_slope(double a, double b) {
 }
 template <bool ALBADA>
 __device__ __forceinline__ double fixed_slope(double a, double b) {
+#pragma clang fp contract(off)
   const double phi = ALBADA ? (1.0e12 + 1.0e6) / (1.0e12 + 1.0) : 2.0e6 / (1.0 + 1.0e6);
   return (b > 0.0) ? 0.5 * a * phi : 0.0;
 }
@@ -115,6 +121,7 @@ __device__ __forceinline__ bool slope_guard(double a, double b) { return r_abs(b
 template <bool ALBADA>
 __device__ __forceinline__ void muscl(double q0, double q1, double q2, double q3, double &left,
                                       double &right, bool &guard) {
+#pragma clang fp contract(off)
   const double d0 = q1 - q0, d1 = q2 - q1, d2 = q3 - q2;
   left = q1 + half_slope<ALBADA>(d0, d1);
   right = q2 - half_slope<ALBADA>(d2, d1);
@@ -123,6 +130,7 @@ __device__ __forceinline__ void muscl(double q0, double q1, double q2, double q3
 template <bool ALBADA>
 __device__ __forceinline__ void muscl_guarded(double q0, double q1, double q2, double q3,
                                               double &left, double &right) {
+#pragma clang fp contract(off)
   const double d0 = q1 - q0, d1 = q2 - q1, d2 = q3 - q2;
   if (slope_guard(d0, d1)) left = q1 + fixed_slope<ALBADA>(d0, d1);
   if (slope_guard(d2, d1)) right = q2 - fixed_slope<ALBADA>(d2, d1);
@@ -147,11 +155,15 @@ __device__ __forceinline__ void muscl_guarded(double q0, double q1, double q2, d
 // launches go from 134 to 118 us (2D) and from 294 to 242 us (3D, both with
 // block tiles).  Error of the 2D flux against 80-bit arithmetic over jumps of
 // 1e-1 .. 1e-6: rms 0.97e-16 (26-division form 0.98e-16).
+// The fused operations are written out here and in the viscous flux below, so
+// that block and general tiles, whose faces have a known direction or not,
+// round alike and the tile size does not change a bit of the results.
 // Output: (mass, normal, tangential momenta, energy).
 template <int D>
 __device__ __forceinline__ void roe_normal(const Prim<double, D> &t0, const Prim<double, D> &t1,
                                            const Prim<double, D> &t2, const Prim<double, D> &t3, double area,
                                            const PhysR<double> &ph, int lim, double *flux) {
+#pragma clang fp contract(off)
   double lr, rr, lu, ru, lv, rv, lw = 0.0, rw = 0.0, lp, rp;
   auto reconstruct = [&](auto albada) {
     constexpr bool A = decltype(albada)::value;
@@ -173,58 +185,57 @@ __device__ __forceinline__ void roe_normal(const Prim<double, D> &t0, const Prim
   else reconstruct(std::false_type());
   const double ilr = n_rcp(lr);
   const double plr = lp * ilr, prr = rp * n_rcp(rr);
-  const double lke = (D == 3) ? 0.5 * (lu * lu + lv * lv + lw * lw) : 0.5 * (lu * lu + lv * lv);
-  const double rke = (D == 3) ? 0.5 * (ru * ru + rv * rv + rw * rw) : 0.5 * (ru * ru + rv * rv);
-  const double hl = ph.cpR * plr + lke, hr = ph.cpR * prr + rke;
-  // central part 1/2 (F_L + F_R) A
+  double lq = fma(lu, lu, lv * lv), rq = fma(ru, ru, rv * rv);
+  if (D == 3) { lq = fma(lw, lw, lq); rq = fma(rw, rw, rq); }
+  const double hl = fma(ph.cpR, plr, 0.5 * lq), hr = fma(ph.cpR, prr, 0.5 * rq);
+  // central part 1/2 (F_L + F_R) A, without the factor A/2
   const double ml = lr * lu, mr = rr * ru;
   const double ha = 0.5 * area;
-  const double c0 = (ml + mr) * ha;
-  const double c1 = ((ml * lu + lp) + (mr * ru + rp)) * ha;
-  const double c2 = (ml * lv + mr * rv) * ha;
-  const double c4 = (ml * hl + mr * hr) * ha;
+  const double c0 = fma(lr, lu, mr);
+  const double c1 = fma(ml, lu, lp) + fma(mr, ru, rp);
+  const double c2 = fma(ml, lv, mr * rv);
+  const double c4 = fma(ml, hl, mr * hr);
   const double droe = rr - lr, dp = rp - lp, dubar = ru - lu;
   // Roe average: sqrt(rr / lr) = sqrt(lr rr) / lr
   const double a_roe = n_sqrt(lr * rr);
   const double q = a_roe * ilr;
   const double wl = n_rcp(1.0 + q);
-  const double a_u = (lu + ru * q) * wl;
-  const double a_v = (lv + rv * q) * wl;
-  const double a_w = (D == 3) ? (lw + rw * q) * wl : 0.0;
-  const double a_h = (hl + hr * q) * wl;
-  const double q2 = (D == 3) ? (a_u * a_u + a_v * a_v + a_w * a_w) : (a_u * a_u + a_v * a_v);
-  const double csq = ph.gm1 * (a_h - 0.5 * q2);
+  const double a_u = fma(ru, q, lu) * wl;
+  const double a_v = fma(rv, q, lv) * wl;
+  const double a_w = (D == 3) ? fma(rw, q, lw) * wl : 0.0;
+  const double a_h = fma(hr, q, hl) * wl;
+  double q2 = fma(a_u, a_u, a_v * a_v);
+  if (D == 3) q2 = fma(a_w, a_w, q2);
+  const double csq = ph.gm1 * fma(-0.5, q2, a_h);
   const double a_c = n_sqrt(csq);
   const double icsq = n_rcp(csq);
   const double faa = area * r_abs(a_u);
-  const double coef12 = ha * icsq;
-  const double rcu = a_roe * a_c * dubar;
-  const double al0 = faa * (droe - dp * icsq);
+  const double coef12 = (0.5 * ha) * icsq;   // times 2 n1, 2 n2
+  const double rc = a_roe * a_c;
+  const double al0 = faa * fma(-dp, icsq, droe);
   // all-speed eigenvalues (NS_Solver.H:66-77): f = min(max(Ma_face, Ma_inf), 1)
   double f = r_abs((lu + ru) * 0.5) * n_rsqrt(ph.gama * ((plr + prr) * 0.5));
   f = f < ph.Ma ? ph.Ma : f;
   f = f > 1.0 ? 1.0 : f;
-  const double s0 = (1.0 - f) * (1.0 - f);
-  const double n0 = n_sqrt(4.0 * csq * f + s0 * a_u * a_u);
-  const double n1 = r_abs(0.5 * ((1.0 + f) * a_u + n0));
-  const double n2 = r_abs(0.5 * ((1.0 + f) * a_u - n0));
-  const double al1 = coef12 * n1 * (dp + rcu);
-  const double al2 = coef12 * n2 * (dp - rcu);
-  const double al3 = al0 + al1 + al2;
-  const double al4 = a_c * (al1 - al2);
+  const double g = (1.0 - f) * a_u, f1 = 1.0 + f;
+  const double n0 = n_sqrt(fma(4.0 * csq, f, g * g));
+  const double n1 = coef12 * r_abs(fma(f1, a_u, n0));
+  const double n2 = coef12 * r_abs(fma(f1, a_u, -n0));
+  const double x1 = fma(rc, dubar, dp), x2 = fma(-rc, dubar, dp);
+  const double al3 = fma(n2, x2, fma(n1, x1, al0));
+  const double al4 = a_c * fma(n1, x1, -(n2 * x2));
   const double fr = faa * a_roe;
   const double al6 = fr * (rv - lv);
   const double al7 = (D == 3) ? fr * (rw - lw) : 0.0;
-  flux[0] = c0 - al3;
-  flux[1] = c1 - (a_u * al3 + al4);
-  flux[2] = c2 - (a_v * al3 + al6);
-  if (D == 3) {
-    const double c3 = (ml * lw + mr * rw) * ha;
-    flux[3] = c3 - (a_w * al3 + al7);
-    flux[4] = c4 - (a_h * al3 + a_u * al4 + a_v * al6 + a_w * al7 - csq * ph.ig1 * al0);
-  } else {
-    flux[3] = c4 - (a_h * al3 + a_u * al4 + a_v * al6 - csq * ph.ig1 * al0);
-  }
+  flux[0] = fma(c0, ha, -al3);
+  flux[1] = fma(c1, ha, -fma(a_u, al3, al4));
+  flux[2] = fma(c2, ha, -fma(a_v, al3, al6));
+  double en = fma(a_h, al3, a_u * al4);
+  en = fma(a_v, al6, en);
+  if (D == 3) en = fma(a_w, al7, en);
+  en = fma(-(csq * ph.ig1), al0, en);
+  if (D == 3) flux[3] = fma(fma(ml, lw, mr * rw), ha, -fma(a_w, al3, al7));
+  flux[D == 3 ? 4 : 3] = fma(c4, ha, -en);
 }
 
 // Into and out of the frame of a face of direction dir: the normal velocity
@@ -438,10 +449,9 @@ struct ViscPhys {
   R ar0, ar1, ar2;   // face areas
   R iqkt;            // 1 / (Re*Pr_tur*(gama-1)*Ma^2) (SA closure)
 };
-// reciprocal of a constant divisor of the viscous terms: the hardware's in
-// FP32, as every quotient of that mode
+// reciprocal of a constant divisor of the FP32 viscous terms: the hardware's,
+// as every quotient of that mode
 __device__ __forceinline__ float c_rcp(float x) { return f_rcp(x); }
-__device__ __forceinline__ double c_rcp(double x) { return 1.0 / x; }
 
 // Spalart-Allmaras constants, Turbulence.cpp:3-19
 struct SA {
@@ -495,31 +505,24 @@ __device__ __forceinline__ double sa_r(double nu, double sd2, const SaPhys<doubl
 }
 
 // Viseddy2mut (Turbulence.cpp:23-30): mu_t = roe fv1 nu, X = nu/(mu/roe)
-// clamped at 0, fv1 = X^3/(X^3 + cv1^3).
-template <typename R>
-__device__ __forceinline__ R sa_mut(R nu, R roe, R mu) {
-  R bigx = v_div(nu, v_div(mu, roe));
-  if (bigx < R(0.0)) bigx = R(0.0);
-  const R b3 = bigx * bigx * bigx;
-  const R fv1 = v_div(b3, b3 + R(SA::cv1three));
+// clamped at 0, fv1 = X^3/(X^3 + cv1^3).  nul = mu/roe.
+__device__ __forceinline__ double sa_mut(double nu, double roe, double nul) {
+#pragma clang fp contract(off)
+  double bigx = v_div(nu, nul);
+  if (bigx < 0.0) bigx = 0.0;
+  const double b2 = bigx * bigx;
+  const double fv1 = v_div(b2 * bigx, fma(b2, bigx, SA::cv1three));
   return roe * fv1 * nu;
-}
-
-// four-point tangential difference pfpkesai1 (NS_Solver.H:153-154)
-template <typename R>
-__device__ __forceinline__ R pf1(R up1, R up2, R dn1, R dn2) {
-  return R(0.25) * (up1 + up2 - dn1 - dn2);
 }
 
 // Velocity and temperature of a viscous stencil cell, T = p/(roe Rg)
 // (Get_T_ideal_gas).
-template <typename R>
 struct VelT {
-  R u, v, w, T;
+  double u, v, w, T;
 };
-template <typename R, int D>
-__device__ __forceinline__ VelT<R> vel_t(const Prim<R, D> &q, R Rg) {
-  return VelT<R>{q.u, q.v, q.w, v_div(q.p, q.r * Rg)};
+template <int D>
+__device__ __forceinline__ VelT vel_t(const Prim<double, D> &q, double Rg) {
+  return VelT{q.u, q.v, q.w, v_div(q.p, q.r * Rg)};
 }
 
 // Viscous face flux of ComptViscousStress (NS_Solver.cpp:426-581, laminar).
@@ -535,89 +538,76 @@ __device__ __forceinline__ VelT<R> vel_t(const Prim<R, D> &q, R Rg) {
 // (nu_f + mu/roe_f) (d nu / d n) / sigma * A (the face keisa is the unit
 // axis, so the dot product picks the normal derivative).  Constant divisors
 // (Re, sigma, 3, Re Pr_t (gama-1) Ma^2) are multiplications.
-template <typename R, int D>
-__device__ __forceinline__ void visc_flux(const VelT<R> &L, const VelT<R> &Rr, R rL, R rR,
-                                          const VelT<R> *t, int d, const ViscPhys<R, D> &vp,
-                                          R *out, bool turb, R nuL, R nuR, R *mflux) {
-  // normal differences (pfpkesai0) and the first tangential axis
-  const R nu = Rr.u - L.u, nv = Rr.v - L.v, nw = Rr.w - L.w, nT = Rr.T - L.T;
-  const R au = pf1(t[0].u, t[1].u, t[2].u, t[3].u);
-  const R av = pf1(t[0].v, t[1].v, t[2].v, t[3].v);
-  const R aw = (D == 3) ? pf1(t[0].w, t[1].w, t[2].w, t[3].w) : R(0);
-  const R aT = pf1(t[0].T, t[1].T, t[2].T, t[3].T);
-  R bu = R(0), bv = R(0), bw = R(0), bT = R(0);
+template <int D>
+__device__ __forceinline__ void visc_flux(const VelT &L, const VelT &Rr, double rL, double rR,
+                                          const VelT *t, int d, const ViscPhys<double, D> &vp,
+                                          double *out, bool turb, double nuL, double nuR,
+                                          double *mflux) {
+#pragma clang fp contract(off)
+  const bool x = d == 0, y = d == 1;
+  auto pf1 = [](double a, double b, double c, double e) { return 0.25 * (a + b - c - e); };
+  // velocity gradients along x, y, z: the normal difference (pfpkesai0) along
+  // d, the tangential ones on the other axes in order (the heat flux is along
+  // the normal)
+  const double n[3] = {Rr.u - L.u, Rr.v - L.v, Rr.w - L.w};
+  const double a[3] = {pf1(t[0].u, t[1].u, t[2].u, t[3].u), pf1(t[0].v, t[1].v, t[2].v, t[3].v),
+                       (D == 3) ? pf1(t[0].w, t[1].w, t[2].w, t[3].w) : 0.0};
+  double b[3] = {0.0, 0.0, 0.0};
   if constexpr (D == 3) {
-    bu = pf1(t[4].u, t[5].u, t[6].u, t[7].u);
-    bv = pf1(t[4].v, t[5].v, t[6].v, t[7].v);
-    bw = pf1(t[4].w, t[5].w, t[6].w, t[7].w);
-    bT = pf1(t[4].T, t[5].T, t[6].T, t[7].T);
+    b[0] = pf1(t[4].u, t[5].u, t[6].u, t[7].u);
+    b[1] = pf1(t[4].v, t[5].v, t[6].v, t[7].v);
+    b[2] = pf1(t[4].w, t[5].w, t[6].w, t[7].w);
   }
-  // gradients in kesai: normal along d, first tangential t1, second t2
-  R gu[3], gv[3], gw[3], gT[3];
-  const int t1 = (d == 0) ? 1 : 0;
-  const int t2 = (d == 2) ? 1 : 2;
+  double gx[3], gy[3], gz[3];
 #pragma unroll
   for (int k = 0; k < 3; ++k) {
-    const bool isn = (k == d), is1 = (k == t1), is2 = (D == 3) && (k == t2);
-    gu[k] = isn ? nu : (is1 ? au : (is2 ? bu : R(0)));
-    gv[k] = isn ? nv : (is1 ? av : (is2 ? bv : R(0)));
-    gw[k] = isn ? nw : (is1 ? aw : (is2 ? bw : R(0)));
-    gT[k] = isn ? nT : (is1 ? aT : (is2 ? bT : R(0)));
+    gx[k] = x ? n[k] : a[k];
+    gy[k] = y ? n[k] : (x ? a[k] : b[k]);
+    gz[k] = (x || y) ? b[k] : n[k];
   }
-  if (D == 2) { gw[0] = gw[1] = gw[2] = R(0); }
-  // VarReflect with keisa = diag(1/dh)
-  const R dux = gu[0] * vp.ih0, duy = gu[1] * vp.ih1, duz = gu[2] * vp.ih2;
-  const R dvx = gv[0] * vp.ih0, dvy = gv[1] * vp.ih1, dvz = gv[2] * vp.ih2;
-  const R dwx = gw[0] * vp.ih0, dwy = gw[1] * vp.ih1, dwz = gw[2] * vp.ih2;
-  const R dTx = gT[0] * vp.ih0, dTy = gT[1] * vp.ih1, dTz = gT[2] * vp.ih2;
-  const R ftemp = (L.T + Rr.T) * R(0.5);
-  R mu0 = v_sqrt(ftemp * ftemp * ftemp) * v_div(R(1.0) + vp.SoT, ftemp + vp.SoT);
-  R qk0 = vp.qk * mu0;
   // (x*1 + 0 + 0 is exact; written as a sum so that no per-lane table is built)
-  const R area = (d == 0 ? R(1) : R(0)) * vp.ar0 + (d == 1 ? R(1) : R(0)) * vp.ar1 +
-                 (d == 2 ? R(1) : R(0)) * vp.ar2;
+  auto axis = [&](double v0, double v1, double v2) {
+    return (x ? 1.0 : 0.0) * v0 + (y ? 1.0 : 0.0) * v1 + ((x || y) ? 0.0 : 1.0) * v2;
+  };
+  const double ih = axis(vp.ih0, vp.ih1, vp.ih2), area = axis(vp.ar0, vp.ar1, vp.ar2);
+  const double ftemp = (L.T + Rr.T) * 0.5;
+  double mu0 = v_sqrt(ftemp * ftemp * ftemp) * v_div(1.0 + vp.SoT, ftemp + vp.SoT);
+  double qk0 = vp.qk * mu0;
   if (turb) {
-    const R ih = (d == 0 ? R(1) : R(0)) * vp.ih0 + (d == 1 ? R(1) : R(0)) * vp.ih1 +
-                 (d == 2 ? R(1) : R(0)) * vp.ih2;
-    const R fvis = (nuL + nuR) * R(0.5);
-    const R froe = (rL + rR) * R(0.5);
-    const R faceroexvis = fvis + v_div(mu0, froe);
-    const R mut0 = sa_mut(fvis, froe, mu0);
+    const double fvis = (nuL + nuR) * 0.5;
+    const double froe = (rL + rR) * 0.5;
+    const double nul = v_div(mu0, froe);
+    const double mut0 = sa_mut(fvis, froe, nul);
     mu0 += mut0;
-    qk0 += mut0 * vp.iqkt;
-    *mflux = (faceroexvis * ((nuR - nuL) * ih)) * c_rcp(R(SA::segma)) * area;
+    qk0 = fma(mut0, vp.iqkt, qk0);
+    *mflux = ((fvis + nul) * ((nuR - nuL) * ih)) * (1.0 / SA::segma) * area;
   }
-  const R divu = (D == 3) ? (dux + dvy + dwz) : (dux + dvy);
-  const R third = c_rcp(R(3.0));
-  const R mur = mu0 * vp.iRe;
-  const R tauxx = R(2.0) * mu0 * (dux - divu * third) * vp.iRe;
-  const R tauyy = R(2.0) * mu0 * (dvy - divu * third) * vp.iRe;
-  const R tauxy = mur * (duy + dvx);
-  const R fu = (L.u + Rr.u) * R(0.5), fv = (L.v + Rr.v) * R(0.5);
+  const double mur = mu0 * vp.iRe;
+  const double dvy = gy[1] * vp.ih1;
+  double divu = fma(gx[0], vp.ih0, dvy);
+  if (D == 3) divu = fma(gz[2], vp.ih2, divu);
+  const double dn = x ? gx[0] * vp.ih0 : (y ? dvy : gz[2] * vp.ih2);
+  const double tnn = 2.0 * mu0 * fma(divu, -1.0 / 3.0, dn) * vp.iRe;
+  const double txy = mur * fma(gy[0], vp.ih1, gx[1] * vp.ih0);
+  const double fu = (L.u + Rr.u) * 0.5, fv = (L.v + Rr.v) * 0.5;
+  double t1, t2, work;
   if (D == 2) {
-    if (d == 0) {
-      const R bx = fu * tauxx + fv * tauxy + qk0 * dTx;
-      out[0] = R(0); out[1] = tauxx * area; out[2] = tauxy * area; out[3] = bx * area;
-    } else {
-      const R by = fu * tauxy + fv * tauyy + qk0 * dTy;
-      out[0] = R(0); out[1] = tauxy * area; out[2] = tauyy * area; out[3] = by * area;
-    }
+    t1 = x ? tnn : txy;
+    t2 = x ? txy : tnn;
+    work = fma(fu, t1, fv * t2);
   } else {
-    const R tauzz = R(2.0) * mu0 * (dwz - divu * third) * vp.iRe;
-    const R tauxz = mur * (duz + dwx);
-    const R tauyz = mur * (dvz + dwy);
-    const R fw = (L.w + Rr.w) * R(0.5);
-    if (d == 0) {
-      const R bx = fu * tauxx + fv * tauxy + fw * tauxz + qk0 * dTx;
-      out[0] = R(0); out[1] = tauxx * area; out[2] = tauxy * area; out[3] = tauxz * area; out[4] = bx * area;
-    } else if (d == 1) {
-      const R by = fu * tauxy + fv * tauyy + fw * tauyz + qk0 * dTy;
-      out[0] = R(0); out[1] = tauxy * area; out[2] = tauyy * area; out[3] = tauyz * area; out[4] = by * area;
-    } else {
-      const R bz = fu * tauxz + fv * tauyz + fw * tauzz + qk0 * dTz;
-      out[0] = R(0); out[1] = tauxz * area; out[2] = tauyz * area; out[3] = tauzz * area; out[4] = bz * area;
-    }
+    const double txz = mur * fma(gz[0], vp.ih2, gx[2] * vp.ih0);
+    const double tyz = mur * fma(gz[1], vp.ih2, gy[2] * vp.ih1);
+    t1 = x ? tnn : (y ? txy : txz);
+    t2 = x ? txy : (y ? tnn : tyz);
+    const double t3 = x ? txz : (y ? tyz : tnn);
+    work = fma((L.w + Rr.w) * 0.5, t3, fma(fu, t1, fv * t2));
+    out[3] = t3 * area;
   }
+  out[0] = 0.0;
+  out[1] = t1 * area;
+  out[2] = t2 * area;
+  out[D == 3 ? 4 : 3] = fma(qk0, (Rr.T - L.T) * ih, work) * area;
 }
 
 // The same in 2D FP32 with its fused operations written out, so that the
@@ -748,11 +738,11 @@ __device__ __forceinline__ void visc_flux_cells(const Prim<R, D> &L, const Prim<
     visc_flux_3d<-1>(L, Rr, f_rcp(L.r * vp.Rg), f_rcp(Rr.r * vp.Rg), t, d, vp, out, turb, nuL, nuR,
                      mflux);
   } else {
-    VelT<R> vt[(D == 3) ? 8 : 4];
+    VelT vt[(D == 3) ? 8 : 4];
 #pragma unroll
-    for (int k = 0; k < ((D == 3) ? 8 : 4); ++k) vt[k] = vel_t<R, D>(t[k], vp.Rg);
-    visc_flux<R, D>(vel_t<R, D>(L, vp.Rg), vel_t<R, D>(Rr, vp.Rg), L.r, Rr.r, vt, d, vp, out, turb,
-                    nuL, nuR, mflux);
+    for (int k = 0; k < ((D == 3) ? 8 : 4); ++k) vt[k] = vel_t<D>(t[k], vp.Rg);
+    visc_flux<D>(vel_t<D>(L, vp.Rg), vel_t<D>(Rr, vp.Rg), L.r, Rr.r, vt, d, vp, out, turb, nuL, nuR,
+                 mflux);
   }
 }
 

@@ -406,10 +406,10 @@ __device__ __forceinline__ void block_visc_faces(const BlockLds<R> &b, const Vis
     const int tp[4] = {l + tt, p + tt, l - tt, p - tt};
     auto cell = [&](int q) {
       const typename V4<R>::T s = b.S[q];
-      return VelT<R>{s.y, s.z, R(0), b.T[q]};
+      return VelT{s.y, s.z, 0.0, b.T[q]};
     };
-    const VelT<R> t[4] = {cell(tp[0]), cell(tp[1]), cell(tp[2]), cell(tp[3])};
-    visc_flux<R, 2>(cell(l), cell(p), b.S[l].x, b.S[p].x, t, dir, vp, out, turb, nl, nr, &mf);
+    const VelT t[4] = {cell(tp[0]), cell(tp[1]), cell(tp[2]), cell(tp[3])};
+    visc_flux<2>(cell(l), cell(p), b.S[l].x, b.S[p].x, t, dir, vp, out, turb, nl, nr, &mf);
     typename V4<R>::T o;
     o.x = mf; o.y = out[1]; o.z = out[2]; o.w = out[3];
     b.fx.put(p - box_pos(0, 0) + (dir == 0 ? 0 : kFxSlots), o);
@@ -631,12 +631,12 @@ __device__ __forceinline__ void visc_prep_block3(const ViscArgs<R, 3> &a, const 
         } else {
           auto cell = [&](int q) {
             const V v = b.S[q];
-            return VelT<R>{v.y, v.z, v.w, b.e[q]};
+            return VelT{v.y, v.z, v.w, b.e[q]};
           };
-          VelT<R> t[8];
+          VelT t[8];
 #pragma unroll
           for (int k = 0; k < 8; ++k) t[k] = cell(tp[k]);
-          visc_flux<R, 3>(cell(l), cell(p), b.S[l].x, b.S[p].x, t, d, vp, out, a.turb, nl, nr, &mf);
+          visc_flux<3>(cell(l), cell(p), b.S[l].x, b.S[p].x, t, d, vp, out, a.turb, nl, nr, &mf);
         }
         V o;
         o.x = mf; o.y = out[1]; o.z = out[2]; o.w = out[3];
@@ -877,6 +877,15 @@ struct StageShared {
   unsigned mlc[2];   // learned closure: network / fallback cells of this tile
   double red[kRpart][kTile / 64];
 };
+
+// |u|^2 (FP64 mode; fused as written in every variant of the tile)
+template <int D>
+__device__ __forceinline__ double sq_speed(double u, double v, double w) {
+#pragma clang fp contract(off)
+  double q = fma(u, u, v * v);
+  if (D == 3) q = fma(w, w, q);
+  return q;
+}
 
 // One tile.  WRES: the network's weights are resident at a.mlw_off
 // (persistent schedule); otherwise the ML instantiation stages them after
@@ -1279,11 +1288,14 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
       double U[NV];
       {
         if constexpr (!kAhead) w0 = pload<double, D>(rebase(a.W64, c0), c);
-        const double ke0 = (D == 3) ? 0.5 * (w0.u * w0.u + w0.v * w0.v + w0.w * w0.w)
-                                    : 0.5 * (w0.u * w0.u + w0.v * w0.v);
         double re0;
-        if constexpr (kMixed) re0 = w0.r * (P.Cv * n_div(w0.p, w0.r * P.Rg) + ke0);
-        else re0 = P.cvR * w0.p + w0.r * ke0;   // roe T = p / Rg
+        if constexpr (kMixed) {
+          const double ke0 = (D == 3) ? 0.5 * (w0.u * w0.u + w0.v * w0.v + w0.w * w0.w)
+                                      : 0.5 * (w0.u * w0.u + w0.v * w0.v);
+          re0 = w0.r * (P.Cv * n_div(w0.p, w0.r * P.Rg) + ke0);
+        } else {
+          re0 = fma(P.cvR, w0.p, w0.r * (0.5 * sq_speed<D>(w0.u, w0.v, w0.w)));   // roe T = p / Rg
+        }
         U[0] = w0.r; U[1] = w0.r * w0.u; U[2] = w0.r * w0.v;
         if (D == 3) { U[3] = w0.r * w0.w; U[4] = re0; } else U[3] = re0;
       }
@@ -1318,8 +1330,8 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
           wu = over_r(U[1]);
           wv = over_r(U[2]);
           if (D == 3) ww = over_r(U[3]);
-          const double ke = (D == 3) ? 0.5 * (wu * wu + wv * wv + ww * ww) : 0.5 * (wu * wu + wv * wv);
-          wp = (U[D == 3 ? 4 : 3] - ke * wr) * (P.gama - 1.0);
+          const double ke = 0.5 * sq_speed<D>(wu, wv, ww);
+          wp = fma(-ke, wr, U[D == 3 ? 4 : 3]) * (P.gama - 1.0);
         }
         // T = p/(roe Rg) < 0  (NS_Solver.cpp:55-66), Rg > 0
         if ((wp < 0.0) != (wr < 0.0)) report_error(a.err, c0 + (int)c, 37);
