@@ -90,24 +90,48 @@ struct Prim {
 // Limited half slope 0.5 a phi(r), r = b / a, of SlopeCorrection_Left/Right
 // (Slopelimiter.H:22-58, comptqleft/right NS_Solver.H:21-27): left of a face
 // a = qi - q_i, b = qi1 - qi, added to qi; right of it a = qi1 - qi,
-// b = qi - q_i, subtracted.  With one division: for r > 0
-//   van Leer   phi = 2r/(1+r):        0.5 a phi = a b / (a + b)
-//   van Albada phi = (r^2+r)/(r^2+1): 0.5 a phi = 0.5 a b (a + b) / (a^2 + b^2)
-// and 0 otherwise (the reference forms r and phi with a division each).
+// b = qi - q_i, subtracted.  With one division, as a product of a weight and
+// b or a + b: for a and b of one sign (r > 0)
+//   van Leer   phi = 2r/(1+r):        0.5 a phi = |a| / (|a| + |b|)  b
+//   van Albada phi = (r^2+r)/(r^2+1): 0.5 a phi = 0.5 |a| |b| / (a^2 + b^2)  (a + b)
+// and 0 otherwise (the reference forms r and phi with a division each): the
+// weight has max(a sign(b), 0) for |a|.
+// No intermediate leaves the range of a normal number, whatever the size of
+// a and b: the front of a disturbance in a uniform stream decays from cell to
+// cell through differences of 1e-100, 1e-200 and less, whose products and
+// square sums are denormal or zero and whose reciprocal is infinite.  So the
+// signs are compared as such, van Leer's divisor has an addend of 2^-1021
+// (lost in rounding above 2^-967), and van Albada's squares are formed of
+// |a| and |b| scaled to at most one by a power of two.
+// A NaN or infinite difference gives NaN.  Van Leer's weight takes no more
+// instructions than the form a b / (a + b), whose product cannot fuse with the
+// cell value (the moving 2D section, 128 steps, 70.8 -> 70.0 ms), van Albada's
+// four more a slope (the mid-size laminar case 5.30 -> 5.33 ms).
 // The reference's guard, |r| > 1e10 or NaN: r becomes 1e6 for b > 0, else
 // -1, so phi is 1e6's or 0 whatever the sign of a.
 // fixed_slope is the value where the guard holds.  That needs a jump beside
 // a difference 1e10 times smaller, flow uniform but for rounding: the waves
 // that meet one take a second pass over the limiters (muscl_guarded).
+struct HalfSlope {
+  double w, d;   // the half slope as a product
+};
+// a sign(b)
+__device__ __forceinline__ double along(double a, double b) {
+  return __hiloint2double(__double2hiint(a) ^ (__double2hiint(b) & (int)0x80000000), __double2loint(a));
+}
+// s = a sign(b) in the place of a
 template <bool ALBADA>
-__device__ __forceinline__ double half_slope(double a, double b) {
+__device__ __forceinline__ HalfSlope half_slope(double s, double b) {
 #pragma clang fp contract(off)
-  const double pr = a * b;
-  const bool pos = pr > 0.0;
-  double x;
-  if (ALBADA) x = 0.5 * pr * (a + b) * n_rcp(fma(a, a, b * b));
-  else x = pr * n_rcp(a + b);
-  return pos ? x : pr * 0.0;   // 0, or NaN from a NaN or infinite difference
+  double m;
+  asm("v_max_f64 %0, %1, 0" : "=v"(m) : "v"(s));   // (fmax would quiet s first; 0 for a NaN)
+  const double y = r_abs(b);
+  if (ALBADA) {
+    const int k = -__builtin_amdgcn_frexp_exp(r_abs(s) + y);
+    const double u = __builtin_ldexp(m, k), v = __builtin_ldexp(y, k);
+    return {0.5 * u * v * n_rcp(fma(u, u, fma(v, v, 0x1p-1000))), along(s, b) + b};
+  }
+  return {m * n_rcp(r_abs(s) + (y + 0x1p-1021)), b};
 }
 template <bool ALBADA>
 __device__ __forceinline__ double fixed_slope(double a, double b) {
@@ -123,17 +147,19 @@ __device__ __forceinline__ void muscl(double q0, double q1, double q2, double q3
                                       double &right, bool &guard) {
 #pragma clang fp contract(off)
   const double d0 = q1 - q0, d1 = q2 - q1, d2 = q3 - q2;
-  left = q1 + half_slope<ALBADA>(d0, d1);
-  right = q2 - half_slope<ALBADA>(d2, d1);
-  guard = guard | slope_guard(d0, d1) | slope_guard(d2, d1);
+  const double s0 = along(d0, d1), s2 = along(d2, d1);
+  const HalfSlope l = half_slope<ALBADA>(s0, d1), r = half_slope<ALBADA>(s2, d1);
+  left = fma(l.w, l.d, q1);
+  right = fma(-r.w, r.d, q2);
+  guard = guard | slope_guard(s0, d1) | slope_guard(s2, d1);
 }
 template <bool ALBADA>
 __device__ __forceinline__ void muscl_guarded(double q0, double q1, double q2, double q3,
                                               double &left, double &right) {
 #pragma clang fp contract(off)
   const double d0 = q1 - q0, d1 = q2 - q1, d2 = q3 - q2;
-  if (slope_guard(d0, d1)) left = q1 + fixed_slope<ALBADA>(d0, d1);
-  if (slope_guard(d2, d1)) right = q2 - fixed_slope<ALBADA>(d2, d1);
+  if (slope_guard(along(d0, d1), d1)) left = q1 + fixed_slope<ALBADA>(d0, d1);
+  if (slope_guard(along(d2, d1), d1)) right = q2 - fixed_slope<ALBADA>(d2, d1);
 }
 
 // All-speed Roe flux of one face from the 4-cell stencil (t0,t1 | t2,t3),
