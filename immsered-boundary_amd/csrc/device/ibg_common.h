@@ -54,8 +54,9 @@ struct DevPhys {
   // conduction denominator Re*Pr_tur*(gama-1)*Ma^2 (NS_Solver.cpp:540),
   // Pr^(1/3) of the wall-temperature relation (FlowConstants.cpp:44)
   double nut_inf, nut_inlet, qkt_den, pr_cuberoot;
-  // derived: 1/(gama - 1), Cv/Rg, Cv/Rg + 1, 1/Re, 1/qkt_den
-  double ig1, cvR, cpR, iRe, iqkt;
+  // derived: 1/(gama - 1), Cv/Rg, Cv/Rg + 1, what the rounding of the two left
+  // out, 1/Re, 1/qkt_den
+  double ig1, cvR, cpR, cvRl, cpRl, iRe, iqkt;
 };
 
 // Tables that no kernel reading them writes and whose index is uniform over

@@ -1283,7 +1283,9 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
     P.pr_cuberoot = pow(p.Pr, 1.0 / 3.0);
     P.ig1 = 1.0 / (p.gama - 1.0);
     P.cvR = p.Cv / p.Rg;
+    P.cvRl = std::fma(-P.cvR, p.Rg, p.Cv) / p.Rg;
     P.cpR = P.cvR + 1.0;
+    P.cpRl = ((P.cvR - (P.cpR - 1.0)) + (1.0 - (P.cpR - (P.cpR - 1.0)))) + P.cvRl;
     P.iRe = 1.0 / p.Re;
     P.iqkt = 1.0 / P.qkt_den;
   }

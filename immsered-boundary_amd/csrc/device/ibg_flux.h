@@ -34,9 +34,17 @@ __device__ __forceinline__ double n_div(double n, double x) {
   const double q = n * y;
   return fma(fma(-x, q, n), y, q);
 }
-// FP64 reciprocal and roots to a unit in the last place: v_rcp_f64 and
-// v_rsq_f64 are good to 2^-24 (measured on gfx950: 2^-24.4 and 2^-24.2), so
-// one step of third order (e + e^2, e/2 + 3/8 e^2) reaches 2^-72.
+// The same by a constant c of reciprocal ic.
+__device__ __forceinline__ double c_div(double n, double c, double ic) {
+#pragma clang fp contract(off)
+  const double q = n * ic;
+  return fma(fma(-c, q, n), ic, q);
+}
+// FP64 reciprocal and roots to half a unit in the last place (and 2^-18 of
+// one): v_rcp_f64 and v_rsq_f64 are good to 2^-24 (measured on gfx950:
+// 2^-24.4 and 2^-24.2), so one step of third order (e + e^2, e/2 + 3/8 e^2) on
+// an exact error e reaches 2^-72, and so does a step of second order followed
+// by one with the exact residual x - g^2.
 __device__ __forceinline__ double n_rcp(double x) {
 #pragma clang fp contract(off)
   const double y = __builtin_amdgcn_rcp(x);
@@ -45,14 +53,15 @@ __device__ __forceinline__ double n_rcp(double x) {
 }
 __device__ __forceinline__ double n_sqrt(double x) {   // x > 0
 #pragma clang fp contract(off)
-  const double y = __builtin_amdgcn_rsq(x), g = x * y;
-  const double e = fma(-g, y, 1.0);
-  return fma(g * e, fma(e, 0.375, 0.5), g);
+  const double y = __builtin_amdgcn_rsq(x), h = 0.5 * y;
+  double g = x * y;
+  g = fma(g, fma(-h, g, 0.5), g);
+  return fma(fma(-g, g, x), h, g);
 }
 __device__ __forceinline__ double n_rsqrt(double x) {   // x > 0
 #pragma clang fp contract(off)
-  const double y = __builtin_amdgcn_rsq(x);
-  const double e = fma(-x * y, y, 1.0);
+  const double y = __builtin_amdgcn_rsq(x), t = x * y, tl = fma(x, y, -t);
+  const double e = fma(-tl, y, fma(-t, y, 1.0));
   return fma(y * e, fma(e, 0.375, 0.5), y);
 }
 
@@ -63,6 +72,7 @@ struct PhysR {
   R gm1, ig1;    // gama - 1 and its reciprocal
   R iRg;         // 1 / Rg (FP32 only)
   R cpR;         // Cv / Rg + 1: enthalpy h = cpR p / roe + |u|^2 / 2
+  R cpRl;        // what its rounding left out (FP64 only)
 };
 template <typename R, class Q>
 __device__ __forceinline__ PhysR<R> phys_r(const Q &P) {
@@ -70,16 +80,16 @@ __device__ __forceinline__ PhysR<R> phys_r(const Q &P) {
   ph.gama = (R)P.gama; ph.Rg = (R)P.Rg; ph.Cv = (R)P.Cv; ph.Ma = (R)P.Ma;
   ph.cpR = (R)P.cpR;
   if constexpr (sizeof(R) == 4) {
-    ph.gm1 = ph.gama - 1.0f; ph.ig1 = f_rcp(ph.gm1); ph.iRg = f_rcp(ph.Rg);
+    ph.gm1 = ph.gama - 1.0f; ph.ig1 = f_rcp(ph.gm1); ph.iRg = f_rcp(ph.Rg); ph.cpRl = 0.0f;
   } else {
-    ph.gm1 = P.gama - 1.0; ph.ig1 = P.ig1; ph.iRg = 0.0;
+    ph.gm1 = P.gama - 1.0; ph.ig1 = P.ig1; ph.iRg = 0.0; ph.cpRl = P.cpRl;
   }
   return ph;
 }
 // the same from the table of the FP32 constants
 template <class Q>
 __device__ __forceinline__ PhysR<float> phys_r32(const Q &F) {
-  return PhysR<float>{F.gama, F.Rg, F.Cv, F.Ma, F.gm1, F.ig1, F.iRg, F.cpR};
+  return PhysR<float>{F.gama, F.Rg, F.Cv, F.Ma, F.gm1, F.ig1, F.iRg, F.cpR, 0.0f};
 }
 
 template <typename R, int D>
@@ -170,17 +180,21 @@ __device__ __forceinline__ void muscl_guarded(double q0, double q1, double q2, d
 // u is the normal velocity, v (and w) the tangential ones, so the normal's
 // products with 0 and 1 are gone, and the terms of the tangential jump
 // along the normal (du_n - dubar = 0) with them.  Energy and temperature
-// enter as p/roe only: e + p/roe = cpR p/roe + |u|^2/2 and gama Rg T =
-// gama p/roe.  Per face 4 reciprocals or quotients, 4 roots and the 2 NV
+// enter as p/roe only: gama Rg T = gama p/roe, and roe e + p = cpR p +
+// roe |u|^2/2 needs no quotient.  Per face 4 reciprocals, 4 roots and the 2 NV
 // limiter quotients; the reference's form has 26 divisions and 5 roots (2D),
 // in FP64 each a chain of 10 to 15 instructions, and the kernels were bound
-// by their FP64 issue.  With the SA functions below and constant divisors as
-// products: 128 steps of the moving 2.6M-cell 2D section 127.7 -> 99.4 ms,
-// 32 steps of the 2.7M-cell 3D section 70.2 -> 57.0 ms; with third-order
-// reciprocals and roots and the guard out of the common path the stage
-// launches go from 134 to 118 us (2D) and from 294 to 242 us (3D, both with
-// block tiles).  Error of the 2D flux against 80-bit arithmetic over jumps of
-// 1e-1 .. 1e-6: rms 0.97e-16 (26-division form 0.98e-16).
+// by their FP64 issue.  With the SA functions below: 128 steps of the moving
+// 2.6M-cell 2D section 127.7 -> 99.4 ms, 32 steps of the 2.7M-cell 3D section
+// 70.2 -> 57.0 ms; with third-order reciprocals and the guard out of the common
+// path the stage launches go from 134 to 118 us (2D) and from 294 to 242 us
+// (3D, both with block tiles).
+// rms error against 80-bit arithmetic over the faces of small 2D (3D) sections
+// with jumps of 1e-4 .. 5e-2, relative to the rms flux, the 26-division form
+// -> this one: mass 1.08e-16 -> 1.08e-16 (1.60 -> 1.60), normal momentum 0.82
+// -> 0.81 (0.95 -> 0.95), energy 1.28 -> 1.21 (1.67 -> 1.61).  The energy is
+// the component that is easily lost: formed from p/roe, with the rounded
+// constant Cv/Rg + 1, it had 1.43 (1.80).
 // The fused operations are written out here and in the viscous flux below, so
 // that block and general tiles, whose faces have a known direction or not,
 // round alike and the tile size does not change a bit of the results.
@@ -210,17 +224,20 @@ __device__ __forceinline__ void roe_normal(const Prim<double, D> &t0, const Prim
   if (lim == 1) reconstruct(std::true_type());   // lim is uniform: one branch a face
   else reconstruct(std::false_type());
   const double ilr = n_rcp(lr);
-  const double plr = lp * ilr, prr = rp * n_rcp(rr);
   double lq = fma(lu, lu, lv * lv), rq = fma(ru, ru, rv * rv);
   if (D == 3) { lq = fma(lw, lw, lq); rq = fma(rw, rw, rq); }
-  const double hl = fma(ph.cpR, plr, 0.5 * lq), hr = fma(ph.cpR, prr, 0.5 * rq);
+  // roe h per volume, formed without the quotient p / roe
+  const double el = fma(ph.cpR, lp, fma(ph.cpRl, lp, (0.5 * lr) * lq));
+  const double er = fma(ph.cpR, rp, fma(ph.cpRl, rp, (0.5 * rr) * rq));
+  const double irr = n_rcp(rr);
+  const double hl = el * ilr, hr = er * irr;
   // central part 1/2 (F_L + F_R) A, without the factor A/2
   const double ml = lr * lu, mr = rr * ru;
   const double ha = 0.5 * area;
   const double c0 = fma(lr, lu, mr);
   const double c1 = fma(ml, lu, lp) + fma(mr, ru, rp);
   const double c2 = fma(ml, lv, mr * rv);
-  const double c4 = fma(ml, hl, mr * hr);
+  const double c4 = fma(el, lu, er * ru);
   const double droe = rr - lr, dp = rp - lp, dubar = ru - lu;
   // Roe average: sqrt(rr / lr) = sqrt(lr rr) / lr
   const double a_roe = n_sqrt(lr * rr);
@@ -240,7 +257,7 @@ __device__ __forceinline__ void roe_normal(const Prim<double, D> &t0, const Prim
   const double rc = a_roe * a_c;
   const double al0 = faa * fma(-dp, icsq, droe);
   // all-speed eigenvalues (NS_Solver.H:66-77): f = min(max(Ma_face, Ma_inf), 1)
-  double f = r_abs((lu + ru) * 0.5) * n_rsqrt(ph.gama * ((plr + prr) * 0.5));
+  double f = r_abs((lu + ru) * 0.5) * n_rsqrt(ph.gama * (fma(rp, irr, lp * ilr) * 0.5));
   f = f < ph.Ma ? ph.Ma : f;
   f = f > 1.0 ? 1.0 : f;
   const double g = (1.0 - f) * a_u, f1 = 1.0 + f;
@@ -474,6 +491,7 @@ struct ViscPhys {
   R ih0, ih1, ih2;   // 1/dh
   R ar0, ar1, ar2;   // face areas
   R iqkt;            // 1 / (Re*Pr_tur*(gama-1)*Ma^2) (SA closure)
+  R Re, qkt;         // (FP64 only)
 };
 // reciprocal of a constant divisor of the FP32 viscous terms: the hardware's,
 // as every quotient of that mode
@@ -531,14 +549,14 @@ __device__ __forceinline__ double sa_r(double nu, double sd2, const SaPhys<doubl
 }
 
 // Viseddy2mut (Turbulence.cpp:23-30): mu_t = roe fv1 nu, X = nu/(mu/roe)
-// clamped at 0, fv1 = X^3/(X^3 + cv1^3).  nul = mu/roe.
-__device__ __forceinline__ double sa_mut(double nu, double roe, double nul) {
+// clamped at 0, fv1 = X^3/(X^3 + cv1^3).  Here roe fv1, with nul = mu/roe.
+__device__ __forceinline__ double sa_roe_fv1(double nu, double roe, double nul) {
 #pragma clang fp contract(off)
   double bigx = v_div(nu, nul);
   if (bigx < 0.0) bigx = 0.0;
   const double b2 = bigx * bigx;
   const double fv1 = v_div(b2 * bigx, fma(b2, bigx, SA::cv1three));
-  return roe * fv1 * nu;
+  return roe * fv1;
 }
 
 // Velocity and temperature of a viscous stencil cell, T = p/(roe Rg)
@@ -562,8 +580,10 @@ __device__ __forceinline__ VelT vel_t(const Prim<double, D> &q, double Rg) {
 // face eddy viscosity mu_t = Viseddy2mut(nu_f, roe_f, mu) joins mu and the
 // heat conduction, and mflux receives the face flux of the working variable
 // (nu_f + mu/roe_f) (d nu / d n) / sigma * A (the face keisa is the unit
-// axis, so the dot product picks the normal derivative).  Constant divisors
-// (Re, sigma, 3, Re Pr_t (gama-1) Ma^2) are multiplications.
+// axis, so the dot product picks the normal derivative).  The quotients by the
+// constants 3, Re and Re Pr_t (gama-1) Ma^2 are c_div's, three instructions
+// each (as products with the rounded reciprocals the rms error of the normal
+// stress grew by 3 %).  FP64.
 template <int D>
 __device__ __forceinline__ void visc_flux(const VelT &L, const VelT &Rr, double rL, double rR,
                                           const VelT *t, int d, const ViscPhys<double, D> &vp,
@@ -603,17 +623,20 @@ __device__ __forceinline__ void visc_flux(const VelT &L, const VelT &Rr, double 
     const double fvis = (nuL + nuR) * 0.5;
     const double froe = (rL + rR) * 0.5;
     const double nul = v_div(mu0, froe);
-    const double mut0 = sa_mut(fvis, froe, nul);
-    mu0 += mut0;
-    qk0 = fma(mut0, vp.iqkt, qk0);
-    *mflux = ((fvis + nul) * ((nuR - nuL) * ih)) * (1.0 / SA::segma) * area;
+    const double rf = sa_roe_fv1(fvis, froe, nul);
+    qk0 += c_div(rf * fvis, vp.qkt, vp.iqkt);
+    mu0 = fma(rf, fvis, mu0);
+    // (1 / segma = 3/2 is exact, segma = 2/3 is not)
+    *mflux = (fvis + nul) * ((nuR - nuL) * ih) * (1.0 / SA::segma) * area;
   }
-  const double mur = mu0 * vp.iRe;
-  const double dvy = gy[1] * vp.ih1;
-  double divu = fma(gx[0], vp.ih0, dvy);
-  if (D == 3) divu = fma(gz[2], vp.ih2, divu);
-  const double dn = x ? gx[0] * vp.ih0 : (y ? dvy : gz[2] * vp.ih2);
-  const double tnn = 2.0 * mu0 * fma(divu, -1.0 / 3.0, dn) * vp.iRe;
+  const double mur = c_div(mu0, vp.Re, vp.iRe);
+  // the normal's own term rounded by itself: its rounding is then the same in
+  // the sum, and a third of it cancels
+  const double dn = x ? gx[0] * vp.ih0 : (y ? gy[1] * vp.ih1 : gz[2] * vp.ih2);
+  double divu = y ? gx[0] * vp.ih0 : gy[1] * vp.ih1;
+  if (D == 3) divu = fma((x || y) ? gz[2] : gx[0], (x || y) ? vp.ih2 : vp.ih0, divu);
+  divu += dn;
+  const double tnn = c_div(2.0 * mu0 * (dn - c_div(divu, 3.0, 1.0 / 3.0)), vp.Re, vp.iRe);
   const double txy = mur * fma(gy[0], vp.ih1, gx[1] * vp.ih0);
   const double fu = (L.u + Rr.u) * 0.5, fv = (L.v + Rr.v) * 0.5;
   double t1, t2, work;

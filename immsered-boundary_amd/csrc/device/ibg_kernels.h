@@ -144,6 +144,7 @@ __device__ __forceinline__ ViscPhys<R, D> visc_phys(const BlkInfo *blks, const D
     vp.ih0 = bi.invh[0]; vp.ih1 = bi.invh[1]; vp.ih2 = bi.invh[2];
     vp.ar0 = bi.area[0]; vp.ar1 = bi.area[1]; vp.ar2 = bi.area[2];
     vp.iqkt = P.iqkt;
+    vp.Re = P.Re; vp.qkt = P.qkt_den;
   }
   return vp;
 }
@@ -1294,13 +1295,14 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
                                       : 0.5 * (w0.u * w0.u + w0.v * w0.v);
           re0 = w0.r * (P.Cv * n_div(w0.p, w0.r * P.Rg) + ke0);
         } else {
-          re0 = fma(P.cvR, w0.p, w0.r * (0.5 * sq_speed<D>(w0.u, w0.v, w0.w)));   // roe T = p / Rg
+          // roe T = p / Rg
+          re0 = fma(P.cvR, w0.p, fma(P.cvRl, w0.p, w0.r * (0.5 * sq_speed<D>(w0.u, w0.v, w0.w))));
         }
         U[0] = w0.r; U[1] = w0.r * w0.u; U[2] = w0.r * w0.v;
         if (D == 3) { U[3] = w0.r * w0.w; U[4] = re0; } else U[3] = re0;
       }
       // cv_old + source * level_ts / v  (NS_Solver.cpp:870)
-      const double sc = level_ts * bi.invvol;
+      const double sc = kMixed ? level_ts * bi.invvol : c_div(level_ts, bi.vol, bi.invvol);
 #pragma unroll
       for (int k = 0; k < NV; ++k) U[k] = fma(s[k], sc, U[k]);
       if (a.turb) {
