@@ -798,8 +798,9 @@ __device__ __forceinline__ void visc_flux_cells(const Prim<R, D> &L, const Prim<
 // exp, x^6 and x^(1/6) of the SA functions.  FP32: (x^2)^3 and the hardware
 // exp2/log2 (v_exp_f32, v_log_f32, ~1 ulp).  FP64: exp is libm's; x^6 is
 // (x^2)^3 with the rounding errors of x^2 and x^4 added back; x^(1/6) of
-// (0, 65/64] takes the FP32 value as the seed (relative error < 1e-5) of two
-// Newton steps on y = x^(-1/6), whose error e becomes 7/2 e^2 (1e-5 ->
+// [6.5e-35, 65/64] (the arguments of sa_fw; below 1.2e-38 the seed would fail)
+// takes the FP32 value as the seed (relative error < 1e-5) of two Newton steps
+// on y = x^(-1/6), whose error e becomes 7/2 e^2 (1e-5 ->
 // 4e-10 -> 5e-19), and returns 1/y.  libm's pow costs ~150 instructions a
 // call and the source has three.  Error of fw(r) against 80-bit arithmetic,
 // r uniform in [0, 10]: rms 0.9e-16, max 4.4e-16 (pow: 4.5e-16, 6.9e-16);
@@ -831,6 +832,24 @@ template <> __device__ __forceinline__ double r_root6<double>(double x) {
 }
 template <> __device__ __forceinline__ float r_root6<float>(float x) {
   return __builtin_amdgcn_exp2f(__builtin_amdgcn_logf(x) * (1.0f / 6.0f));
+}
+
+// fw(r) of the SA destruction term: g = r + cw2 (r^6 - r),
+// fw = g ((1 + cw3^6) / (g^6 + cw3^6))^(1/6), cw3 = 2.  r is at most 10, but
+// has no lower bound where the working variable is negative (set by the
+// caller, read from a file, extrapolated): g then grows as r^6 and leaves the
+// range of r_root6's FP32 seed.  In FP64 g is held at 1e6, where 64 no longer
+// counts beside g^6 and fw has its limit to rounding; once g^6 is infinite
+// the formula gives g 0, as pow does.
+__device__ __forceinline__ float sa_fw(float r) {
+  const float g = r + (float)SA::cw2 * (r_pow6(r) - r);
+  return g * r_root6(v_div(65.0f, r_pow6(g) + 64.0f));
+}
+__device__ __forceinline__ double sa_fw(double r) {
+  const double g = r + SA::cw2 * (r_pow6(r) - r);
+  const double h = g > 1.0e6 ? 1.0e6 : g;
+  const double fw = h * r_root6(v_div(65.0, r_pow6(h) + 64.0));
+  return g < 2.3757e51 ? fw : g * 0.0;   // 2^(1024 / 6); NaN stays NaN
 }
 
 // ComptMutSource (NS_Solver.cpp:648-808) for one non-solid cell: central
@@ -880,11 +899,7 @@ __device__ __forceinline__ R sa_source(R u, R v, R w, R T, R roe, R nu, R sd, co
   const R ft2 = R(SA::ct3) * r_exp(-R(SA::ct4) * bigx * bigx);
   R rr = sa_r(nu, bigs * segdis, sp);
   rr = (R(10.0) < rr) ? R(10.0) : rr;
-  const R rsix = r_pow6(rr);
-  const R g = rr + R(SA::cw2) * (rsix - rr);
-  const R gsix = r_pow6(g);
-  const R cw3six = R(64.0);
-  const R fw = g * r_root6(v_div(R(1.0) + cw3six, gsix + cw3six));
+  const R fw = sa_fw(rr);
   R src = -(u * dvisx + v * dvisy + w * dvisz);
   src += R(SA::cb1) * (R(1.0) - ft2) * bigs * nu;
   src -= over_re((R(SA::cw1) * fw - v_div(R(SA::cb1) * ft2, R(SA::kappa * SA::kappa))) * (vis2d * vis2d), sp);

@@ -223,10 +223,7 @@ __device__ __forceinline__ R sa_pointwise(R nu, R mu0, R roe, R sd, R olen,
   const R ft2 = R(SA::ct3) * r_exp(-R(SA::ct4) * bigx * bigx);
   R rr = sa_r(nu, bigs * segdis, sp);
   rr = (R(10.0) < rr) ? R(10.0) : rr;
-  const R rsix = r_pow6(rr);
-  const R g = rr + R(SA::cw2) * (rsix - rr);
-  const R gsix = r_pow6(g);
-  const R fw = g * r_root6(v_div(R(65.0), gsix + R(64.0)));
+  const R fw = sa_fw(rr);
   const R prod = R(SA::cb1) * (R(1.0) - ft2) * bigs * nu;
   const R dest = over_re((R(SA::cw1) * fw - v_div(R(SA::cb1) * ft2, R(SA::kappa * SA::kappa))) * (vis2d * vis2d), sp);
   return prod - dest;
