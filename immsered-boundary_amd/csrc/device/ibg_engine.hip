@@ -1271,7 +1271,7 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
   for (int cs = 0; cs < nc; ++cs) {
     DevPhys &P = c->hphys[cs];
     const ibg_physics &p = ph[cs];
-    P.gama = p.gama; P.Ma = p.Ma; P.Re = p.Re; P.Rg = p.Rg; P.Cv = p.Cv; P.Cp = p.Cp; P.mu = p.mu;
+    P.gama = p.gama; P.Ma = p.Ma; P.Rg = p.Rg; P.Cv = p.Cv; P.Cp = p.Cp; P.mu = p.mu;
     P.qk = p.qk; P.SoT = p.S_over_T_ref;
     for (int k = 0; k < IBG_NFV; ++k) P.init[k] = p.initvar[k];
     P.inlet_T0 = p.inlet_T0; P.inlet_p0 = p.inlet_p0;
@@ -1279,14 +1279,16 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
     P.outlet_p = p.outlet_p; P.cfl = p.cfl; P.dt_ratio = p.dt_ratio;
     P.force_ref = p.force_ref; P.p_ref_area = p.p_ref_area; P.shear_ref_area = p.shear_ref_area;
     P.nut_inf = p.nut_inf; P.nut_inlet = p.nut_inlet;
-    P.qkt_den = p.Re * p.Pr_tur * (p.gama - 1) * pow(p.Ma, 2);
+    // (finite, as the refined quotients of the kernels want their divisors)
+    P.Re = std::min(p.Re, 1e300);
+    P.qkt_den = std::min(p.Re * p.Pr_tur * (p.gama - 1) * pow(p.Ma, 2), 1e300);
     P.pr_cuberoot = pow(p.Pr, 1.0 / 3.0);
     P.ig1 = 1.0 / (p.gama - 1.0);
     P.cvR = p.Cv / p.Rg;
     P.cvRl = std::fma(-P.cvR, p.Rg, p.Cv) / p.Rg;
     P.cpR = P.cvR + 1.0;
     P.cpRl = ((P.cvR - (P.cpR - 1.0)) + (1.0 - (P.cpR - (P.cpR - 1.0)))) + P.cvRl;
-    P.iRe = 1.0 / p.Re;
+    P.iRe = 1.0 / P.Re;
     P.iqkt = 1.0 / P.qkt_den;
   }
   // ---- per-cell arrays (device order)

@@ -18,8 +18,10 @@ __device__ __forceinline__ float r_abs(float x) { return fabsf(x); }
 
 // Reciprocal, quotient and square root of the flux arithmetic.  FP32: the
 // hardware v_rcp_f32 / v_sqrt_f32 (~1 ulp).  FP64: the hardware estimate
-// refined.  A zero, denormal or infinite operand gives NaN, so the few places
-// that meet one in earnest divide with '/'.
+// refined.  A zero, denormal or infinite divisor (or root) gives NaN: the
+// places that meet one in earnest keep it in range or divide with '/' (the
+// limiters' sums of tiny differences, the eigenvalues' root at rest, S~ of a
+// uniform stream, a wall infinitely far away, an infinite Reynolds number).
 __device__ __forceinline__ float f_rcp(float x) { return __builtin_amdgcn_rcpf(x); }
 __device__ __forceinline__ float f_sqrt(float x) { return __builtin_amdgcn_sqrtf(x); }
 __device__ __forceinline__ float n_div(float n, float x) { return n * f_rcp(x); }
@@ -54,6 +56,14 @@ __device__ __forceinline__ double n_rcp(double x) {
 __device__ __forceinline__ double n_sqrt(double x) {   // x > 0
 #pragma clang fp contract(off)
   const double y = __builtin_amdgcn_rsq(x), h = 0.5 * y;
+  double g = x * y;
+  g = fma(g, fma(-h, g, 0.5), g);
+  return fma(fma(-g, g, x), h, g);
+}
+// the same of a value that may be zero (not of a negative one)
+__device__ __forceinline__ double n_sqrt0(double x) {
+#pragma clang fp contract(off)
+  const double y = __builtin_amdgcn_rsq(fmax(x, 0x1p-1000)), h = 0.5 * y;
   double g = x * y;
   g = fma(g, fma(-h, g, 0.5), g);
   return fma(fma(-g, g, x), h, g);
@@ -261,7 +271,7 @@ __device__ __forceinline__ void roe_normal(const Prim<double, D> &t0, const Prim
   f = f < ph.Ma ? ph.Ma : f;
   f = f > 1.0 ? 1.0 : f;
   const double g = (1.0 - f) * a_u, f1 = 1.0 + f;
-  const double n0 = n_sqrt(fma(4.0 * csq, f, g * g));
+  const double n0 = n_sqrt0(fma(4.0 * csq, f, g * g));   // 0 at rest where Ma_inf is 0
   const double n1 = coef12 * r_abs(fma(f1, a_u, n0));
   const double n2 = coef12 * r_abs(fma(f1, a_u, -n0));
   const double x1 = fma(rc, dubar, dp), x2 = fma(-rc, dubar, dp);
@@ -547,6 +557,9 @@ __device__ __forceinline__ float sa_r(float nu, float sd2, const SaPhys<float> &
 __device__ __forceinline__ double sa_r(double nu, double sd2, const SaPhys<double> &sp) {
   return nu / (sd2 * sp.Re);
 }
+// the wall distance with a square in range: the terms of a farther wall vanish
+__device__ __forceinline__ float sa_dist(float d) { return d; }
+__device__ __forceinline__ double sa_dist(double d) { return r_abs(d) > 1.0e150 ? 1.0e150 : d; }
 
 // Viseddy2mut (Turbulence.cpp:23-30): mu_t = roe fv1 nu, X = nu/(mu/roe)
 // clamped at 0, fv1 = X^3/(X^3 + cv1^3).  Here roe fv1, with nul = mu/roe.
@@ -864,6 +877,7 @@ __device__ __forceinline__ R sa_source(R u, R v, R w, R T, R roe, R nu, R sd, co
                                        const R *nr, const R *ul, const R *ur, const R *vl,
                                        const R *vr, const R *wl, const R *wr, R ih0, R ih1, R ih2,
                                        const SaPhys<R> &sp, R mutf) {
+  sd = sa_dist(sd);
   const R h = R(0.5);
   const R dvisx = ((nr[0] - nl[0]) * h) * ih0;
   const R dvisy = ((nr[1] - nl[1]) * h) * ih1;

@@ -204,6 +204,7 @@ __device__ __forceinline__ R sa_olen(const VelGrad<R> &g, const SaPhys<R> &sp) {
 template <typename R>
 __device__ __forceinline__ R sa_pointwise(R nu, R mu0, R roe, R sd, R olen,
                                           const SaPhys<R> &sp) {
+  sd = sa_dist(sd);
   const R vis0 = v_div(mu0, roe);
   const R bigx = v_div(nu, vis0);
   const R b3 = bigx * bigx * bigx;
