@@ -44,6 +44,7 @@
 #include "ibg_kernels.h"
 #include "ibg_closure.h"
 #include "ibg_move.h"
+#include "ibg_pinned.h"
 #include "ibg_reflux.h"
 
 using namespace ibg;
@@ -173,18 +174,7 @@ struct ibg_ctx {
   // pinned buffers of ibg_closure_infer: rows [kInferChunk][8], then results
   // [kInferChunk]; made by ibg_closure_init, kept until the context is
   // destroyed
-  struct InferStage {
-    float *buf[2] = {nullptr, nullptr};
-    hipEvent_t done[2] = {nullptr, nullptr};
-    void release() {
-      for (int b = 0; b < 2; ++b) {
-        if (buf[b]) (void)hipHostFree(buf[b]);
-        if (done[b]) (void)hipEventDestroy(done[b]);
-        buf[b] = nullptr;
-        done[b] = nullptr;
-      }
-    }
-  } infer;
+  PinnedPair infer;
   double *dt = nullptr, *cflpart = nullptr, *rpart = nullptr, *probe = nullptr;
   unsigned long long *err = nullptr;
   unsigned long long *err2 = nullptr;   // error word of the next step's move, run ahead
@@ -2832,10 +2822,9 @@ ibg_status ibg_closure_init(ibg_ctx *c, int64_t capacity, uint64_t seed) {
   L.cap = capacity;
   L.max_wg = 1024;   // batch up to 65536 rows
   ibg_status st;
-  for (int b = 0; b < 2 && !c->infer.done[b]; ++b) {
-    HIPCHK(hipHostMalloc((void **)&c->infer.buf[b], sizeof(float) * kInferChunk * (kMlpIn + 1),
-                         hipHostMallocDefault));
-    HIPCHK(hipEventCreateWithFlags(&c->infer.done[b], hipEventDisableTiming));
+  if (!c->infer.make(sizeof(float) * kInferChunk * (kMlpIn + 1))) {
+    fprintf(stderr, "ibgpu: pinned buffers of the inference: %s\n", hipGetErrorString(hipGetLastError()));
+    return IBG_ERR_HIP;
   }
   if ((st = cl_alloc(c, &L.X, (size_t)capacity * kMlpIn))) return st;
   if ((st = cl_alloc(c, &L.Z, (size_t)capacity))) return st;
@@ -3044,7 +3033,7 @@ ibg_status ibg_closure_infer(ibg_ctx *c, const float *x, float *z, int64_t n) {
   // (two device allocations, two pageable copies and three waits a call).
   // A chunk is about 7 us of host copy and 12 us of link; 65536 rows a chunk
   // are 10 % faster from 100000 rows on, but pinning them costs 1 ms.
-  ibg_ctx::InferStage &S = c->infer;
+  PinnedPair &S = c->infer;
   constexpr int64_t R = kInferChunk;
   const int64_t nc = (n + R - 1) / R;
   ibg_status st = IBG_OK;
