@@ -102,7 +102,7 @@ struct ibg_ctx {
     std::vector<void *> allocs;
   } cl;
   uint8_t *flags = nullptr;
-  int *cellcase = nullptr, *nb27 = nullptr;
+  int *nb27 = nullptr;
   TileInfo *tiles = nullptr;
   int *halo = nullptr;         // halo lists of the block tiles (ibg_block.h)
   int nblock = 0;              // block tiles
@@ -1283,14 +1283,12 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
   }
   // ---- per-cell arrays (device order)
   std::vector<int16_t> cellblk(N);
-  std::vector<int> cellcase(N);
   hvec<int> nb27((size_t)N * 27);
   std::vector<double> sd(N);
   host_parallel(N, [&](int lo, int hi) {
     for (int i = lo; i < hi; ++i) {
       const int g = order[i];
       cellblk[i] = (int16_t)hblk[g];
-      cellcase[i] = hblk[g] / L;
       sd[i] = m->signdis[g];
       for (int q = 0; q < 27; ++q) {
         const int a = m->nb[(size_t)g * 27 + q];
@@ -1703,7 +1701,6 @@ ibg_status ibg_upload_mesh(ibg_ctx *c, const ibg_mesh_soa *m, const ibg_physics 
     if (c->turb && (st = dalloc_bytes(c, &c->NUs[k], rs * (size_t)N))) return st;
   }
   UP(c->flags, flags);
-  UP(c->cellcase, cellcase);
   UP(c->nb27, nb27);
   c->hcellblk = cellblk;
   UP(c->tiles, tiles);

@@ -310,7 +310,8 @@ __device__ __forceinline__ void from_face(double *f, int dir) {
 }
 
 // Flux of an axis-aligned face.  Output: D == 2: (mass, x-mom, y-mom,
-// energy); D == 3: (mass, x, y, z momentum, energy).
+// energy); D == 3: (mass, x, y, z momentum, energy).  DIR, FLAT: as the FP32
+// form below, which the tiles call alike (FLAT changes nothing here).
 template <int D, int DIR = -1, bool FLAT = false>
 __device__ __forceinline__ void roe_flux(const Prim<double, D> &t0, const Prim<double, D> &t1,
                                          const Prim<double, D> &t2, const Prim<double, D> &t3,

@@ -1597,8 +1597,7 @@ __global__ void k_restrict(int n, const int2 *cc, const int4 *fi, StateOut<D> o,
     re += e * s.r;
     nu += nv;
   };
-  // the sons of the low z half first, all in flight, then (a level refined
-  // in z too) the others: sums in son order either way
+  // every son's loads in flight, then the sums in son order
   Prim<double, D> s[8];
   double nv[8];
 #pragma unroll
