@@ -18,14 +18,14 @@
 // learned closure's 97 -> 87 us), k_visc_prep FP32 66 -> 43 us (30 with the
 // layout below).  3D, 2.7M
 // cells: k_stage FP32 147 -> 124 us, FP64 300 -> 294 us, k_visc_prep FP32
-// 172 -> 72 us, FP64 321 -> 141 us.  The FP32 stages then issue vector
+// 172 -> 72 us, FP64 321 -> 128 us.  The FP32 stages then issue vector
 // instructions for 77 % (3D) to 92 % (2D) of their time (2D: the bytes alone
-// would take 36 us at the copy rate), the FP64 ones for 65 to 77 %.  So the
+// would take 36 us at the copy rate), the FP64 ones for 65 to 79 %.  So the
 // code spends them sparingly: the limiters without branches, one
 // position per thread for every phase, the last column's and row's faces in
 // one pass (2D), FP32 constants from a table (Flow32), uniform bases with 32-bit
 // offsets.  With those and leaner FP64 arithmetic the 2D stages take 53 us
-// (FP32), 81 (learned closure) and 106 (FP64), the 3D ones 111 and 212.
+// (FP32), 81 (learned closure) and 104 (FP64), the 3D ones 111 and 210.
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>

@@ -200,11 +200,11 @@ __device__ __forceinline__ void muscl_guarded(double q0, double q1, double q2, d
 // path the stage launches go from 134 to 118 us (2D) and from 294 to 242 us
 // (3D, both with block tiles).
 // rms error against 80-bit arithmetic over the faces of small 2D (3D) sections
-// with jumps of 1e-4 .. 5e-2, relative to the rms flux, the 26-division form
-// -> this one: mass 1.08e-16 -> 1.08e-16 (1.60 -> 1.60), normal momentum 0.82
-// -> 0.81 (0.95 -> 0.95), energy 1.28 -> 1.21 (1.67 -> 1.61).  The energy is
-// the component that is easily lost: formed from p/roe, with the rounded
-// constant Cv/Rg + 1, it had 1.43 (1.80).
+// with jumps of a percent between cells, relative to the rms flux, the
+// 26-division form -> this one: mass 1.08e-16 -> 1.08e-16 (1.60 -> 1.60),
+// normal momentum 0.82 -> 0.81 (0.95 -> 0.95), energy 1.28 -> 1.21 (1.67 ->
+// 1.61).  The energy is the component that is easily lost: formed from p/roe,
+// with the rounded constant Cv/Rg + 1, it had 1.43 (1.80).
 // The fused operations are written out here and in the viscous flux below, so
 // that block and general tiles, whose faces have a known direction or not,
 // round alike and the tile size does not change a bit of the results.

@@ -576,8 +576,8 @@ __device__ __forceinline__ void block3_load(const Pack<R, 3> &W, const R *nu, bo
 
 // The sums are formed here: left to the compiler, the subtractions of all
 // three directions move behind the last one and their operands, sixty
-// registers in FP64, are held until then (168 registers and 8 spilled, 145
-// now: k_stage 221 -> 212 us).
+// registers in FP64, are held until then (168 registers and 8 spilled; with
+// the sums formed here 145: k_stage 221 -> 212 us).
 __device__ __forceinline__ void sum_now(double (&s)[5]) {
 #pragma unroll
   for (int k = 0; k < 5; ++k) asm volatile("" : "+v"(s[k]));
@@ -673,8 +673,8 @@ __device__ __forceinline__ void visc_prep_block3(const ViscArgs<R, 3> &a, const 
   if (a.turb) a.mutf[c] = (R)n_div(n_div(tot, bi.vol), P.Re);
 }
 
-// (waves per SIMD as the LDS of its block tiles allows; the 3D FP64 form
-// takes 184 registers unless held to three)
+// (waves per SIMD as the LDS of its block tiles allows: three for the 3D FP64
+// form, at 137 registers)
 template <typename R, int D>
 __global__ void __launch_bounds__(kTile, ((D == 3 && sizeof(R) == 8) ? 3 : 1))
 k_visc_prep(ViscArgs<R, D> a) {
@@ -1071,9 +1071,10 @@ __device__ __forceinline__ void stage_tile(const StageArgs<R, D> &a, const TileI
   const double level_ts = a.alpha * uni(a.dt)[bi.case_id] * bi.step_num;
   // The cell's operands of phase 2, all in flight at once: left at their uses
   // the master would wait for the SA source, and all of them for the flag
-  // (the learned closure spills with them held across the network).  16 steps
-  // of a small FP64 mesh 1634 -> 1569 us, the moving FP64 section 72.4 -> 71.1
-  // ms, 3D mixed 52.3 -> 50.4; even where eight waves hide it (2D FP32).
+  // (the learned closure spills with them held across the network).  The
+  // moving FP64 section 72.4 -> 71.1 ms, 3D mixed 52.3 -> 50.4; even where
+  // eight waves hide it (2D FP32), and within the 6 % spread of a small mesh's
+  // steps.
   constexpr bool kAhead = !ML;
   Prim<double, D> w0;
   R sd_c = R(0), mutf_c = R(0);
